@@ -65,8 +65,8 @@ typedef struct sa_linear_args {
  * app/gpu/ops.js:35-43 + app/gpu/gemm.js:116-223. */
 int sa_linear_f32(const sa_linear_args* args, void* stream);
 
-/* Name of the kernel sa_linear_f32 would launch for `args` ("linear_mfma_128x192", ...,
- * "linear_generic"), or NULL if the arguments are invalid. Host only; no counterpart in the
+/* Name of the kernel class sa_linear_f32 would launch for `args`, after the tile its size fills
+ * ("linear_mfma_128x192", ..., "linear_generic"; the larger classes pick their tiles within), or NULL if the arguments are invalid. Host only; no counterpart in the
  * reference (its app/gpu/ops.js:17-24 tile choice is internal). */
 const char* sa_linear_kernel_name(const sa_linear_args* args);
 

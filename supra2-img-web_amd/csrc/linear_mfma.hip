@@ -1,4 +1,4 @@
-// Linear layer y = epilogue(alpha * x W^T) on fp32 MFMA for gfx950: the projections either side of
+// Linear layer y = epilogue(alpha * x W^T) on the matrix cores of gfx950: the projections either side of
 // the attention operator (app/gpu/ops.js:35-43 `linear`, app/gpu/gemm.js:116-223 `matmulShader`
 // with A mode "rows" and B format "f32"): the DiT qkv / proj / q / kv / cproj / fc1 / fc2 layers.
 //
@@ -6,7 +6,11 @@
 //   r = alpha * sum_k x[m][k] W[n][k] (+ bias[n]), then act (GELU erf / GELU tanh / SiLU), then
 //   y[m][n] = r, y[m][n] += r, or y[m][n] += gate[gate_off + n] * r (gemm.js:127-137).
 //
-// Work decomposition
+// Three kernels: linear_split_kernel (large and medium grids, bf16 matrix cores, described there),
+// linear_mfma_kernel (fp32 MFMA, grids between those and the small ones) and linear_ksplit_kernel (small
+// grids, fp32 MFMA); split_tile and linear_mfma_tile choose. Any other alignment: linear_generic_kernel.
+//
+// Work decomposition of linear_mfma_kernel
 //   A workgroup is 4 wave64s in a 2 x 2 grid computing a BM x BN tile (BM = 64*WM, BN = 64*WN);
 //   each wave owns (32*WM) x (32*WN) outputs as WM x WN 32x32 accumulators of
 //   v_mfma_f32_32x32x2f32. The x rows are the MFMA A operand and the W rows the B operand, so
@@ -46,6 +50,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "split.h"
 
 
 namespace sa {
@@ -113,6 +118,260 @@ __device__ __forceinline__ void tile_coords(int t, const TileOrder& o, int& mi, 
   const int w = min(o.group_n, o.tiles_n - g * o.group_n);
   mi = sb * o.sb_rows + off / w;
   ni = g * o.group_n + off % w;
+}
+
+// f(std::integral_constant<int, 0>{}) ... f(std::integral_constant<int, N - 1>{}), in order
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
+// Waves per SIMD that the register budget of linear_split_kernel is set for (its VGPRs: 64 x 96 110,
+// 128 x 96 168, 256 x 144 196, 256 x 192 224).
+template <int NW, int MT, int NT>
+constexpr int split_waves_per_simd() {
+  return MT * NT <= 6 ? 4 : MT * NT <= 12 ? 3 : 2;
+}
+
+// Large and medium grids: the product on the bf16 matrix cores, each float32 operand as three bfloat16
+// terms (split.h) and each product as the six term products of 2^-24 and more of its size, smallest
+// first, summed in the float32 accumulators: x w ~ xl wh + xh wl + xm wm + xm wh + xh wm + xh wh.
+// Error against 64 bits (2-norm, N(0, 1) rows, K = 576 / 2304): 3.4e-7 / 7.2e-7, the fp32 MFMA chain
+// 4.3e-7 / 8.6e-7: one rounding per 32 k and term product instead of one per 2 k, and the terms
+// dropped are below the rounding of the sum.
+//
+// A workgroup is NW waves stacked along the rows; a wave owns 16*MT rows x 16*NT columns as MT x NT
+// accumulators of v_mfma_f32_16x16x32_bf16. W is the A operand and x the B operand, so a lane holds 4
+// consecutive columns of one row and stores 16 bytes. Each wave loads its own x rows straight into the
+// operand layout (nobody shares them) and splits them in registers; the 16-column fragments of W are
+// dealt to the waves, which split them and leave the terms in LDS in operand order (every access is one
+// contiguous 1 KB row: no bank conflicts), two stages, one barrier per 32 k. So each element of W is
+// split once per row block, and an LDS read of one term feeds MT or more MFMAs.
+//
+// What bounds it: the matrix cores at the clock they hold under this load (random operands: 2.06 of
+// the nominal 2.5 PFLOP/s measured with nothing but these MFMAs, i.e. 344 TFLOP/s of products) and the
+// issue slots the split takes beside them (11 VALU instructions per two elements; without the split,
+// results discarded, 263 TFLOP/s at K = 2304, with it 235). 16x16x32 measured faster than 32x32x16 on
+// whole grids (qkv layer of 16384 rows 160 against 191-211 us), and 8 waves over 256 rows faster than
+// twice 4 waves over 128 (half the W splits).
+template <int NW, int MT, int NT, int ACT, int EPI>
+__global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void linear_split_kernel(LinArgs p, TileOrder order) {
+  constexpr int BM = 16 * MT * NW, BN = 16 * NT, BK = 32;
+  constexpr int GW = NT % 3 == 0 ? 3 : 2;   // column fragments per group: MT * GW independent chains
+  constexpr int G = NT / GW;
+  constexpr int NF = (NT + NW - 1) / NW;    // W fragments per wave (the last waves may have one less)
+  constexpr int STAGE = NT * 3 * 64;        // 16-byte chunks per stage: [fragment][term][lane]
+  static_assert(G * GW == NT, "column fragments must split into groups");
+
+  __shared__ u32x4 lds[2 * STAGE];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15;  // operand row (x row or W row) of the lane
+  const int lc = lane >> 4;  // its 8 consecutive k of every 32
+
+  int mi, ni;
+  tile_coords(xcd_remap(blockIdx.x, order.tiles_m * order.tiles_n), order, mi, ni);
+  const int mw = mi * BM + wave * 16 * MT;  // the wave's first row; waves past M re-read the last row
+  const int n0 = ni * BN;
+  const int mb = min(mw, p.M - 1);
+  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(p.x + (int64_t)mb * p.ldx);
+  const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(p.w + (int64_t)n0 * p.ldw);
+  unsigned xoff[MT], woff[NF];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xoff[i] = 4u * (unsigned)(min(16 * i + lr, p.M - 1 - mb) * p.ldx + 8 * lc);
+#pragma unroll
+  for (int f = 0; f < NF; ++f) woff[f] = 4u * (unsigned)(min(16 * (f * NW + wave) + lr, p.N - 1 - n0) * p.ldw + 8 * lc);
+  const int nkt = (p.K + BK - 1) / BK;
+  const int nfull = p.K / BK;  // whole k-tiles; with K % 32 != 0 the last tile (nfull) holds K
+
+  f32x4 xa[MT][2], wb[NF][2];  // the next k-tile as loaded
+  auto load = [&](int kt) {
+    const unsigned s = 4u * (unsigned)(kt * BK);
+    unsigned back = 0;  // chunks of 8 k past K re-read the last one (zeroed by cut)
+    if (kt >= nfull) back = 4u * (unsigned)max(kt * BK + 8 * lc + 8 - p.K, 0);
+    auto ld = [&](__amdgpu_buffer_rsrc_t r, unsigned v) {
+      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0));
+    };
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      if (f * NW + wave < NT) {
+        wb[f][0] = ld(wr, woff[f] - back);
+        wb[f][1] = ld(wr, woff[f] - back + 16);
+      }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      xa[i][0] = ld(xr, xoff[i] - back);
+      xa[i][1] = ld(xr, xoff[i] - back + 16);
+    }
+  };
+  auto cut = [&](int kt) {
+    if (kt >= nfull && kt * BK + 8 * lc >= p.K) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) wb[f][0] = wb[f][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < MT; ++i) xa[i][0] = xa[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  auto put = [&](int f, int stage) {
+    if (f * NW + wave < NT) {
+      const Split8 s = split8(wb[f][0], wb[f][1]);
+      u32x4* d = lds + stage * STAGE + (f * NW + wave) * 192 + lane;
+      d[0] = s.h;
+      d[64] = s.m;
+      d[128] = s.l;
+    }
+  };
+  Split8 a[2][MT];
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // k-tile kt from stage C; the splits of the next tile go between the groups' MFMAs
+  auto step = [&](int kt, auto stage) {
+    constexpr int C = decltype(stage)::value;
+    const bool more = kt + 1 < nkt;
+    if (more) cut(kt + 1);
+    static_for<G>([&](auto gg) {
+      constexpr int g = decltype(gg)::value;
+      u32x4 b[GW][3];
+#pragma unroll
+      for (int j = 0; j < GW; ++j)
+#pragma unroll
+        for (int t = 0; t < 3; ++t) b[j][t] = lds[C * STAGE + (g * GW + j) * 192 + t * 64 + lane];
+      auto products = [&](int t, auto term) {
+#pragma unroll
+        for (int j = 0; j < GW; ++j)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) acc[i][g * GW + j] = mfma16(b[j][t], term(a[C][i]), acc[i][g * GW + j]);
+      };
+      products(2, [](const Split8& s) { return s.h; });
+      products(0, [](const Split8& s) { return s.l; });
+      products(1, [](const Split8& s) { return s.m; });
+      products(1, [](const Split8& s) { return s.h; });
+      products(0, [](const Split8& s) { return s.m; });
+      products(0, [](const Split8& s) { return s.h; });
+      if (more) {
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          if (f % G == g) put(f, C ^ 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          if ((i + NF) % G == g) a[C ^ 1][i] = split8(xa[i][0], xa[i][1]);
+      }
+    });
+    if (kt + 2 < nkt) load(kt + 2);
+    __syncthreads();
+  };
+  load(0);
+  cut(0);
+#pragma unroll
+  for (int f = 0; f < NF; ++f) put(f, 0);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) a[0][i] = split8(xa[i][0], xa[i][1]);
+  if (nkt > 1) load(1);
+  __syncthreads();
+  int kt = 0;
+  for (; kt + 2 <= nkt; kt += 2) {
+    step(kt, std::integral_constant<int, 0>{});
+    step(kt + 1, std::integral_constant<int, 1>{});
+  }
+  if (kt < nkt) step(kt, std::integral_constant<int, 0>{});
+
+  // An infinity, a NaN or a magnitude that rounds past the bfloat16 range has no three terms: the
+  // differences turn into NaN. A wave that finds anything not finite in its sums takes its whole tile
+  // again with fp32 MFMAs straight from memory, so such inputs give what float32 products give.
+  float z = 0.f;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z = fmaf(acc[i][j][e], 0.f, z);
+  if (__builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float* xrow[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) xrow[i] = p.x + (int64_t)min(mw + 16 * i + lr, p.M - 1) * p.ldx + lc;
+    const float* w0 = p.w + (int64_t)n0 * p.ldw + lc;
+#pragma unroll 1
+    for (int k = 0; k < p.K; k += 4) {
+      float xv[MT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) xv[i] = xrow[i][k];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const float wv = w0[(int64_t)min(16 * j + lr, p.N - 1 - n0) * p.ldw + k];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv[i], acc[i][j], 0, 0, 0);
+      }
+    }
+  }
+
+  // ---- epilogue: lane holds columns n0 + 16j + 4*lc .. +3 of row mw + 16i + lr. Rows, bias and gate are
+  // read and written 16 bytes at a time where they are aligned, element by element otherwise and at
+  // the edge of N. Plain stores are non-temporal: y is not read back here, and keeping it out of the L2
+  // leaves the W panels and x rows there; the residual epilogues, which have just read their rows, keep
+  // the default policy.
+  auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  const bool row_vec = a16(p.y) && a16(p.resid) && (p.ldy & 3) == 0;
+  const bool bias_vec = a16(p.bias), gate_vec = a16(p.gate);
+  auto load4 = [&](const float* src, bool vec, int left) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (vec && left >= 4) return *reinterpret_cast<const f32x4*>(src);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (e < left) v[e] = src[e];
+    return v;
+  };
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = mw + 16 * i + lr;
+    if (m >= p.M) continue;
+    const int nl = n0 + 4 * lc;
+    const int64_t row = (int64_t)m * p.ldy;
+    f32x4 old[EPI != LIN_EPI_STORE ? NT : 1];
+    if constexpr (EPI != LIN_EPI_STORE) {  // the old values of the row together, then combined
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        if (nl + 16 * j < p.N) old[j] = load4(p.resid + row + nl + 16 * j, row_vec, p.N - nl - 16 * j);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int n = nl + 16 * j;
+      const int left = p.N - n;
+      if (left <= 0) continue;
+      f32x4 v = {0.f, 0.f, 0.f, 0.f}, g = {1.f, 1.f, 1.f, 1.f};
+      if (p.bias) v = load4(p.bias + n, bias_vec, left);
+      if constexpr (EPI == LIN_EPI_RESID_GATE) g = load4(p.gate + n, gate_vec, left);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = apply_act<ACT>(fmaf(acc[i][j][e], p.alpha, v[e]));
+        if constexpr (EPI != LIN_EPI_STORE) v[e] = fmaf(g[e], v[e], old[j][e]);
+      }
+      float* dst = p.y + row + n;
+      if (row_vec && left >= 4) {
+        if constexpr (EPI == LIN_EPI_STORE) __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(dst));
+        else *reinterpret_cast<f32x4*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e < left) {
+            if constexpr (EPI == LIN_EPI_STORE) __builtin_nontemporal_store(v[e], dst + e);
+            else dst[e] = v[e];
+          }
+      }
+    }
+  }
 }
 
 // WM x WN accumulators per wave, BK k per tile (16 or 32), NS tiles in flight (LDS stages); the
@@ -608,6 +867,37 @@ hipError_t launch_epi(const LinearParams& p, hipStream_t stream) {
   }
 }
 
+template <int NW, int MT, int NT, int ACT, int EPI>
+hipError_t launch_split_tiles(const LinearParams& p, hipStream_t stream) {
+  const int64_t tm = (p.M + 16 * MT * NW - 1) / (16 * MT * NW);
+  const int64_t tn = (p.N + 16 * NT - 1) / (16 * NT);
+  if (tm * tn > 0x7fffffff) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((linear_split_kernel<NW, MT, NT, ACT, EPI>), dim3((unsigned)(tm * tn)), dim3(64 * NW), 0, stream,
+                     lin_args(p), tile_order(p, 16 * MT * NW, 16 * NT));
+  return hipGetLastError();
+}
+
+template <int NW, int MT, int NT, int ACT>
+hipError_t launch_split_epi(const LinearParams& p, hipStream_t stream) {
+  switch (p.epi) {
+    case LIN_EPI_STORE: return launch_split_tiles<NW, MT, NT, ACT, LIN_EPI_STORE>(p, stream);
+    case LIN_EPI_RESID: return launch_split_tiles<NW, MT, NT, ACT, LIN_EPI_RESID>(p, stream);
+    case LIN_EPI_RESID_GATE: return launch_split_tiles<NW, MT, NT, ACT, LIN_EPI_RESID_GATE>(p, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int NW, int MT, int NT>
+hipError_t launch_split(const LinearParams& p, hipStream_t stream) {
+  switch (p.act) {
+    case LIN_ACT_NONE: return launch_split_epi<NW, MT, NT, LIN_ACT_NONE>(p, stream);
+    case LIN_ACT_GELU: return launch_split_epi<NW, MT, NT, LIN_ACT_GELU>(p, stream);
+    case LIN_ACT_GELU_TANH: return launch_split_epi<NW, MT, NT, LIN_ACT_GELU_TANH>(p, stream);
+    case LIN_ACT_SILU: return launch_split_epi<NW, MT, NT, LIN_ACT_SILU>(p, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <int TM, int TN, int KS, int ACT, int EPI>
 hipError_t launch_ksplit_tiles(const LinearParams& p, hipStream_t stream) {
   TileOrder o;
@@ -666,21 +956,19 @@ bool linear_mfma_supported(const LinearParams& p) {
          (int64_t)64 * 2 * p.ldy * 4 < 0x7fffffffLL;
 }
 
+// Size class of a call: the tile of the fp32 kernels that its grid fills, and the kernel's name in the
+// API. Classes 128 x 192 and 64 x 192 (at least one 128 x 192 tile per CU, or three 64 x 192 ones) run
+// linear_split_kernel, class 64 x 64 linear_split_kernel or linear_mfma_kernel (split_tile below).
+// Grids of fewer 64 x 64 tiles than 1.25 per CU take linear_ksplit_kernel, whose quarter-K waves
+// spread them over the SIMDs (us, 64 x 64 -> k-split: VAE output projection 1024 x 512 x 512 11.75 ->
+// 8.1, context k|v 77 x 1152 x 576 13.2 -> 6.3, batch-2 proj/q/cproj 512 x 576 x 576 12.6-13.0 ->
+// 8.4-8.7, fc1 512 x 2304 x 576 21.4 -> 19.2, fc2 512 x 576 x 2304 43.4 -> 23.0). Grids of 1.25 to 2
+// such tiles per CU take 32 x 64 tiles with k split in two, whose count is twice that and so shares
+// out more evenly over the CUs (VAE q|k|v 1024 x 1536 x 512, 384 tiles: 64 x 64 18.7-19.2, 32 x 64 /
+// two splits 17.4, 64 x 32 17.5, 64 x 32 / four splits 17.9, 64 x 64 / two splits 20.7, 32 x 32 / four
+// splits 18.9-19.4). The split kernel's smallest tiles (64 x 48) measured slower than both there: 13-20
+// against 6-15 us at K = 576, its loads being one k-tile ahead.
 LinearTile linear_mfma_tile(const LinearParams& p, int num_cus) {
-  // Measured per layer on the DiT linears at 16384 rows (after a warm-up; seven tile / k-depth /
-  // stage variants): 128 x 192 tiles (2 x 3 accumulators per wave, k-depth 32, two stages) for the
-  // 2304-wide fc1 (324 us; 64 x 192: 336 us); 64 x 192 tiles (one 32 x 96 strip per wave, each x
-  // operand read feeding three MFMAs) with k-depth 16 and three stages at three workgroups per CU
-  // for qkv (245 us; k-depth 32 / two stages 254, 128 x 192 271) and the 576-wide layers (proj/q/
-  // cproj 85-88 us, fc2 320 us; 64 x 64: 90-95 and 337). Grids of fewer 64 x 64 tiles than 1.25
-  // per CU take linear_ksplit_kernel, whose quarter-K waves spread them over the SIMDs (us, 64 x 64
-  // -> k-split: VAE output projection 1024 x 512 x 512 11.75 -> 8.1, context k|v 77 x 1152 x 576 13.2
-  // -> 6.3, batch-2 proj/q/cproj 512 x 576 x 576 12.6-13.0 -> 8.4-8.7, fc1 512 x 2304 x 576 21.4 ->
-  // 19.2, fc2 512 x 576 x 2304 43.4 -> 23.0). Grids of 1.25 to 2 such tiles per CU take 32 x 64
-  // tiles with k split in two, whose count is twice that and so shares out more evenly over the CUs
-  // (VAE q|k|v 1024 x 1536 x 512, 384 tiles: 64 x 64 18.7-19.2, 32 x 64 / two splits 17.4, 64 x 32
-  // 17.5, 64 x 32 / four splits 17.9, 64 x 64 / two splits 20.7, 32 x 32 / four splits 18.9-19.4);
-  // wider grids keep 64 x 64 tiles.
   const int64_t tiles_wide = ((p.M + 127) / 128) * ((p.N + 191) / 192);
   const int64_t tiles_tall = ((p.M + 63) / 64) * ((p.N + 191) / 192);
   const int64_t tiles_64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
@@ -690,6 +978,46 @@ LinearTile linear_mfma_tile(const LinearParams& p, int num_cus) {
   if (tiles_64 < 2 * (int64_t)num_cus) return {1, 2, 64, 2, 2};
   return {1, 1, 32, 2, 0};
 }
+
+namespace {
+
+// The tile that linear_split_kernel runs a call of the larger classes with, or kMfma64: linear_mfma_kernel
+// on 64 x 64 tiles. Each candidate's time is estimated from how many of its tiles every CU gets, with
+// the times of 1, 2, ... tiles per CU measured at K = 576 and 2304 and linear in K (us; u = K / 576):
+//   256 x 144, 8 waves: 56 / 206 per tile of a CU            (N = 576, 16384 rows: exactly one)
+//   256 x 192, 8 waves: 70 / 249
+//   128 x 96, 4 waves:  35 / 120, 45 / 152, 56 / 213 for 1, 2, 3 tiles on a CU at once
+//   64 x 96, 4 waves:   22 / 78, 30 / 98, 39 / 128, 50 / 165 for 1 .. 4
+//   64 x 64 fp32 MFMA:  6 us + 125 TFLOP/s
+// Measured over 8 (N, K) of 512..2304 x 14 row counts from 64 to 16128: the choices take 5.60 ms in all,
+// the fp32 kernels alone 7.13, the best of 13 tiles each time (256 x 128, 256 x 96, 128 x 64, 64 x 64,
+// 128 x 48, 64 x 48 and 128 x 96 in 8 waves too) 5.41.
+enum SplitTile { kMfma64, kSplit64x96, kSplit128x96, kSplit256x144, kSplit256x192 };
+SplitTile split_tile(const LinearParams& p, int num_cus, bool allow_mfma) {
+  const double u = p.K / 576.0;
+  auto per_cu = [&](int bm, int bn) {
+    const int64_t tiles = (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+    return (tiles + num_cus - 1) / num_cus;
+  };
+  const int64_t n64 = per_cu(64, 96), n128 = per_cu(128, 96);
+  const double t64[5] = {0, 3.5 + 18.5 * u, 7.5 + 22.5 * u, 9 + 30 * u, 12 + 38 * u};
+  const double t128[4] = {0, 6 + 28.5 * u, 9 + 36 * u, 4 + 52 * u};
+  double best = n64 / 4 * t64[4] + t64[n64 % 4];
+  SplitTile t = kSplit64x96;
+  auto take = [&](double cost, SplitTile c) {
+    if (cost < best) {
+      best = cost;
+      t = c;
+    }
+  };
+  take(n128 / 3 * t128[3] + t128[n128 % 3], kSplit128x96);
+  take(per_cu(256, 144) * (6 + 50 * u), kSplit256x144);
+  take(per_cu(256, 192) * (10 + 60 * u), kSplit256x192);
+  if (allow_mfma) take(6 + 2e-6 / 125 * p.M * (double)p.N * p.K, kMfma64);
+  return t;
+}
+
+}  // namespace
 
 const char* linear_kernel_name(const LinearParams& p, int num_cus) {
   if (!linear_mfma_supported(p)) return "linear_generic";
@@ -711,9 +1039,13 @@ hipError_t launch_linear(const LinearParams& p, int num_cus, hipStream_t stream)
   const LinearTile t = linear_mfma_tile(p, num_cus);
   if (t.ksplit == 4) return launch_ksplit<1, 1, 4>(p, stream);
   if (t.ksplit == 2) return launch_ksplit<1, 2, 2>(p, stream);
-  if (t.wm == 2) return launch_act<2, 3, 32, 2>(p, stream);
-  if (t.wn == 3) return launch_act<1, 3, 16, 3>(p, stream);
-  return launch_act<1, 1, 32, 2>(p, stream);
+  switch (split_tile(p, num_cus, t.wn == 1)) {
+    case kSplit64x96: return launch_split<4, 1, 6>(p, stream);
+    case kSplit128x96: return launch_split<4, 2, 6>(p, stream);
+    case kSplit256x144: return launch_split<8, 2, 9>(p, stream);
+    case kSplit256x192: return launch_split<8, 2, 12>(p, stream);
+    default: return launch_act<1, 1, 32, 2>(p, stream);
+  }
 }
 
 }  // namespace sa

@@ -1,0 +1,72 @@
+"""The linear layer on the bf16 matrix cores (linear_split_kernel): every tile at ragged M, N and K, every
+epilogue, rows that are not 16-byte aligned, and values that have no three bfloat16 terms.
+
+Tolerance: each operand is held to 24 bits and six of the nine term products are kept, so a sum of K
+products differs from 64 bits by the rounding of its K/32 * 6 float32 additions, at most
+6 * ceil(K/32) * 2^-24 of sum |x w| and about its square root in the 2-norm. 2e-6 covers K = 584 with
+the spread of sum |x w| over |sum x w| (about sqrt(K)) taken in."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import linear as ol
+from supra_attn import _lib
+from supra_attn.linear_workloads import make_linear
+from supra_attn.runner import StagedLinear
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-6
+
+# (M, N, K): 64 x 96, 128 x 96, 256 x 144 and 256 x 192 tiles on 256 CUs, each ragged in M and N, with
+# K % 32 of 8, 24 and 16 (and one k-tile more or less than even), and K shorter than one k-tile
+SIZES = [(2047, 2050, 776), (3071, 1730, 584), (16300, 570, 40), (16300, 760, 72), (16299, 571, 24), (16299, 763, 48),
+         (16333, 1729, 8)]
+
+
+def run(dev, call):
+    print(f"[linear split] {call.name} M={call.M} N={call.N} K={call.K} act={call.act} epi={call.epi}", flush=True)
+    st = StagedLinear(dev, call)
+    try:
+        return st.run()
+    finally:
+        st.release()
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("epi,act,kw", [
+    (_lib.SA_EPI_STORE, _lib.SA_ACT_NONE, {}),
+    (_lib.SA_EPI_RESID_GATE, _lib.SA_ACT_GELU_TANH, dict(gate_off=3)),  # gate not 16-byte aligned
+    (_lib.SA_EPI_RESID, _lib.SA_ACT_SILU, dict(y_off=1)),               # rows of y not aligned
+])
+def test_tiles(dev, M, N, K, epi, act, kw):
+    kw = dict(kw, ldy=(N + 7) // 4 * 4)
+    call = make_linear(f"split_{M}x{N}x{K}", M, N, K, seed=M + N + K + epi, act=act, epi=epi, **kw)
+    got = run(dev, call)
+    e = ol.errors(got, ol.linear_fp64(call.x, call.w, call.y0, **call.oracle_kwargs()))
+    assert e["finite"] and e["rel_l2"] <= TOL and e["max_rel"] <= 1e-5, e
+
+
+@pytest.mark.parametrize("M,N,K", [(2047, 2050, 776), (16300, 570, 40)])
+def test_values_without_three_terms(dev, M, N, K):
+    """Infinities, NaN, and magnitudes that round past the bfloat16 range (finite products) give what
+    float32 products give: the same elements infinite, NaN or finite, and the finite ones to tolerance."""
+    call = make_linear(f"special_{M}x{N}x{K}", M, N, K, seed=K)
+    x = call.x.reshape(-1)
+    x[5 * K + 3] = np.inf
+    x[700 * K + 7] = -np.inf
+    x[1400 * K] = np.nan
+    x[2046 * K + 1] = np.float32(3.4e38)
+    w = call.w.reshape(-1)
+    w[(N - 1) * K + 2] = np.inf
+    w[40 * K + 3] = 0.0  # inf * 0
+    got = run(dev, call).reshape(-1)
+    ref = ol.linear_torch_fp32(call.x, call.w, call.y0, **call.oracle_kwargs()).reshape(-1)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(ref))
+    np.testing.assert_array_equal(got[np.isinf(got)], ref[np.isinf(ref)])
+    fin = np.isfinite(ref)
+    rows = np.repeat(np.abs(np.where(fin, ref, 0)).reshape(M, N).max(axis=1), N)  # 3.4e38 sets its row's scale
+    assert np.all(np.abs(got[fin] - ref[fin]) <= 1e-5 * rows[fin])
