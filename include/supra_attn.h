@@ -115,7 +115,7 @@ typedef struct sa_attn_args {
   const int32_t* key_len_host;
 } sa_attn_args;
 
-/* Fused attention, fp32 in and out, fp32 MFMA arithmetic. Replaces ops.attention
+/* Fused attention, fp32 in and out, products and sums to fp32 accuracy. Replaces ops.attention
  * (app/gpu/ops.js:103-149) for every caller in app/models/{dit,t5,vae}.js; B folds the
  * per-sample host loops of app/models/dit.js:170-185 into one launch. Asynchronous on `stream`. */
 int sa_attention_f32(const sa_attn_args* args, void* stream);
@@ -157,7 +157,10 @@ const char* sa_attention_kernel_name(const sa_attn_args* args);
  * The reference picks a matmul tile (app/gpu/ops.js:15-31) and decides fused vs unfused
  * (ops.js:111-112) inside the operator; these host-only queries make the equivalent choice of
  * this library inspectable, so tests can show that every compiled variant runs. */
-#define SA_KERNEL_FLASH 1   /* flash_mfma_kernel<head_dim, key_split, bias_mode, mask_variant> */
+#define SA_KERNEL_FLASH 1   /* flash attention, head dim 64 or 128. A plan counts these calls by launch class:
+                               units of 128 queries (64 at key_split 2), units past the last whole
+                               round as a tail. The kernel that runs a class (flash_split_kernel) groups
+                               queries, splits keys and shapes its grid by itself. */
 #define SA_KERNEL_WIDE 2    /* wide_mfma_kernel<head_dim, bias_mode, mask_variant> (no bias or a dense one), + a
                                 merge kernel when key_chunks > 1 */
 #define SA_KERNEL_GENERIC 3 /* generic_kernel (any head dim <= 1024, any alignment) */

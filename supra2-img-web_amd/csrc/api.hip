@@ -723,7 +723,7 @@ int run_attention(const sa_attn_args* args, void* stream, bool own_scratch) {
   apply_schedule(p, c);
   hipError_t e;
   if (c.path == Path::kFlash) {
-    e = sa::launch_flash_mfma(p, c.nsplit, num_cus(), (hipStream_t)stream);
+    e = sa::launch_flash_split(p, num_cus(), (hipStream_t)stream);
   } else if (c.path == Path::kSmall) {
     e = sa::launch_flash_small(p, (hipStream_t)stream);
   } else if (c.path == Path::kSmall16) {

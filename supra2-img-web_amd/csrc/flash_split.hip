@@ -1,0 +1,515 @@
+// Flash attention on the bf16 matrix cores of gfx950, head dim 64 or 128, for launches that fill the chip
+// (app/gpu/kernels.js:164-316 and, with bias and masks fused, the unfused chain of
+// app/gpu/ops.js:119-147): every float32 operand as three bfloat16 terms (split.h), every product as
+// six term products summed in float32, smallest first. Same contract as flash_mfma.hip.
+//
+// Work decomposition
+//   A workgroup is QG * KS waves: QG groups of 32 queries of one (sequence, head), each seen by KS waves
+//   that take every KS-th block of 32 keys and merge their softmax states through LDS at the end. A step
+//   covers KS blocks. All waves load the step's K and V rows into registers one step ahead, split
+//   them once for the workgroup, and leave the terms in LDS in operand order.
+//   Scores S^T = K Q^T and output O^T += V^T P^T with v_mfma_f32_32x32x16_bf16: a lane holds query l%32 and
+//   keys 8(r/4) + 4(l/32) + r%4 in register r, as with the fp32 32x32x2 products, so the softmax, masks and
+//   epilogue are those of flash_mfma.hip. The 8 keys that a half-wave multiplies per product step of 16
+//   are the 8 of its own registers (order of the sum over keys: any), so P needs no exchange: V is laid out
+//   to match. Q is pre-scaled and split once.
+//   LDS: K terms [product step][term][half][key ^ chunk], so that the 8 threads of a row write 8 different
+//   bank groups; V terms [product step][32 dims][term][half][dim], transposed by loading a
+//   row of 64 dims per instruction, 8 keys per thread.
+
+#include <string.h>
+
+#include <type_traits>
+
+#include "common.h"
+#include "kernels.h"
+#include "split.h"
+
+namespace sa {
+
+namespace {
+
+constexpr float kRescaleSlack = 8.f;  // log2 units: p stays <= 256 between rescales
+
+struct FlashOrder {
+  uint8_t order[kMaxOrder];
+};
+struct NoOrder {};
+
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ f32x16 zero16() {
+  f32x16 z;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) z[i] = 0.f;
+  return z;
+}
+
+__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+template <int D, int QG, int KS, int STAGES, int WPE, int BIAS, int MASK, typename Order>
+__global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArgs p, Order ord) {
+  constexpr int NW = QG * KS;
+  constexpr int QT = 32 * QG;            // queries per workgroup
+  constexpr int KT = 32 * KS;            // keys per step
+  constexpr int FK = D / 16;             // product steps of the scores
+  constexpr int NDB = D / 32;            // 32-dim output tiles
+  constexpr int CPR = D / 8;             // chunks of 8 dims per K row
+  constexpr int NC = D / (16 * QG);      // K chunks and V units per thread and step
+  constexpr int KBLK = FK * 3 * 64;      // 16-byte chunks of one block's K terms (V: the same)
+  constexpr int BLK = 2 * KBLK;
+  constexpr int STAGE = KS * BLK;
+  constexpr int MSTRIDE = 16 * NDB + 2;  // merge record per lane: O tiles, m, l
+  constexpr bool kLen = MASK == MASK_KEY_LEN || MASK == MASK_KEY_LEN_ORDERED;
+  static_assert(NC * 16 * QG == D, "a step's rows must split over the threads");
+  constexpr int OUT = KS == 1 ? NW * 32 * D / 4 : 0;  // the output rows reuse the tiles
+  constexpr int LDS = STAGES * STAGE > OUT ? STAGES * STAGE : OUT;
+  static_assert((KS - 1) * QG * 64 * MSTRIDE <= 4 * LDS, "merge records must fit in the tiles");
+
+  constexpr int RB = QT + KT - 1;        // relative distances per step
+  static_assert(BIAS != BIAS_RELPOS || RB <= 64 * NW, "one relative distance per thread");
+  static_assert(KT <= 64 * NW, "one key mask per thread");
+
+  __shared__ u32x4 lds[LDS];
+  __shared__ float lds_rb[BIAS == BIAS_RELPOS ? STAGES * RB : 1];
+  __shared__ float lds_km[MASK == MASK_KEY_MASK ? STAGES * KT : 1];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qg = wave % QG;
+  const int ks = wave / QG;
+  const int col = lane & 31;
+  const int half = lane >> 5;
+
+  const int q_tiles = (p.Lq + QT - 1) / QT;
+  int tile = xcd_remap(blockIdx.x, p.tiles);
+  const int qtile = tile % q_tiles;
+  tile /= q_tiles;
+  const int h = tile % p.H;
+  int b = tile / p.H;
+  if constexpr (MASK == MASK_KEY_LEN_ORDERED) b = ord.order[b];  // the host schedule
+  const int q0 = qtile * QT;
+  const int qi = q0 + qg * 32 + col;
+  const bool q_valid = qi < p.Lq;
+
+  int kv_len = p.Lk;
+  if constexpr (kLen) kv_len = min(max(static_cast<const int32_t*>(p.mask)[b], 0), p.Lk);
+  const int nblk = (kv_len + 31) >> 5;
+  const int nstep = (nblk + KS - 1) / KS;
+  const uint8_t* kmask = MASK == MASK_KEY_MASK ? static_cast<const uint8_t*>(p.mask) + (int64_t)b * p.aux : nullptr;
+  const float* kbase = p.k + (int64_t)b * p.sk + h * D;
+  const float* vbase = p.v + (int64_t)b * p.sv + h * D;
+  const float* qrow = p.q + (int64_t)b * p.sq + (int64_t)min(qi, p.Lq - 1) * p.ldq + h * D;
+  const float* brow = nullptr;
+  if constexpr (BIAS == BIAS_DENSE) brow = p.bias + (int64_t)b * p.sbias + ((int64_t)h * p.Lq + min(qi, p.Lq - 1)) * p.Lk;
+
+  // ---- a step's K and V as loaded: rows past the last valid key re-read it (masked out of the softmax).
+  // With them the step's bias and mask: the dense-bias values of the lane's 16 keys; the table value of
+  // one relative distance per thread (its bucket is loaded a step earlier) and one key's mask, which go
+  // to LDS with the terms.
+  f32x4 kx[NC][2];
+  float vx[NC][8];
+  float bx[BIAS == BIAS_DENSE ? 16 : 1];
+  float rbx = 0.f, kmx = 0.f;
+  int bucket = -1;
+  float bcur[BIAS == BIAS_DENSE ? 16 : 1];
+  auto load_bucket = [&](int step) {
+    // entry e covers LUT index key0 - (q0 + QT - 1) + (Lq - 1) + e
+    const int li = step * KT - (q0 + QT - 1) + (p.Lq - 1) + tid;
+    bucket = tid < RB && li >= 0 && li <= p.Lq + p.Lk - 2 ? max(p.lut[li], 0) : -1;
+  };
+  auto load = [&](int step) {
+    const int key0 = step * KT;
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const int id = n * 64 * NW + tid;
+      const float* src = kbase + (int64_t)min(key0 + id / CPR, kv_len - 1) * p.ldk + 8 * (id % CPR);
+      kx[n][0] = *reinterpret_cast<const f32x4*>(src);
+      kx[n][1] = *reinterpret_cast<const f32x4*>(src + 4);
+    }
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const int u = n * NW + wave;  // unit: block u / (D/16), product step, half, 64 dims
+      const int s = (u / (D / 64)) >> 1 & 1, hh = (u / (D / 64)) & 1;
+      const int k0 = key0 + 32 * (u / (D / 16)) + 16 * s + 4 * hh;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = min(k0 + (j & 3) + 8 * (j >> 2), kv_len - 1);
+        vx[n][j] = vbase[(int64_t)key * p.ldv + 64 * (u % (D / 64)) + lane];
+      }
+    }
+    if constexpr (BIAS == BIAS_DENSE) {
+      const int k0 = key0 + 32 * ks + 4 * half;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (key0 + 32 * ks + 32 <= p.Lk) {  // runs of 4 keys at any 4-byte alignment
+          const f32x4_a4 v = *reinterpret_cast<const f32x4_a4*>(brow + k0 + 8 * g);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bx[4 * g + e] = v[e];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bx[4 * g + e] = brow[min(k0 + 8 * g + e, p.Lk - 1)];
+        }
+      }
+    }
+    if constexpr (BIAS == BIAS_RELPOS) {
+      rbx = bucket >= 0 ? p.bias[min(bucket, p.num_buckets - 1) * p.H + h] : 0.f;
+      load_bucket(step + 1);
+    }
+    if constexpr (MASK == MASK_KEY_MASK) {
+      const int key = key0 + tid;
+      kmx = tid < KT && key < p.Lk && kmask[min(key, p.Lk - 1)] != 0 ? 0.f : -INFINITY;
+    }
+  };
+  auto store = [&](int stage) {
+    u32x4* base = lds + stage * STAGE;
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const int id = n * 64 * NW + tid;
+      const int key = id / CPR, c = id % CPR;
+      const Split8 t = split8(kx[n][0], kx[n][1]);
+      u32x4* d = base + (key >> 5) * BLK + (c >> 1) * 192 + (c & 1) * 32 + ((key & 31) ^ (c & 7));
+      d[0] = t.h;
+      d[64] = t.m;
+      d[128] = t.l;
+    }
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const int u = n * NW + wave;
+      const int s = (u / (D / 64)) >> 1 & 1, hh = (u / (D / 64)) & 1;
+      const int t32 = 2 * (u % (D / 64)) + half;
+      const Split8 t = split8(f32x4{vx[n][0], vx[n][1], vx[n][2], vx[n][3]}, f32x4{vx[n][4], vx[n][5], vx[n][6], vx[n][7]});
+      u32x4* d = base + (u / (D / 16)) * BLK + KBLK + (s * NDB + t32) * 192 + hh * 32 + col;
+      d[0] = t.h;
+      d[64] = t.m;
+      d[128] = t.l;
+    }
+    if constexpr (BIAS == BIAS_DENSE) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bcur[r] = bx[r] * kLog2e;
+    }
+    if constexpr (BIAS == BIAS_RELPOS) {
+      if (tid < RB) lds_rb[stage * RB + tid] = rbx * kLog2e;
+    }
+    if constexpr (MASK == MASK_KEY_MASK) {
+      if (tid < KT) lds_km[stage * KT + tid] = kmx;
+    }
+  };
+
+  if constexpr (BIAS == BIAS_RELPOS) load_bucket(0);
+  if (nstep > 0) load(0);
+
+  // ---- Q terms, pre-scaled: product step s holds dims 16s + 8*half + 0..7 of query qi
+  Split8 q[FK];
+  {
+    const float sc = q_valid ? p.scale_log2 : 0.f;
+#pragma unroll
+    for (int s = 0; s < FK; ++s) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * s + 8 * half);
+      const f32x4 c = *reinterpret_cast<const f32x4*>(qrow + 16 * s + 8 * half + 4);
+      q[s] = split8(a * sc, c * sc);
+    }
+  }
+
+  f32x16 oacc[NDB];
+#pragma unroll
+  for (int t = 0; t < NDB; ++t) oacc[t] = zero16();
+  float m = kMaxSeed;
+  float l = 0.f;
+
+  // base-2 scores of the 32 keys from k0 -> probabilities; moves (m, l, O) on
+  auto softmax = [&](float (&u)[16], int k0, bool first) {
+    if (MASK != MASK_KEY_MASK && k0 + 32 > kv_len) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + 8 * (r >> 2) + 4 * half + (r & 3);
+        u[r] = key < kv_len ? u[r] : -INFINITY;
+      }
+    }
+    float mb = u[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mb = max_nan(mb, u[r]);
+    mb = max_with_partner(mb);
+    if (first) {
+      m = max_nan(m, mb);
+    } else if (__builtin_amdgcn_ballot_w64(mb > m + kRescaleSlack) != 0) {
+      const float m_new = max_nan(m, mb);
+      const float alpha = fast_exp2(m - m_new);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int t = 0; t < NDB; ++t) oacc[t] *= alpha;
+    }
+    u[0] = fast_exp2(u[0] - m);
+    float ps = u[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) {
+      u[r] = fast_exp2(u[r] - m);
+      ps += u[r];
+    }
+    l += ps;
+  };
+
+  // scores of block blk from stage `stage`, bias and key mask added
+  auto scores = [&](int stage, float (&u)[16]) {
+    const u32x4* kb = lds + stage * STAGE + ks * BLK;
+    f32x16 s = zero16();
+#pragma unroll
+    for (int i = 0; i < FK; ++i) {
+      const u32x4* f = kb + i * 192 + half * 32 + (col ^ ((2 * i + half) & 7));
+      const u32x4 kh = f[0], km = f[64], kl = f[128];
+      s = mfma32(kl, q[i].h, s);
+      s = mfma32(kh, q[i].l, s);
+      s = mfma32(km, q[i].m, s);
+      s = mfma32(km, q[i].h, s);
+      s = mfma32(kh, q[i].m, s);
+      s = mfma32(kh, q[i].h, s);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      u[r] = s[r];
+      const int e = 8 * (r >> 2) + 4 * half + (r & 3);  // the register's key in the block
+      if constexpr (BIAS == BIAS_DENSE) u[r] += bcur[r];
+      if constexpr (BIAS == BIAS_RELPOS) u[r] += lds_rb[stage * RB + 32 * ks + e - qi + q0 + QT - 1];
+      if constexpr (MASK == MASK_KEY_MASK) u[r] += lds_km[stage * KT + 32 * ks + e];
+    }
+  };
+  auto output = [&](int stage, const float (&pr)[16]) {
+    const u32x4* vb = lds + stage * STAGE + ks * BLK + KBLK;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const Split8 pt = split8(f32x4{pr[8 * i], pr[8 * i + 1], pr[8 * i + 2], pr[8 * i + 3]},
+                               f32x4{pr[8 * i + 4], pr[8 * i + 5], pr[8 * i + 6], pr[8 * i + 7]});
+#pragma unroll
+      for (int t0 = 0; t0 < NDB; t0 += 2) {
+        u32x4 v[2][3];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 3; ++e) v[t][e] = vb[(i * NDB + t0 + t) * 192 + e * 64 + lane];
+        auto products = [&](int e, const u32x4& x) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t) oacc[t0 + t] = mfma32(v[t][e], x, oacc[t0 + t]);
+        };
+        products(2, pt.h);
+        products(0, pt.l);
+        products(1, pt.m);
+        products(1, pt.h);
+        products(0, pt.m);
+        products(0, pt.h);
+      }
+    }
+  };
+
+  if (nstep > 0) {
+    store(0);
+    if (nstep > 1) load(1);
+  }
+  __syncthreads();
+  for (int step = 0; step < nstep; ++step) {
+    const int stage = STAGES == 2 ? step & 1 : 0;
+    const int blk = step * KS + ks;
+    if (blk < nblk) {
+      float u[16];
+      scores(stage, u);
+      softmax(u, blk * 32, step == 0);
+      output(stage, u);
+    }
+    if constexpr (STAGES == 1) __syncthreads();  // every wave is done with the stage
+    if (step + 1 < nstep) {
+      store(STAGES == 2 ? stage ^ 1 : 0);
+      if (step + 2 < nstep) load(step + 2);
+    }
+    __syncthreads();
+  }
+
+  // Values without three terms (infinity, NaN, past the bfloat16 range) turn into NaN: a wave that finds
+  // anything not finite in its state takes its key blocks again with fp32 products straight from memory,
+  // so such inputs give what float32 products give.
+  {
+    float z = l * 0.f;
+#pragma unroll
+    for (int t = 0; t < NDB; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) z = fmaf(oacc[t][r], 0.f, z);
+    if (__builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0) {
+#pragma unroll
+      for (int t = 0; t < NDB; ++t) oacc[t] = zero16();
+      m = kMaxSeed;
+      l = 0.f;
+      const float sc = q_valid ? p.scale_log2 : 0.f;
+#pragma unroll 1
+      for (int blk = ks; blk < nblk; blk += KS) {
+        const float* krow = kbase + (int64_t)min(blk * 32 + col, kv_len - 1) * p.ldk;
+        f32x16 s = zero16();
+#pragma unroll 1
+        for (int d = 0; d < D; d += 2) s = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[d + half], qrow[d + half] * sc, s, 0, 0, 0);
+        float pr[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = blk * 32 + 8 * (r >> 2) + 4 * half + (r & 3), kc = min(key, p.Lk - 1);
+          pr[r] = s[r];
+          if constexpr (BIAS == BIAS_DENSE) pr[r] = fmaf(brow[kc], kLog2e, pr[r]);
+          if constexpr (BIAS == BIAS_RELPOS) {
+            const int bk = min(max(p.lut[kc - min(qi, p.Lq - 1) + p.Lq - 1], 0), p.num_buckets - 1);
+            pr[r] = fmaf(p.bias[bk * p.H + h], kLog2e, pr[r]);
+          }
+          if constexpr (MASK == MASK_KEY_MASK) pr[r] += key < p.Lk && kmask[kc] != 0 ? 0.f : -INFINITY;
+        }
+        softmax(pr, blk * 32, blk == ks);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float* vrow = vbase + (int64_t)min(blk * 32 + 8 * (r >> 2) + 4 * half + (r & 3), kv_len - 1) * p.ldv + col;
+#pragma unroll
+          for (int t = 0; t < NDB; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * t], pr[r], oacc[t], 0, 0, 0);
+        }
+      }
+    }
+  }
+
+  // ---- merge the key splits: waves ks > 0 publish (O, m, l), wave ks == 0 combines
+  float* const ldsf = reinterpret_cast<float*>(lds);
+  if constexpr (KS > 1) {
+    if (ks > 0) {
+      float* rec = ldsf + ((ks - 1) * QG + qg) * 64 * MSTRIDE + lane;
+#pragma unroll
+      for (int t = 0; t < NDB; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) rec[(16 * t + r) * 64] = oacc[t][r];
+      rec[(16 * NDB) * 64] = m;
+      rec[(16 * NDB + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (ks > 0) return;
+    float mt = m;
+#pragma unroll
+    for (int sp = 1; sp < KS; ++sp) mt = fmaxf(mt, ldsf[((sp - 1) * QG + qg) * 64 * MSTRIDE + lane + (16 * NDB) * 64]);
+    const float a0 = fast_exp2(m - mt);
+    l *= a0;
+#pragma unroll
+    for (int t = 0; t < NDB; ++t) oacc[t] *= a0;
+#pragma unroll
+    for (int sp = 1; sp < KS; ++sp) {
+      const float* o2 = ldsf + ((sp - 1) * QG + qg) * 64 * MSTRIDE + lane;
+      const float a = fast_exp2(o2[(16 * NDB) * 64] - mt);
+      l = fmaf(o2[(16 * NDB + 1) * 64], a, l);
+#pragma unroll
+      for (int t = 0; t < NDB; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[t][r] = fmaf(o2[(16 * t + r) * 64], a, oacc[t][r]);
+    }
+  }
+
+  // ---- normalise and store: lane holds O[qi][32t + 8g + 4*half + 0..3] in registers 4g..4g+3
+  const float lt = sum_with_partner(l);
+  const float inv = lt > 0.f ? __builtin_amdgcn_rcpf(lt) : 0.f;  // v_rcp_f32 (1 ulp)
+  if constexpr (KS == 1) {
+    // through LDS, as whole rows (16-byte chunks swizzled by row); each wave its own 32 x D tile
+    constexpr int CPO = D / 4;       // 16-byte chunks per row
+    constexpr int RPI = 64 / CPO;    // rows per store instruction
+    float* ot = ldsf + wave * 32 * D;
+#pragma unroll
+    for (int t = 0; t < NDB; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = {oacc[t][4 * g] * inv, oacc[t][4 * g + 1] * inv, oacc[t][4 * g + 2] * inv, oacc[t][4 * g + 3] * inv};
+        *reinterpret_cast<f32x4*>(ot + col * D + 4 * ((8 * t + 2 * g + half) ^ (col & 15))) = x;
+      }
+    const int rsub = lane / CPO, cidx = lane % CPO;
+    float* obase = p.o + (int64_t)b * p.so + h * D;
+#pragma unroll
+    for (int j = 0; j < 32 / RPI; ++j) {
+      const int row = RPI * j + rsub;
+      const f32x4 x = *reinterpret_cast<const f32x4*>(ot + row * D + 4 * (cidx ^ (row & 15)));
+      const int orow = q0 + qg * 32 + row;
+      // non-temporal: O is not read again here, and K/V tiles of the neighbouring workgroups stay in the L2
+      if (orow < p.Lq) __builtin_nontemporal_store(x, reinterpret_cast<f32x4*>(obase + (int64_t)orow * p.ldo + 4 * cidx));
+    }
+  } else if (q_valid) {
+    float* dst = p.o + (int64_t)b * p.so + (int64_t)qi * p.ldo + h * D + 4 * half;
+#pragma unroll
+    for (int t = 0; t < NDB; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = {oacc[t][4 * g] * inv, oacc[t][4 * g + 1] * inv, oacc[t][4 * g + 2] * inv, oacc[t][4 * g + 3] * inv};
+        *reinterpret_cast<f32x4*>(dst + 32 * t + 8 * g) = x;
+      }
+  }
+}
+
+template <int D, int QG, int KS, int STAGES, int WPE, int BIAS, int MASK>
+hipError_t launch_one(const AttnParams& p, hipStream_t stream) {
+  const int64_t n = (int64_t)p.B * p.H * ((p.Lq + 32 * QG - 1) / (32 * QG));
+  if (n > 0x7fffffff) return hipErrorInvalidConfiguration;
+  const FlashArgs a = flash_args(p, n);
+  const dim3 grid((unsigned)n), block(64 * QG * KS);
+  if constexpr (MASK == MASK_KEY_LEN_ORDERED) {
+    FlashOrder ord;
+    memcpy(ord.order, p.order, sizeof ord.order);
+    hipLaunchKernelGGL((flash_split_kernel<D, QG, KS, STAGES, WPE, BIAS, MASK, FlashOrder>), grid, block, 0, stream, a, ord);
+  } else {
+    hipLaunchKernelGGL((flash_split_kernel<D, QG, KS, STAGES, WPE, BIAS, MASK, NoOrder>), grid, block, 0, stream, a, NoOrder{});
+  }
+  return hipGetLastError();
+}
+
+template <int D, int QG, int KS, int STAGES, int WPE, int BIAS>
+hipError_t launch_mask(const AttnParams& p, hipStream_t stream) {
+  switch (p.mask_mode) {
+    case MASK_NONE: return launch_one<D, QG, KS, STAGES, WPE, BIAS, MASK_NONE>(p, stream);
+    case MASK_KEY_LEN:
+      if (p.order_n > 0) return launch_one<D, QG, KS, STAGES, WPE, BIAS, MASK_KEY_LEN_ORDERED>(p, stream);
+      return launch_one<D, QG, KS, STAGES, WPE, BIAS, MASK_KEY_LEN>(p, stream);
+    case MASK_KEY_MASK: return launch_one<D, QG, KS, STAGES, WPE, BIAS, MASK_KEY_MASK>(p, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int D, int QG, int KS, int STAGES, int WPE>
+hipError_t launch_bias(const AttnParams& p, hipStream_t stream) {
+  switch (p.bias_mode) {
+    case BIAS_NONE: return launch_mask<D, QG, KS, STAGES, WPE, BIAS_NONE>(p, stream);
+    case BIAS_DENSE: return launch_mask<D, QG, KS, STAGES, WPE, BIAS_DENSE>(p, stream);
+    case BIAS_RELPOS: return launch_mask<D, QG, KS, STAGES, WPE, BIAS_RELPOS>(p, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+
+// Waves per workgroup by how many 128-query units every CU gets (us, unmasked, 256 keys unless stated;
+// fp32: the fp32 MFMA flash kernel that these replace):
+//   head dim 64                    4 groups x 1   4 x 2 splits   2 x 4 splits   fp32
+//     72 units                          16.7           15.4            12.0     13.7
+//     72 units, 77 keys                  8.7            9.8             8.5      9.0
+//     192 units, 512 keys               29.5           26.5            34.9     38.7
+//     234 units                         17.0           17.0            22.8     22.1
+//     234 units, 77 keys                 9.3           10.8            15.8     14.0
+//     288 units                         24.1           30.9            33.0     32.8
+//     1026 units                        57.2           80.9            96.9     77.2
+//   head dim 128             4 x 1, two stages  4 x 1, one stage   2 x 2 splits   fp32
+//     64 units of 64, 500 keys          51.5           69.7            37.0     42.8
+//     256 units, 777 keys               87.5          124              117      142
+//     384 units, 1000 keys             195            188              206      238
+// So: at most half a unit per CU, 64-query workgroups that split the keys; one per CU, the 4 x 2 split
+// for long keys; past that 4 groups (three workgroups per CU at head dim 64, two at 128 in one stage).
+hipError_t launch_flash_split(const AttnParams& p, int num_cus, hipStream_t stream) {
+  const int64_t units = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
+  const int nblk = (p.Lk + 31) / 32;
+  if (p.D == 64) {
+    if (2 * units <= num_cus) return launch_bias<64, 2, 4, 1, 2>(p, stream);
+    if (units <= num_cus && nblk > 8) return launch_bias<64, 4, 2, 2, 2>(p, stream);
+    return launch_bias<64, 4, 1, 2, 2>(p, stream);
+  }
+  if (p.D == 128) {
+    if (2 * units <= num_cus) return launch_bias<128, 2, 2, 1, 1>(p, stream);
+    if (units <= num_cus) return launch_bias<128, 4, 1, 2, 1>(p, stream);
+    return launch_bias<128, 4, 1, 1, 2>(p, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace sa

@@ -60,54 +60,47 @@ struct FlashArgs {
   int32_t tiles;               // workgroups of the launch (the grid size, for the XCD remap)
   int16_t H, num_buckets;
   float scale_log2;
-  int32_t aux;       // start-up stagger period in workgroups (unbiased single-split kernels) | key-mask row stride
+  int32_t aux;       // key-mask row stride
   const void* mask;  // key lengths (int32) | key mask (uint8)
   const float* bias; // dense bias | relative-position table
   union {
     const int32_t* lut;  // relative-position bucket LUT
     int64_t sbias;       // dense bias batch stride
-    struct {
-      int32_t first, count;  // folded launch: the 64-query units [first, first + count) left over
-    } fold;
   };
 };
 static_assert(sizeof(FlashArgs) == 112, "flash kernel arguments must stay within 112 bytes");
 // The packed arguments of a call whose launch has `tiles` workgroups (flash_mfma_args_fit(p)).
 FlashArgs flash_args(const AttnParams& p, int64_t tiles);
 
-// Flash kernel on fp32 MFMA for D in {64, 128} with 16-byte aligned rows.
-// nsplit in {1, 2}: key blocks are split across the 4 waves of a workgroup (small head-dim-64
-// launches take flash_small instead). num_cus (the device's CU count) sets the start-up stagger of
-// the single-split kernels.
-hipError_t launch_flash_mfma(const AttnParams& p, int nsplit, int num_cus, hipStream_t stream);
+// Flash kernel on the bf16 matrix cores, three-term operands (csrc/flash_split.hip), for D in {64, 128} with
+// 16-byte aligned rows (small head-dim-64 launches take flash_small instead).
+hipError_t launch_flash_split(const AttnParams& p, int num_cus, hipStream_t stream);
+// Launch classes of that kernel (csrc/flash_mfma.hip): nsplit in {1, 2}, units of 128 / 64 queries.
 const char* flash_mfma_name(int D, int nsplit);
 // The flash kernels take 32-bit strides, at most 32767 heads and buckets; other calls take the
 // generic kernel.
 bool flash_mfma_args_fit(const AttnParams& p);
 
-// One compiled flash_mfma_kernel instantiation: <D, nsplit, bias (BIAS_*), mask (MASK_* or
-// MASK_KEY_LEN_ORDERED)>.
+// One kernel variant as plans report it: <D, nsplit, bias (BIAS_*), mask (MASK_* or MASK_KEY_LEN_ORDERED)>.
 struct FlashVariant {
   int D, nsplit, bias, mask;
 };
 // The variant a call launches with this key split.
 FlashVariant flash_mfma_variant(const AttnParams& p, int nsplit);
-// Workgroups of that launch.
+// Units of that launch class.
 int64_t flash_mfma_workgroups(const AttnParams& p, int nsplit, int num_cus);
-// Queries per workgroup of the flash kernel with this key split, and the workgroups of that variant
-// one CU holds at once (4 for the unbiased head-dim-64 single-split kernels, 1 for the others).
+// Queries per unit of a class, and the units per CU that its key-length schedule assumes (4 for unbiased
+// head-dim-64 single-split classes, 1 for the others).
 int flash_mfma_unit_queries(int nsplit);
 int flash_mfma_per_cu(const AttnParams& p, int nsplit);
-// Units (128-query tiles) of a flash launch that go to a second launch (0 = none), the kernel of
-// that launch, and the work items [*first, *first + count) it runs (returns count): 32-query groups
-// of flash_small, or 64-query units of the 2-way key-split flash kernel.
+// Units (128-query tiles) past the last whole round that a plan reports as a tail (0 = none), the kernel
+// class of that tail, and its work items [*first, *first + count) (returns count): 32-query groups or
+// 64-query units.
 constexpr int TAIL_NONE = 0, TAIL_SMALL = 1, TAIL_SPLIT2 = 2, TAIL_FOLD = 3;
 int64_t flash_mfma_tail_units(const AttnParams& p, int nsplit, int num_cus);
 int flash_mfma_tail_kernel(const AttnParams& p, int nsplit, int num_cus);
 int64_t flash_mfma_tail_groups(const AttnParams& p, int nsplit, int num_cus, int64_t* first);
-// 32-query groups [first, first + count) of the call through flash_small_kernel (no key mask).
-hipError_t launch_flash_small_groups(const AttnParams& p, int64_t first, int64_t count, hipStream_t stream);
-// Every compiled variant, in a fixed order: returns the count and fills out[0, min(count, cap)).
+// Every variant, in a fixed order: returns the count and fills out[0, min(count, cap)).
 int flash_mfma_variants(FlashVariant* out, int cap);
 
 // Small launches with head dim 64 (csrc/flash_small.hip): one workgroup per group of 32 queries,

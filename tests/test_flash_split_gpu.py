@@ -1,0 +1,73 @@
+"""Flash attention on the bf16 matrix cores (flash_split_kernel): every workgroup shape it is launched with, at
+ragged query and key lengths, each bias and mask, and values that have no three bfloat16 terms.
+
+Tolerance: scores and outputs are sums of six-term products whose dropped terms and roundings are below
+those of a float32 sum of the same length (2^-24 per addition); an error e in a score enters a
+probability as the factor 1 + e. 2e-6 in the 2-norm and 1e-5 normwise hold four times what float32
+sums of 64 to 1000 terms show."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cases import make_call
+from oracle import attention as orc
+from supra_attn import _lib
+from supra_attn.runner import Staged
+
+pytestmark = pytest.mark.gpu
+
+BIAS = [_lib.SA_BIAS_NONE, _lib.SA_BIAS_DENSE, _lib.SA_BIAS_RELPOS]
+MASK = [_lib.SA_MASK_NONE, _lib.SA_MASK_KEY_LEN, _lib.SA_MASK_KEY_MASK]
+
+# 128-query units per CU (256 CUs): under half, at most one with over 8 key blocks, and more, per head dim;
+# query and key counts that end inside a group, a block and a step (1 key past one included)
+SHAPES = [(64, 9, 5, 333, 289), (64, 12, 12, 130, 33), (64, 10, 11, 129, 321), (64, 20, 13, 131, 65),
+          (128, 3, 5, 200, 97), (128, 9, 9, 257, 161), (128, 22, 12, 150, 33)]
+
+
+def run(dev, call):
+    print(f"[flash split] {call.name} bias={call.bias_mode} mask={call.mask_mode}", flush=True)
+    st = Staged(dev, call)
+    try:
+        assert st.kernel.startswith("flash_mfma")
+        return orc.output_view(st.run(), call)
+    finally:
+        st.release()
+
+
+@pytest.mark.parametrize("mask", MASK)
+@pytest.mark.parametrize("bias", BIAS)
+@pytest.mark.parametrize("D,B,H,Lq,Lk", SHAPES)
+def test_shapes(dev, D, B, H, Lq, Lk, bias, mask):
+    lens = None
+    if mask == _lib.SA_MASK_KEY_LEN:  # none, one, a block and one more, all
+        lens = ([0, 1, 32, 33, Lk, Lk - 1] * B)[:B]
+    call = make_call(B, H, D, Lq, Lk, seed=B + Lq + Lk, packed=Lq == Lk, pad_cols=4, o_off=4, ldo_pad=8, bias_mode=bias,
+                     mask_mode=mask, key_len=lens, dense_bias_batched=B % 2 == 1)
+    e = orc.errors(run(dev, call), orc.reference_fp64(call))
+    assert e["finite"] and e["rel_l2"] <= 2e-6 and e["max_rel"] <= 1e-5, e
+
+
+@pytest.mark.parametrize("D,B,H,Lq,Lk", [(64, 9, 5, 333, 289), (64, 20, 13, 131, 65), (128, 9, 9, 257, 161)])
+def test_values_without_three_terms(dev, D, B, H, Lq, Lk):
+    """Infinities and magnitudes that round past the bfloat16 range give what float32 products give: a key
+    whose scores are -inf drops out, a query or value that is not finite shows where it reaches."""
+    call = make_call(B, H, D, Lq, Lk, seed=3)
+    k = call.k.reshape(B, Lk, H, D)
+    q = call.q.reshape(B, Lq, H, D)
+    v = call.v.reshape(B, Lk, H, D)
+    q[0, :, 0] = np.abs(q[0, :, 0]) + 0.01
+    k[0, 5, 0, 3] = -np.inf              # scores -inf for every query of that head: as if masked
+    q[1, 7, 1, 2] = np.inf               # one query's row NaN
+    v[2, 9, 2, 1] = np.inf               # one output column of every query infinite
+    v[3, 3, 3, 4] = np.nan
+    k[4, 0, 4, 0] = np.float32(3.4e38)   # finite or infinite scores, by the query's sign
+    q[4, :, 4] = -np.abs(q[4, :, 4]) * np.float32(1e-38)
+    got = run(dev, call)
+    ref = orc.reference_torch(call)
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(ref))
+    fin = np.isfinite(ref)
+    assert np.abs(got[fin] - ref[fin]).max() <= 1e-5 * np.abs(ref[fin]).max()
