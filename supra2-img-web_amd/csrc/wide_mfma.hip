@@ -2,7 +2,7 @@
 // (app/models/vae.js:86: one head, D = C = 512, 1024 tokens), which the reference sends down its
 // unfused GEMM -> softmax -> GEMM path (app/gpu/ops.js:119-147).
 //
-// Work decomposition (wide_mfma_kernel, D = 256; D = 512 runs wide_rows_kernel, described there)
+// Work decomposition (wide_mfma_kernel, D = 256; D = 512 runs wide_split_kernel, described there)
 //   One workgroup = NW = 4 wave64s = 32 queries x one chunk of keys. Wave w owns the head-dim
 //   slice [w*D/NW, (w+1)*D/NW) of Q, K, V and O:
 //   per 32-key block it computes the partial score tile S_w^T = K_w Q_w^T over its slice
@@ -26,6 +26,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "split.h"
 
 namespace sa {
 
@@ -41,6 +42,19 @@ __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// Asks the scheduler for N times one MFMA and V VALU instructions, in turn.
+template <int N, int V>
+__device__ __forceinline__ void mix() {
+  static_for<N>([](auto) {
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x2, V, 0);
+  });
+}
+
+__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 __device__ __forceinline__ f32x16 zero16() {
@@ -418,31 +432,34 @@ __global__ __launch_bounds__(64 * NW, 1) void wide_mfma_kernel(WideArgs p) {
   }
 }
 
-// D = 512: one workgroup = 4 waves = 32 queries x one chunk of keys, taken in rounds of four
-// 32-key blocks. In a round wave w computes the whole score tile of block w over all 512 head
-// dims (256 MFMAs in two independent chains: K rows straight from memory into registers, Q^T from
-// a copy of the query tile in LDS), the four block maxima and row sums meet in LDS (one reference
-// m per query for the round, so the probabilities need no lazy rescale inside it), each wave
-// publishes its probabilities, and wave w then accumulates O^T for its quarter of the head dims
-// over all four blocks (V rows straight into registers, prefetched a block ahead, with head dim
-// 4i + t of the quarter on row i of output tile t, so one 16-byte load feeds the four tiles).
-// Each probability is computed once per round, where the head-dim-split kernel above summed
-// partial score tiles through LDS and took the softmax in every wave for every block; one wave
-// per SIMD, its loads software-pipelined. Writes the same partial records as wide_mfma_kernel
-// (merged by wide_merge_kernel), staged through LDS into whole-row stores.
+// D = 512, on the bf16 matrix cores with three-term operands (split.h; six term products per product,
+// smallest first): one workgroup = 8 waves = 32 queries x one chunk of keys, in rounds of four 32-key blocks.
+// In a round wave w computes a quarter of the head dims (128 (w % 4)) of the score tiles of two blocks
+// (2 (w / 4) and the next); the four quarter sums meet in LDS, and each wave finishes 16 keys of one block:
+// maxima and row sums of all waves give one reference m per query for the round. Each wave
+// publishes its probabilities, split once, and accumulates O^T for 64 head dims over all four blocks. Head
+// dim 2i + t of those sits on row i of output tile t, so an 8-byte load of a V row feeds both tiles.
+// K and V rows come straight from memory into registers, pipelined ahead of their products, and are split
+// there: with 32 queries per workgroup every element is used once, 7 VALU instructions per MFMA, put
+// between the products that cover them. That is what bounds it: a wave alone issues one of them per
+// 6 cycles, two waves per SIMD one per 4.4, so 8 waves and not 4 (4096 tokens, the whole call: 331 against 345 us; fp32
+// products: 401). Q is split once, into LDS; two blocks per wave halve its reads, which at one block
+// would take LDS (64 bytes per clock and CU) as long as the MFMAs.
+// Writes the same partial records as wide_mfma_kernel (merged by wide_merge_kernel).
 template <int BIAS, int MASK>
-__global__ __launch_bounds__(256, 1) void wide_rows_kernel(WideArgs p) {
+__global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
   constexpr int D = 512;
-  constexpr int NG = D / 8;          // groups of 8 head dims (4 MFMAs) per score tile
-  constexpr int DS = D / 4;          // output head dims per wave
+  constexpr int DS = D / 8;          // output head dims per wave
+  constexpr int NS = D / 64;         // product steps of a quarter of the head dims
   constexpr int REC = 32 * D + 64;   // workspace floats per partial: O [32][D], m [32], l [32]
-  constexpr int KR = 8;              // K groups in flight ahead of the MFMAs (16 measured no faster)
-  constexpr int NQ = 32 * D / 4 / 256;  // 16-byte Q chunks per thread
+  constexpr int KR = 3;              // product steps whose K loads are in flight
 
-  __shared__ __attribute__((aligned(16))) float lds_q[32 * D];      // [quarter][query][128], then the output
-  __shared__ __attribute__((aligned(16))) f32x4 lds_p[4 * 4 * 64];  // [block][r/4][lane]
-  __shared__ float lds_m[4 * 32];                                   // [block][query]
-  __shared__ float lds_l[4 * 32];
+  __shared__ u32x4 lds_q[D / 16 * 3 * 64];  // [product step][term][half][query ^ chunk], then the output
+  __shared__ u32x4 lds_p[8 * 3 * 2 * 64];   // probability terms [16 keys][term][lane] (8 * 3 * 64); before that
+                                            // the quarter sums [wave][neighbour][2][lane]
+  __shared__ float lds_m[8 * 32];           // [16 keys][query]
+  __shared__ float lds_l[8 * 32];
+  __shared__ int lds_bad;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -471,215 +488,313 @@ __global__ __launch_bounds__(256, 1) void wide_rows_kernel(WideArgs p) {
   constexpr bool kTerms = Terms::kBias || Terms::kMask;
   const typename Terms::Rows trows = Terms::rows(p, b, h, q0 + col);
 
+  const float* qbase = p.q + (int64_t)b * p.sq + h * D;
   const float* kbase = p.k + (int64_t)b * p.sk + h * D;
   const float* vbase = p.v + (int64_t)b * p.sv + h * D + wave * DS;
 
-  // ---- Q tile (rows past Lq re-read the last row) into registers, then into LDS a quarter of 128
-  // head dims at a time as the score products reach it: [quarter][query][32 chunks of 16 bytes],
-  // chunk c of row r at c ^ (r & 15). Thread t holds physical chunks n*256 + t (n = 0..15), so
-  // quarter k is its registers 4k..4k+3. (Copies straight into LDS would make the compiler wait
-  // for all of them, and the K loads behind them, before the first LDS read.)
-  f32x4 qst[NQ];
-  {
-    const float* qbase = p.q + (int64_t)b * p.sq + h * D;
+  // ---- K of product step i (dims 128 (w % 4) + 16 i + 8 half + 0..7) of blocks 2 (w / 4) + 0 and 1: rows
+  // past the chunk's last key re-read it
+  f32x4 kring[KR][2][2];
+  const float* kr[2];
+  auto aim_k = [&](int rb0) {
 #pragma unroll
-    for (int n = 0; n < NQ; ++n) {
-      const int pc = (n & 3) * 256 + tid;  // physical chunk within quarter n / 4
-      const int row = pc >> 5;
-      const int c = 32 * (n >> 2) + ((pc & 31) ^ (row & 15));
-      qst[n] = *reinterpret_cast<const f32x4*>(qbase + (int64_t)min(q0 + row, p.Lq - 1) * p.ldq + 4 * c);
-    }
-  }
-
-  // V rows of one block for this wave's head dims: register r holds V[key][4*col .. 4*col + 3] of
-  // key 8(r/4) + 4*half + r%4 of the block. The buffer ends after the chunk's last valid key, so
-  // rows past it read as zeros (their probabilities are zero) and no load needs a branch: a
-  // conditional load is sunk by the compiler to its first use, which would undo the prefetch.
+    for (int e = 0; e < 2; ++e)
+      kr[e] = kbase + (int64_t)min(rb0 + 64 * (wave >> 2) + 32 * e + col, kend - 1) * p.ldk + 128 * (wave & 3) + 8 * half;
+  };
+  auto load_k = [&](int i) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) kring[i % KR][e][x] = *reinterpret_cast<const f32x4*>(kr[e] + 16 * i + 4 * x);
+  };
+  // V rows of one block for this wave's head dims: register r holds V[key][2*col, 2*col + 1] of key
+  // 8(r/4) + 4*half + r%4 of the block (the keys of score register r). The buffer ends after the chunk's
+  // last valid key, so rows past it read as zeros and no load needs a branch.
   unsigned vrow_off[16];  // byte offset of register r's row and columns from the block's first row
 #pragma unroll
-  for (int r = 0; r < 16; ++r) vrow_off[r] = 4u * (unsigned)((4 * half + 8 * (r >> 2) + (r & 3)) * (int)p.ldv + 4 * col);
-  auto load_v = [&](int kb0, f32x4* dst) {
-    // (in a scalar register: a clamp the compiler computes on the vector unit would make the
-    // descriptor look divergent and every load a waterfall loop)
+  for (int r = 0; r < 16; ++r) vrow_off[r] = 4u * (unsigned)((4 * half + 8 * (r >> 2) + (r & 3)) * (int)p.ldv + 2 * col);
+  auto load_v = [&](int kb0, f32x2* dst) {
+    // (in a scalar register: a clamp on the vector unit would make every load a waterfall loop)
     const int rows = __builtin_amdgcn_readfirstlane(max(0, min(32, kend - kb0)));
     const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(vbase + (int64_t)kb0 * p.ldv), 0, rows * (int)p.ldv * 4, 0x00020000);
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-      dst[r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, vrow_off[r], 0, 0));
+      dst[r] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(vr, vrow_off[r], 0, 0));
   };
 
-  f32x16 oacc[4];
+  if (rounds > 0) {
+    aim_k(kbeg);
 #pragma unroll
-  for (int t = 0; t < 4; ++t) oacc[t] = zero16();
+    for (int i = 0; i < KR; ++i) load_k(i);
+  }
+  // ---- Q terms into LDS, pre-scaled (rows past Lq re-read the last row)
+  if (tid == 0) lds_bad = 0;
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const int row = (n * 512 + tid) >> 6, c = lane;
+    const float* src = qbase + (int64_t)min(q0 + row, p.Lq - 1) * p.ldq + 8 * c;
+    const Split8 t = split8(*reinterpret_cast<const f32x4*>(src) * p.scale_log2,
+                            *reinterpret_cast<const f32x4*>(src + 4) * p.scale_log2);
+    u32x4* d = lds_q + (c >> 1) * 192 + (c & 1) * 32 + (row ^ (c & 31));
+    d[0] = t.h;
+    d[64] = t.m;
+    d[128] = t.l;
+  }
+  __syncthreads();
+
+  f32x16 oacc[2] = {zero16(), zero16()};
   float m = kMaxSeed;
   float l = 0.f;
-  // the swizzled Q chunk 2i + half of this lane's query (quarter i / 16)
-  const float* qrow = lds_q + col * 128;
+  const int blk = 2 * (wave >> 2) + ((wave >> 1) & 1), sub = wave & 1;  // the 16 keys this wave finishes
 
   for (int rd = 0; rd < rounds; ++rd) {
     const int rb0 = kbeg + 128 * rd;  // first key of the round
-    if (rd > 0) __syncthreads();      // every wave is done with the previous round's exchange
-    const int kb0 = rb0 + 32 * wave;  // this wave's score block
-    const bool has_keys = kb0 < kend;  // false for the missing blocks of a short last round
-    // K rows of the block (clamped past the chunk's last key), 16 bytes per group of 8 dims
-    const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(kbase + (int64_t)kb0 * p.ldk);
-    const unsigned koff = 4u * (unsigned)((min(kb0 + col, kend - 1) - kb0) * (int)p.ldk + 4 * half);
-    auto load_k = [&](int i) {
-      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(kr, koff + 32u * i, 0, 0));
-    };
-    f32x4 kring[KR];
-    Terms terms;  // the block's bias / mask terms, used after its score products
-    if (has_keys) {
-      if constexpr (kTerms) terms.load(trows, kb0, half);
+    const int kb0 = rb0 + 32 * blk;   // the block this wave finishes 16 keys of
+    Terms terms;                      // its bias / mask terms, used after the score products
+    if constexpr (kTerms) terms.load(trows, kb0, half);
+    f32x2 vbuf[2][16];  // V of the round's blocks, double-buffered
+    f32x16 s[2] = {zero16(), zero16()};
+    if (rb0 + 64 * (wave >> 2) < kend) {
+      auto read_q = [&](int i, u32x4 (&x)[3]) {
+        const int ii = NS * (wave & 3) + i;
+        const u32x4* f = lds_q + ii * 192 + half * 32 + (col ^ ((2 * ii + half) & 31));
 #pragma unroll
-      for (int i = 0; i < KR; ++i) kring[i] = load_k(i);
-    }
-    // round 0 publishes the Q quarters as the products reach them
-    auto q_quarter = [&](auto k) {
-      constexpr int kq = decltype(k)::value;
-      if (rd == 0) {
-#pragma unroll
-        for (int n = 4 * kq; n < 4 * kq + 4; ++n) *reinterpret_cast<f32x4*>(lds_q + n * 1024 + 4 * tid) = qst[n];
-        __syncthreads();
-      }
-    };
-    q_quarter(std::integral_constant<int, 0>{});
-    f32x4 vbuf[2][16];  // V of the round's blocks, double-buffered
-    float u[16];
-    if (has_keys) {
-      f32x16 sa = zero16(), sb = zero16();
-      auto read_q = [&](int i) {
-        return *reinterpret_cast<const f32x4*>(qrow + (i >> 4) * 4096 + 4 * ((2 * (i & 15) + half) ^ (col & 15)));
+        for (int t = 0; t < 3; ++t) x[t] = f[64 * t];
       };
-      // Groups in pairs, group i into sa and i + 1 into sb (the compiler orders the products; pinning
-      // them to alternate between the chains measured the same). The Q operands of the next pair
-      // are read during this one.
-      f32x4 qn0 = read_q(0), qn1 = read_q(1);
-      static_for<NG / 2>([&](auto I) {
-        constexpr int i = 2 * decltype(I)::value;
-        const f32x4 k0v = kring[i % KR], k1v = kring[(i + 1) % KR];
-        const f32x4 q0v = qn0, q1v = qn1;
-        if constexpr (i + KR < NG) {
-          kring[i % KR] = load_k(i + KR);
-          kring[(i + 1) % KR] = load_k(i + 1 + KR);
-        }
-        if constexpr (i == NG - 16) load_v(rb0, vbuf[0]);  // the round's first V block streams in under the last products
-        if constexpr (i + 2 < NG) {
-          if constexpr ((i + 2) % 16 == 0) q_quarter(std::integral_constant<int, (i + 2) / 16>{});
-          qn0 = read_q(i + 2);
-          qn1 = read_q(i + 3);
-        }
+      u32x4 qx[2][3];
+      Split8 kx[2][2];
+      read_q(0, qx[0]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          sa = __builtin_amdgcn_mfma_f32_32x32x2f32(k0v[j], q0v[j], sa, 0, 0, 0);
-          sb = __builtin_amdgcn_mfma_f32_32x32x2f32(k1v[j], q1v[j], sb, 0, 0, 0);
+      for (int e = 0; e < 2; ++e) kx[0][e] = split8(kring[0][e][0], kring[0][e][1]);
+      static_for<NS>([&](auto I) {
+        constexpr int i = decltype(I)::value, cur = i & 1;
+        if constexpr (i + KR < NS) load_k(i + KR);
+        if constexpr (i == NS - 3) load_v(rb0, vbuf[0]);  // the round's first V block streams in under the last products
+        if constexpr (i + 1 < NS) {
+          read_q(i + 1, qx[cur ^ 1]);
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            kx[cur ^ 1][e] = split8(kring[(i + 1) % KR][e][0], kring[(i + 1) % KR][e][1]);
         }
-        // keeps each load where it is issued: left free, the scheduler sinks the ring's loads to
-        // just before their use, one group ahead of the products
+        auto products = [&](auto kt, int qt) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) s[e] = mfma32(kt(kx[cur][e]), qx[cur][qt], s[e]);
+        };
+        products([](const Split8& x) { return x.l; }, 0);
+        products([](const Split8& x) { return x.h; }, 2);
+        products([](const Split8& x) { return x.m; }, 1);
+        products([](const Split8& x) { return x.m; }, 0);
+        products([](const Split8& x) { return x.h; }, 1);
+        products([](const Split8& x) { return x.h; }, 0);
+        if constexpr (i + 1 < NS) mix<12, 8>();
+        // keeps each load where it is issued (left free, the scheduler sinks loads to their use)
         __builtin_amdgcn_sched_barrier(0);
       });
-#pragma unroll
-      for (int r = 0; r < 16; ++r) u[r] = (sa[r] + sb[r]) * p.scale_log2;
-      if constexpr (kTerms) terms.apply(u);
-      if (kb0 + 32 > kend) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb0 + 8 * (r >> 2) + 4 * half + (r & 3);
-          u[r] = key < kend ? u[r] : -INFINITY;
-        }
-      }
     } else {
-      // the score-less wave still takes part in round 0's quarter barriers
-      q_quarter(std::integral_constant<int, 1>{});
-      q_quarter(std::integral_constant<int, 2>{});
-      q_quarter(std::integral_constant<int, 3>{});
       load_v(rb0, vbuf[0]);
+    }
+    // ---- quarter sums of the other three waves' 16 keys (wave ^ x finishes block (.. ^ x) / 2, half (.. ^ x) % 2)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) u[r] = -INFINITY;
+    for (int x = 1; x < 4; ++x) {
+      const int to = (wave & 3) ^ x;
+      u32x4* out = lds_p + (wave * 3 + x - 1) * 128 + lane;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        f32x4 v;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float lo = (to & 1) ? s[0][8 + 4 * e + c] : s[0][4 * e + c];
+          const float hi = (to & 1) ? s[1][8 + 4 * e + c] : s[1][4 * e + c];
+          v[c] = (to & 2) ? hi : lo;
+        }
+        out[64 * e] = __builtin_bit_cast(u32x4, v);
+      }
+    }
+    float u[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const float lo = sub ? s[0][8 + r] : s[0][r], hi = sub ? s[1][8 + r] : s[1][r];
+      u[r] = (wave & 2) ? hi : lo;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 1; x < 4; ++x) {
+      const u32x4* in = lds_p + ((wave ^ x) * 3 + x - 1) * 128 + lane;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const f32x4 v = __builtin_bit_cast(f32x4, in[64 * e]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) u[4 * e + c] += v[c];
+      }
+    }
+    if constexpr (kTerms) {  // of the block's 16 registers per lane, this wave's 8
+      float w[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) w[r] = u[r & 7];
+      terms.apply(w);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) u[r] = sub ? w[8 + r] : w[r];
+    }
+    if (kb0 + 32 > kend) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const int key = kb0 + 16 * sub + 8 * (r >> 2) + 4 * half + (r & 3);
+        u[r] = key < kend ? u[r] : -INFINITY;
+      }
+    }
+    if (rd + 1 < rounds) {  // the next round's first K rows stream in under the rest of this one
+      aim_k(rb0 + 128);
+#pragma unroll
+      for (int i = 0; i < KR; ++i) load_k(i);
     }
     // ---- one reference per query for the round: the maximum over the four blocks
     float mb = u[0];
 #pragma unroll
-    for (int r = 1; r < 16; ++r) mb = max_nan(mb, u[r]);
+    for (int r = 1; r < 8; ++r) mb = max_nan(mb, u[r]);
     mb = max_with_partner(mb);
     if (half == 0) lds_m[wave * 32 + col] = mb;
-    __syncthreads();
-    float m_new = max_nan(m, lds_m[col]);
-    m_new = max_nan(m_new, lds_m[32 + col]);
-    m_new = max_nan(m_new, lds_m[64 + col]);
-    m_new = max_nan(m_new, lds_m[96 + col]);
+    __syncthreads();  // also: every quarter sum has been read
+    float m_new = m;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) m_new = max_nan(m_new, lds_m[32 * w + col]);
     if (rd > 0) {
       const float alpha = fast_exp2(m - m_new);
       l *= alpha;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) oacc[t] *= alpha;
+      oacc[0] *= alpha;
+      oacc[1] *= alpha;
     }
     m = m_new;
     float ps = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
+    for (int r = 0; r < 8; ++r) {
       u[r] = fast_exp2(u[r] - m);
       ps += u[r];
     }
     ps = sum_with_partner(ps);
     if (half == 0) lds_l[wave * 32 + col] = ps;
-#pragma unroll
-    for (int k4 = 0; k4 < 4; ++k4) {
-      f32x4 x;
-      x[0] = u[4 * k4 + 0];
-      x[1] = u[4 * k4 + 1];
-      x[2] = u[4 * k4 + 2];
-      x[3] = u[4 * k4 + 3];
-      lds_p[(wave * 4 + k4) * 64 + lane] = x;
+    {
+      const Split8 t = split8(f32x4{u[0], u[1], u[2], u[3]}, f32x4{u[4], u[5], u[6], u[7]});
+      u32x4* d = lds_p + (blk * 2 + sub) * 192 + lane;
+      d[0] = t.h;
+      d[64] = t.m;
+      d[128] = t.l;
     }
     __syncthreads();
-    l += lds_l[col] + lds_l[32 + col] + lds_l[64 + col] + lds_l[96 + col];
-    // ---- O^T += V^T P^T over the round's blocks, this wave's 128 head dims; the next block's V
-    // is requested before this block's products (a zero-row buffer past the keys: no access)
-    float pr[4][16];
+    {
+      float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int k4 = 0; k4 < 4; ++k4) {
-        const f32x4 x = lds_p[(j * 4 + k4) * 64 + lane];
-        pr[j][4 * k4 + 0] = x[0];
-        pr[j][4 * k4 + 1] = x[1];
-        pr[j][4 * k4 + 2] = x[2];
-        pr[j][4 * k4 + 3] = x[3];
-      }
+      for (int w = 0; w < 8; ++w) sum += lds_l[32 * w + col];
+      l += sum;
+    }
+    // ---- O^T += V^T P^T over the round's blocks, this wave's 64 head dims, 16 keys (8 registers per lane) at a
+    // time; the next block's V is requested before this block's products
     static_for<4>([&](auto J) {
       constexpr int j = decltype(J)::value;
       if constexpr (j + 1 < 4) load_v(rb0 + 32 * (j + 1), vbuf[(j + 1) & 1]);
       __builtin_amdgcn_sched_barrier(0);
       if (rb0 + 32 * j < kend) {  // wave-uniform: blocks past the chunk's keys hold no probabilities
+        Split8 vx[2][2];
+        u32x4 px[2][3];
+        auto prep = [&](auto I) {
+          constexpr int i = decltype(I)::value;
+          const f32x2* vb = vbuf[j & 1] + 8 * i;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+          for (int t = 0; t < 2; ++t)
+            vx[i][t] = split8(f32x4{vb[0][t], vb[1][t], vb[2][t], vb[3][t]}, f32x4{vb[4][t], vb[5][t], vb[6][t], vb[7][t]});
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
-            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vbuf[j & 1][r][t], pr[j][r], oacc[t], 0, 0, 0);
-        }
+          for (int t = 0; t < 3; ++t) px[i][t] = lds_p[(j * 2 + i) * 192 + 64 * t + lane];
+        };
+        prep(std::integral_constant<int, 0>{});
+        static_for<2>([&](auto I) {
+          constexpr int i = decltype(I)::value;
+          if constexpr (i == 0) prep(std::integral_constant<int, 1>{});
+          auto products = [&](auto vt, int pt) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) oacc[t] = mfma32(vt(vx[i][t]), px[i][pt], oacc[t]);
+          };
+          products([](const Split8& v) { return v.l; }, 0);
+          products([](const Split8& v) { return v.h; }, 2);
+          products([](const Split8& v) { return v.m; }, 1);
+          products([](const Split8& v) { return v.m; }, 0);
+          products([](const Split8& v) { return v.h; }, 1);
+          products([](const Split8& v) { return v.h; }, 0);
+          if constexpr (i == 0) mix<12, 8>();
+          __builtin_amdgcn_sched_barrier(0);
+        });
       }
-      __builtin_amdgcn_sched_barrier(0);
     });
+    if (rd + 1 < rounds) __syncthreads();  // every wave is done with the round's exchange
   }
 
-  // ---- output: O^T tile t, register r holds head dim wave*128 + 4i + t of query col, with
-  // i = 8(r/4) + 4*half + r%4, so the four tiles' register r are four consecutive head dims.
-  // The wave stages its 32 x 128 slice in LDS (the Q tile is dead: every wave has passed the
-  // last exchange, after its score products), 16-byte chunk i of query q at i ^ q, and stores
-  // it back as 512-byte row pieces, two rows per instruction, instead of 16 bytes of 32 rows.
-  const float inv = nks == 1 ? (l > 0.f ? 1.f / l : 0.f) : 1.f;
-  float* stage = lds_q + wave * 32 * DS;
+  // Values without three terms (infinity, NaN, past the bfloat16 range) turn into NaN: if any wave finds
+  // anything not finite in its state, all take the chunk again with fp32 products straight from memory.
+  {
+    float z = l * 0.f;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int i = 8 * (r >> 2) + 4 * half + (r & 3);
-    f32x4 x;
-    x[0] = oacc[0][r] * inv;
-    x[1] = oacc[1][r] * inv;
-    x[2] = oacc[2][r] * inv;
-    x[3] = oacc[3][r] * inv;
-    *reinterpret_cast<f32x4*>(stage + col * DS + 4 * (i ^ col)) = x;
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) z = fmaf(oacc[t][r], 0.f, z);
+    if (__builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0 && lane == 0) lds_bad = 1;
+    __syncthreads();  // also: every wave is done with the Q terms
+    if (lds_bad != 0) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) oacc[t] = zero16();
+      m = kMaxSeed;
+      l = 0.f;
+      const float* qrow = qbase + (int64_t)min(q0 + col, p.Lq - 1) * p.ldq;
+#pragma unroll 1
+      for (int kb = kbeg; kb < kend; kb += 32) {
+        const float* krow = kbase + (int64_t)min(kb + col, kend - 1) * p.ldk;
+        f32x16 s = zero16();
+#pragma unroll 1
+        for (int d = 0; d < D; d += 2) s = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[d + half], qrow[d + half], s, 0, 0, 0);
+        Terms terms;
+        if constexpr (kTerms) terms.load(trows, kb, half);
+        float u[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) u[r] = s[r] * p.scale_log2;
+        if constexpr (kTerms) terms.apply(u);
+        float mb = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          u[r] = kb + 8 * (r >> 2) + 4 * half + (r & 3) < kend ? u[r] : -INFINITY;
+          mb = max_nan(mb, u[r]);
+        }
+        const float m_new = max_nan(m, max_with_partner(mb));
+        const float alpha = fast_exp2(m - m_new);
+        l *= alpha;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) oacc[t] *= alpha;
+        m = m_new;
+        float ps = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          u[r] = fast_exp2(u[r] - m);
+          ps += u[r];
+        }
+        l += sum_with_partner(ps);
+        f32x2 vb[16];
+        load_v(kb, vb);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[r][t], u[r], oacc[t], 0, 0, 0);
+      }
+    }
+  }
+
+  // ---- output: O^T tile t, register r holds head dim 64*wave + 2i + t of query col, with
+  // i = 8(r/4) + 4*half + r%4, so the two tiles' registers r and r + 1 (r even) are four consecutive head
+  // dims. The wave stages its 32 x 64 slice in LDS (the Q terms are dead), 16-byte chunk c of query q
+  // at c ^ (q & 15), and stores it back as 256-byte row pieces, four rows per instruction.
+  const float inv = nks == 1 ? (l > 0.f ? 1.f / l : 0.f) : 1.f;
+  float* stage = reinterpret_cast<float*>(lds_q) + wave * 32 * DS;
+#pragma unroll
+  for (int r = 0; r < 16; r += 2) {
+    const int c = 4 * (r >> 2) + 2 * half + ((r & 3) >> 1);
+    const f32x4 x = {oacc[0][r] * inv, oacc[1][r] * inv, oacc[0][r + 1] * inv, oacc[1][r + 1] * inv};
+    *reinterpret_cast<f32x4*>(stage + col * DS + 4 * (c ^ (col & 15))) = x;
   }
   float* dst;
   int64_t ld;
@@ -696,10 +811,10 @@ __global__ __launch_bounds__(256, 1) void wide_rows_kernel(WideArgs p) {
     }
   }
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int row = 2 * j + half;  // query q0 + row; lane col holds chunk col of it
-    const f32x4 x = *reinterpret_cast<const f32x4*>(stage + row * DS + 4 * (col ^ row));
-    if (nks > 1 || q0 + row < p.Lq) *reinterpret_cast<f32x4*>(dst + (int64_t)row * ld + 4 * col) = x;
+  for (int j = 0; j < 8; ++j) {
+    const int row = 4 * j + (lane >> 4), c = lane & 15;
+    const f32x4 x = *reinterpret_cast<const f32x4*>(stage + row * DS + 4 * (c ^ (row & 15)));
+    if (nks > 1 || q0 + row < p.Lq) *reinterpret_cast<f32x4*>(dst + (int64_t)row * ld + 4 * c) = x;
   }
 }
 
@@ -778,14 +893,14 @@ __global__ __launch_bounds__(256) void wide_merge_kernel(MergeArgs p) {
 
 // Waves per workgroup of the head-dim-split kernel (D = 256): each owns D / 4 head dims, 80 KiB of
 // LDS, two workgroups per CU. (At D = 512 it ran 8 waves, two per SIMD, in 160 KiB: VAE call
-// 34.9 us against 29.9 for wide_rows_kernel.)
+// 34.9 us against 29.9 for whole score tiles per wave, as wide_split_kernel has them.)
 template <int D>
 constexpr int kWideWaves = 4;
 
 template <int D, int BIAS, int MASK>
 void launch_main(const WideArgs& a, dim3 grid, hipStream_t stream) {
   if constexpr (D == 512)
-    hipLaunchKernelGGL((wide_rows_kernel<BIAS, MASK>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((wide_split_kernel<BIAS, MASK>), grid, dim3(512), 0, stream, a);
   else
     hipLaunchKernelGGL((wide_mfma_kernel<D, kWideWaves<D>, BIAS, MASK>), grid, dim3(64 * kWideWaves<D>), 0, stream, a);
 }
@@ -907,7 +1022,7 @@ WidePlan wide_mfma_plan(const AttnParams& p, int num_cus) {
   const int64_t base = (int64_t)p.B * p.H * plan.q_groups;
   const int64_t slots = (int64_t)num_cus * (p.D == 512 ? 1 : 2);
   const int nblk = (p.Lk + 31) / 32;
-  // D = 512 takes keys in rounds of four blocks (wide_rows_kernel): chunks of whole rounds
+  // D = 512 takes keys in rounds of four blocks (wide_split_kernel): chunks of whole rounds
   const int unit = p.D == 512 ? 4 : 1;
   const int64_t rec_bytes = (int64_t)(32 * p.D + 64) * (int64_t)sizeof(float);
   auto rounds = [&](int64_t wgs) { return (double)((wgs + slots - 1) / slots); };
