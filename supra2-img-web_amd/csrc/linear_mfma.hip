@@ -136,6 +136,34 @@ constexpr int split_waves_per_simd() {
   return MT * NT <= 6 ? 4 : MT * NT <= 12 ? 3 : 2;
 }
 
+// Rows [m0, m0 + rows) x columns [n0, n0 + cols) in fp32 products straight from memory, by one wave (lane =
+// 16 lc + lr), 16 x 16 outputs at a time and stored from here: merged with the caller's accumulators and
+// epilogue instead, it cost the main loop up to 6% (fc2 of 16384 rows 209 -> 196 us without).
+template <int ACT, int EPI>
+__device__ __forceinline__ void redo_tile(const LinArgs& p, int m0, int n0, int rows, int cols, int lr, int lc) {
+#pragma unroll 1
+  for (int mt = m0; mt < min(m0 + rows, p.M); mt += 16) {
+#pragma unroll 1
+    for (int nt = n0; nt < min(n0 + cols, p.N); nt += 16) {
+      const float* x = p.x + (int64_t)min(mt + lr, p.M - 1) * p.ldx + lc;
+      const float* w = p.w + (int64_t)min(nt + lr, p.N - 1) * p.ldw + lc;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int k = 0; k < p.K; k += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[k], x[k], acc, 0, 0, 0);
+      const int m = mt + lr;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = nt + 4 * lc + e;
+        if (m >= p.M || n >= p.N) continue;
+        float v = apply_act<ACT>(fmaf(acc[e], p.alpha, p.bias ? p.bias[n] : 0.f));
+        const int64_t at = (int64_t)m * p.ldy + n;
+        if constexpr (EPI != LIN_EPI_STORE) v = fmaf(EPI == LIN_EPI_RESID_GATE ? p.gate[n] : 1.f, v, p.resid[at]);
+        p.y[at] = v;
+      }
+    }
+  }
+}
+
 // Large and medium grids: the product on the bf16 matrix cores, each float32 operand as three bfloat16
 // terms (split.h) and each product as the six term products of 2^-24 and more of its size, smallest
 // first, summed in the float32 accumulators: x w ~ xl wh + xh wl + xm wm + xm wh + xh wm + xh wh.
@@ -295,26 +323,8 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
 #pragma unroll
       for (int e = 0; e < 4; ++e) z = fmaf(acc[i][j][e], 0.f, z);
   if (__builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float* xrow[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) xrow[i] = p.x + (int64_t)min(mw + 16 * i + lr, p.M - 1) * p.ldx + lc;
-    const float* w0 = p.w + (int64_t)n0 * p.ldw + lc;
-#pragma unroll 1
-    for (int k = 0; k < p.K; k += 4) {
-      float xv[MT];
-#pragma unroll
-      for (int i = 0; i < MT; ++i) xv[i] = xrow[i][k];
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const float wv = w0[(int64_t)min(16 * j + lr, p.N - 1 - n0) * p.ldw + k];
-#pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv[i], acc[i][j], 0, 0, 0);
-      }
-    }
+    redo_tile<ACT, EPI>(p, mw, n0, 16 * MT, BN, lr, lc);
+    return;
   }
 
   // ---- epilogue: lane holds columns n0 + 16j + 4*lc .. +3 of row mw + 16i + lr. Rows, bias and gate are
