@@ -968,16 +968,18 @@ bool linear_mfma_supported(const LinearParams& p) {
 
 // Size class of a call: the tile of the fp32 kernels that its grid fills, and the kernel's name in the
 // API. Classes 128 x 192 and 64 x 192 (at least one 128 x 192 tile per CU, or three 64 x 192 ones) run
-// linear_split_kernel, class 64 x 64 linear_split_kernel or linear_mfma_kernel (split_tile below).
+// linear_split_kernel, class 64 x 64 that or linear_mfma_kernel, the 32 x 64 class that or
+// linear_ksplit_kernel (split_tile below).
 // Grids of fewer 64 x 64 tiles than 1.25 per CU take linear_ksplit_kernel, whose quarter-K waves
 // spread them over the SIMDs (us, 64 x 64 -> k-split: VAE output projection 1024 x 512 x 512 11.75 ->
 // 8.1, context k|v 77 x 1152 x 576 13.2 -> 6.3, batch-2 proj/q/cproj 512 x 576 x 576 12.6-13.0 ->
 // 8.4-8.7, fc1 512 x 2304 x 576 21.4 -> 19.2, fc2 512 x 576 x 2304 43.4 -> 23.0). Grids of 1.25 to 2
-// such tiles per CU take 32 x 64 tiles with k split in two, whose count is twice that and so shares
+// such tiles per CU are the class of 32 x 64 tiles with k split in two, whose count is twice that and so shares
 // out more evenly over the CUs (VAE q|k|v 1024 x 1536 x 512, 384 tiles: 64 x 64 18.7-19.2, 32 x 64 /
 // two splits 17.4, 64 x 32 17.5, 64 x 32 / four splits 17.9, 64 x 64 / two splits 20.7, 32 x 32 / four
-// splits 18.9-19.4). The split kernel's smallest tiles (64 x 48) measured slower than both there: 13-20
-// against 6-15 us at K = 576, its loads being one k-tile ahead.
+// splits 18.9-19.4). The split kernel's smallest tiles (64 x 48, 32 x 48) measured slower on the small grids:
+// 13-20 against 6-15 us at K = 576, with one, two or four k-tiles of loads in flight alike: a wave alone
+// on its SIMD issues one VALU instruction per 6 cycles, and the splits are most of its work.
 LinearTile linear_mfma_tile(const LinearParams& p, int num_cus) {
   const int64_t tiles_wide = ((p.M + 127) / 128) * ((p.N + 191) / 192);
   const int64_t tiles_tall = ((p.M + 63) / 64) * ((p.N + 191) / 192);
@@ -998,12 +1000,15 @@ namespace {
 //   256 x 192, 8 waves: 70 / 249
 //   128 x 96, 4 waves:  35 / 120, 45 / 152, 56 / 213 for 1, 2, 3 tiles on a CU at once
 //   64 x 96, 4 waves:   22 / 78, 30 / 98, 39 / 128, 50 / 165 for 1 .. 4
+//   64 x 64, 4 waves:   16 / 60, 22 / 72, 30 / 101, 38 / 135 for 1 .. 4
 //   64 x 64 fp32 MFMA:  6 us + 125 TFLOP/s
-// Measured over 8 (N, K) of 512..2304 x 14 row counts from 64 to 16128: the choices take 5.60 ms in all,
-// the fp32 kernels alone 7.13, the best of 13 tiles each time (256 x 128, 256 x 96, 128 x 64, 64 x 64,
-// 128 x 48, 64 x 48 and 128 x 96 in 8 waves too) 5.41.
-enum SplitTile { kMfma64, kSplit64x96, kSplit128x96, kSplit256x144, kSplit256x192 };
-SplitTile split_tile(const LinearParams& p, int num_cus, bool allow_mfma) {
+//   32 x 64 fp32 MFMA, two k splits (its class): 2 us + 6.2 u per tile of a CU, and kept unless 10% slower
+//     (3072 x 576 x 576: 26.8 against 22.3 for 64 x 64, 3072 x 576 x 2304 91 / 72; but 1024 x 1536 x 512 18.3 / 20.4)
+// Measured over 8 (N, K) of 512..2304 x 14 row counts from 64 to 16128: the choices take 5.57 ms in all,
+// the fp32 kernels alone 7.13, the best of 13 tiles each time (256 x 128, 256 x 96, 128 x 64, 128 x 48,
+// 64 x 48 and 128 x 96 in 8 waves too) 5.41.
+enum SplitTile { kMfma64, kKsplit32x64, kSplit64x64, kSplit64x96, kSplit128x96, kSplit256x144, kSplit256x192 };
+SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) {
   const double u = p.K / 576.0;
   auto per_cu = [&](int bm, int bn) {
     const int64_t tiles = (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
@@ -1023,7 +1028,14 @@ SplitTile split_tile(const LinearParams& p, int num_cus, bool allow_mfma) {
   take(n128 / 3 * t128[3] + t128[n128 % 3], kSplit128x96);
   take(per_cu(256, 144) * (6 + 50 * u), kSplit256x144);
   take(per_cu(256, 192) * (10 + 60 * u), kSplit256x192);
-  if (allow_mfma) take(6 + 2e-6 / 125 * p.M * (double)p.N * p.K, kMfma64);
+  const int64_t n64x64 = per_cu(64, 64);
+  const double t64x64[5] = {0, 2 + 14.5 * u, 6 + 16.4 * u, 6.5 + 23.6 * u, 6.5 + 32 * u};
+  take(n64x64 / 4 * t64x64[4] + t64x64[n64x64 % 4], kSplit64x64);
+  if (cls.ksplit == 2) {
+    take(0.9 * (2 + 6.2 * u * per_cu(32, 64)), kKsplit32x64);
+  } else if (cls.wn == 1) {
+    take(6 + 2e-6 / 125 * p.M * (double)p.N * p.K, kMfma64);
+  }
   return t;
 }
 
@@ -1048,8 +1060,9 @@ hipError_t launch_linear(const LinearParams& p, int num_cus, hipStream_t stream)
   }
   const LinearTile t = linear_mfma_tile(p, num_cus);
   if (t.ksplit == 4) return launch_ksplit<1, 1, 4>(p, stream);
-  if (t.ksplit == 2) return launch_ksplit<1, 2, 2>(p, stream);
-  switch (split_tile(p, num_cus, t.wn == 1)) {
+  switch (split_tile(p, num_cus, t)) {
+    case kKsplit32x64: return launch_ksplit<1, 2, 2>(p, stream);
+    case kSplit64x64: return launch_split<4, 1, 4>(p, stream);
     case kSplit64x96: return launch_split<4, 1, 6>(p, stream);
     case kSplit128x96: return launch_split<4, 2, 6>(p, stream);
     case kSplit256x144: return launch_split<8, 2, 9>(p, stream);
