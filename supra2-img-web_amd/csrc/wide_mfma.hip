@@ -1,4 +1,4 @@
-// Attention on fp32 MFMA for wide heads (D = 256 or 512): the SD-VAE mid-block call
+// Attention on the matrix cores for wide heads (D = 256: fp32 MFMA; 512: three-term bf16 products): the SD-VAE mid-block call
 // (app/models/vae.js:86: one head, D = C = 512, 1024 tokens), which the reference sends down its
 // unfused GEMM -> softmax -> GEMM path (app/gpu/ops.js:119-147).
 //
