@@ -500,7 +500,8 @@ hipError_t launch_flash_split(const AttnParams& p, int num_cus, hipStream_t stre
   const int64_t units = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
   const int nblk = (p.Lk + 31) / 32;
   if (p.D == 64) {
-    if (2 * units <= num_cus) return launch_bias<64, 2, 4, 1, 2>(p, stream);
+    // (up to four key blocks two splits, whose merge is a third: 108 units, 40 keys 6.2 us against 7.6)
+    if (2 * units <= num_cus) return nblk <= 4 ? launch_bias<64, 2, 2, 2, 2>(p, stream) : launch_bias<64, 2, 4, 1, 2>(p, stream);
     if (units <= num_cus && nblk > 8) return launch_bias<64, 4, 2, 2, 2>(p, stream);
     return launch_bias<64, 4, 1, 2, 2>(p, stream);
   }

@@ -1001,10 +1001,10 @@ namespace {
 //   128 x 96, 4 waves:  35 / 120, 45 / 152, 56 / 213 for 1, 2, 3 tiles on a CU at once
 //   64 x 96, 4 waves:   22 / 78, 30 / 98, 39 / 128, 50 / 165 for 1 .. 4
 //   64 x 64, 4 waves:   16 / 60, 22 / 72, 30 / 101, 38 / 135 for 1 .. 4
-//   64 x 64 fp32 MFMA:  6 us + 125 TFLOP/s
+//   64 x 64 fp32 MFMA:  4 us + 135 TFLOP/s, its best rate
 //   32 x 64 fp32 MFMA, two k splits (its class): 2 us + 6.2 u per tile of a CU, and kept unless 10% slower
 //     (3072 x 576 x 576: 26.8 against 22.3 for 64 x 64, 3072 x 576 x 2304 91 / 72; but 1024 x 1536 x 512 18.3 / 20.4)
-// Measured over 8 (N, K) of 512..2304 x 14 row counts from 64 to 16128: the choices take 5.57 ms in all,
+// Measured over 8 (N, K) of 512..2304 x 14 row counts from 64 to 16128: the choices take 5.58 ms in all,
 // the fp32 kernels alone 7.13, the best of 13 tiles each time (256 x 128, 256 x 96, 128 x 64, 128 x 48,
 // 64 x 48 and 128 x 96 in 8 waves too) 5.41.
 enum SplitTile { kMfma64, kKsplit32x64, kSplit64x64, kSplit64x96, kSplit128x96, kSplit256x144, kSplit256x192 };
@@ -1034,7 +1034,7 @@ SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) 
   if (cls.ksplit == 2) {
     take(0.9 * (2 + 6.2 * u * per_cu(32, 64)), kKsplit32x64);
   } else if (cls.wn == 1) {
-    take(6 + 2e-6 / 125 * p.M * (double)p.N * p.K, kMfma64);
+    take(4 + 2e-6 / 135 * p.M * (double)p.N * p.K, kMfma64);
   }
   return t;
 }

@@ -23,7 +23,7 @@ MASK = [_lib.SA_MASK_NONE, _lib.SA_MASK_KEY_LEN, _lib.SA_MASK_KEY_MASK]
 
 # 128-query units per CU (256 CUs): under half, at most one with over 8 key blocks, and more, per head dim;
 # query and key counts that end inside a group, a block and a step (1 key past one included)
-SHAPES = [(64, 9, 5, 333, 289), (64, 12, 12, 130, 33), (64, 10, 11, 129, 321), (64, 20, 13, 131, 65),
+SHAPES = [(64, 5, 6, 333, 97), (64, 9, 5, 333, 289), (64, 12, 12, 130, 33), (64, 10, 11, 129, 321), (64, 20, 13, 131, 65),
           (128, 3, 5, 200, 97), (128, 9, 9, 257, 161), (128, 22, 12, 150, 33)]
 
 
