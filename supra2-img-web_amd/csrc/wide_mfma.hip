@@ -439,12 +439,11 @@ __global__ __launch_bounds__(64 * NW, 1) void wide_mfma_kernel(WideArgs p) {
 // maxima and row sums of all waves give one reference m per query for the round. Each wave
 // publishes its probabilities, split once, and accumulates O^T for 64 head dims over all four blocks. Head
 // dim 2i + t of those sits on row i of output tile t, so an 8-byte load of a V row feeds both tiles.
-// K and V rows come from memory into registers, pipelined ahead of their products, and are split there:
-// with 32 queries per workgroup every element is used once, 7 VALU instructions per MFMA, put between
-// the products that cover them. A wave alone issues one of them per 6 cycles, two waves per SIMD one per
-// 4.4, so 8 waves and not 4 (VAE block of 4096 tokens: 331 against 345 us). K is loaded as 64-byte row pieces
-// by 4 lanes each and turned into the operand layout (a row per lane) through wave-private LDS: loaded in that
-// layout, an instruction took the address unit 70 cycles, half of the kernel's time (331 -> 304 us; fp32 products: 401). Q is split once, into LDS; two blocks per wave halve its reads, which at one block
+// K and V rows come straight from memory into registers, pipelined ahead of their products, and are split
+// there: with 32 queries per workgroup every element is used once, 7 VALU instructions per MFMA, put
+// between the products that cover them. That is what bounds it: a wave alone issues one of them per
+// 6 cycles, two waves per SIMD one per 4.4, so 8 waves and not 4 (4096 tokens, the whole call: 331 against 345 us; fp32
+// products: 401). Q is split once, into LDS; two blocks per wave halve its reads, which at one block
 // would take LDS (64 bytes per clock and CU) as long as the MFMAs.
 // Writes the same partial records as wide_mfma_kernel (merged by wide_merge_kernel).
 template <int BIAS, int MASK>
@@ -453,7 +452,7 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
   constexpr int DS = D / 8;          // output head dims per wave
   constexpr int NS = D / 64;         // product steps of a quarter of the head dims
   constexpr int REC = 32 * D + 64;   // workspace floats per partial: O [32][D], m [32], l [32]
-  constexpr int KR = 2;              // product steps whose K loads are in flight
+  constexpr int KR = 3;              // product steps whose K loads are in flight
 
   __shared__ u32x4 lds_q[D / 16 * 3 * 64];  // [product step][term][half][query ^ chunk], then the output
   __shared__ u32x4 lds_p[8 * 3 * 2 * 64];   // probability terms [16 keys][term][lane] (8 * 3 * 64); before that
@@ -493,40 +492,20 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
   const float* kbase = p.k + (int64_t)b * p.sk + h * D;
   const float* vbase = p.v + (int64_t)b * p.sv + h * D + wave * DS;
 
-  // ---- K of product step i (dims 128 (w % 4) + 16 i .. +15) of blocks 2 (w / 4) + 0 and 1, rows 16 y + lane/4,
-  // 16-byte chunk lane % 4: rows past the chunk's last key re-read it
+  // ---- K of product step i (dims 128 (w % 4) + 16 i + 8 half + 0..7) of blocks 2 (w / 4) + 0 and 1: rows
+  // past the chunk's last key re-read it
   f32x4 kring[KR][2][2];
-  const float* kr[2][2];
+  const float* kr[2];
   auto aim_k = [&](int rb0) {
 #pragma unroll
     for (int e = 0; e < 2; ++e)
-#pragma unroll
-      for (int y = 0; y < 2; ++y)
-        kr[e][y] = kbase + (int64_t)min(rb0 + 64 * (wave >> 2) + 32 * e + 16 * y + (lane >> 2), kend - 1) * p.ldk +
-                   128 * (wave & 3) + 4 * (lane & 3);
+      kr[e] = kbase + (int64_t)min(rb0 + 64 * (wave >> 2) + 32 * e + col, kend - 1) * p.ldk + 128 * (wave & 3) + 8 * half;
   };
   auto load_k = [&](int i) {
 #pragma unroll
     for (int e = 0; e < 2; ++e)
 #pragma unroll
-      for (int y = 0; y < 2; ++y) kring[i % KR][e][y] = *reinterpret_cast<const f32x4*>(kr[e][y] + 16 * i);
-  };
-  // through the wave's own part of lds_p (free until its quarter sums): [block][row][chunk ^ row / 4], which
-  // spreads the 16-byte reads of 16 rows over all banks; a wave's LDS accesses run in order, so the rows of
-  // the next step may follow the reads of this one
-  u32x4* const turn = lds_p + wave * 384;
-  const int turn_put = (lane & ~3) + ((lane & 3) ^ ((lane >> 4) & 3));
-  auto put_k = [&](int i) {
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-#pragma unroll
-      for (int y = 0; y < 2; ++y) turn[128 * e + 64 * y + turn_put] = __builtin_bit_cast(u32x4, kring[i % KR][e][y]);
-  };
-  auto get_k = [&](f32x4 (&x)[2][2]) {
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) x[e][c] = __builtin_bit_cast(f32x4, turn[128 * e + 4 * col + ((2 * half + c) ^ ((col >> 2) & 3))]);
+      for (int x = 0; x < 2; ++x) kring[i % KR][e][x] = *reinterpret_cast<const f32x4*>(kr[e] + 16 * i + 4 * x);
   };
   // V rows of one block for this wave's head dims: register r holds V[key][2*col, 2*col + 1] of key
   // 8(r/4) + 4*half + r%4 of the block (the keys of score register r). The buffer ends after the chunk's
@@ -585,26 +564,18 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
       };
       u32x4 qx[2][3];
       Split8 kx[2][2];
-      f32x4 kn[2][2];  // the next step's rows
-      put_k(0);
-      load_k(KR);
-      get_k(kn);
-      put_k(1);
-      load_k(1 + KR);
       read_q(0, qx[0]);
 #pragma unroll
-      for (int e = 0; e < 2; ++e) kx[0][e] = split8(kn[e][0], kn[e][1]);
+      for (int e = 0; e < 2; ++e) kx[0][e] = split8(kring[0][e][0], kring[0][e][1]);
       static_for<NS>([&](auto I) {
         constexpr int i = decltype(I)::value, cur = i & 1;
-        if constexpr (i + 1 < NS) get_k(kn);
-        if constexpr (i + 2 < NS) put_k(i + 2);
-        if constexpr (i + 2 + KR < NS) load_k(i + 2 + KR);
+        if constexpr (i + KR < NS) load_k(i + KR);
         if constexpr (i == NS - 3) load_v(rb0, vbuf[0]);  // the round's first V block streams in under the last products
         if constexpr (i + 1 < NS) {
           read_q(i + 1, qx[cur ^ 1]);
 #pragma unroll
           for (int e = 0; e < 2; ++e)
-            kx[cur ^ 1][e] = split8(kn[e][0], kn[e][1]);
+            kx[cur ^ 1][e] = split8(kring[(i + 1) % KR][e][0], kring[(i + 1) % KR][e][1]);
         }
         auto products = [&](auto kt, int qt) {
 #pragma unroll
