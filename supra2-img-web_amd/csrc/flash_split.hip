@@ -15,7 +15,7 @@
 //   to match. Q is pre-scaled and split once.
 //   LDS: K terms [product step][term][half][key ^ chunk], so that the 8 threads of a row write 8 different
 //   bank groups; V terms [product step][32 dims][term][half][dim], transposed by loading a
-//   row of 64 dims per instruction, 8 keys per thread.
+//   row of 64 dims per instruction, 8 keys per thread. Q, P and V are split as 2^24 times themselves.
 
 #include <string.h>
 
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
       const int u = n * NW + wave;
       const int s = (u / (D / 64)) >> 1 & 1, hh = (u / (D / 64)) & 1;
       const int t32 = 2 * (u % (D / 64)) + half;
-      const Split8 t = split8(f32x4{vx[n][0], vx[n][1], vx[n][2], vx[n][3]}, f32x4{vx[n][4], vx[n][5], vx[n][6], vx[n][7]});
+      const Split8 t = split8(f32x4{vx[n][0], vx[n][1], vx[n][2], vx[n][3]}, f32x4{vx[n][4], vx[n][5], vx[n][6], vx[n][7]}, kUp);
       u32x4* d = base + (u / (D / 16)) * BLK + KBLK + (s * NDB + t32) * 192 + hh * 32 + col;
       d[0] = t.h;
       d[64] = t.m;
@@ -202,15 +202,18 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
   if constexpr (BIAS == BIAS_RELPOS) load_bucket(0);
   if (nstep > 0) load(0);
 
-  // ---- Q terms, pre-scaled: product step s holds dims 16s + 8*half + 0..7 of query qi
+  // ---- Q terms, pre-scaled: product step s holds dims 16s + 8*half + 0..7 of query qi. Times kUp, so the
+  // scores come out in units of kDown. (K needs no scaling: an element below 2^-110 is short of bits by at
+  // most 2^-134, which a scaled query below 2^104 turns into at most 2^-30 of a score; a larger
+  // one overflows here.)
   Split8 q[FK];
   {
-    const float sc = q_valid ? p.scale_log2 : 0.f;
+    const float sc = q_valid ? p.scale_log2 * kUp : 0.f;
 #pragma unroll
     for (int s = 0; s < FK; ++s) {
       const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * s + 8 * half);
       const f32x4 c = *reinterpret_cast<const f32x4*>(qrow + 16 * s + 8 * half + 4);
-      q[s] = split8(a * sc, c * sc);
+      q[s] = split8<true>(a, c, sc);
     }
   }
 
@@ -220,8 +223,10 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
   float m = kMaxSeed;
   float l = 0.f;
 
-  // base-2 scores of the 32 keys from k0 -> probabilities; moves (m, l, O) on
-  auto softmax = [&](float (&u)[16], int k0, bool first) {
+  // Scores of the 32 keys from k0 -> probabilities; moves (m, l, O) on. split: scores of the three-term
+  // products, which are in units of kDown unless a bias has brought them to base 2.
+  auto softmax = [&](float (&u)[16], int k0, bool first, auto split) {
+    constexpr float kUnit = decltype(split)::value && BIAS == BIAS_NONE ? kDown : 1.f;
     if (MASK != MASK_KEY_MASK && k0 + 32 > kv_len) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -232,7 +237,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
     float mb = u[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) mb = max_nan(mb, u[r]);
-    mb = max_with_partner(mb);
+    mb = max_with_partner(mb) * kUnit;
     if (first) {
       m = max_nan(m, mb);
     } else if (__builtin_amdgcn_ballot_w64(mb > m + kRescaleSlack) != 0) {
@@ -243,17 +248,17 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
 #pragma unroll
       for (int t = 0; t < NDB; ++t) oacc[t] *= alpha;
     }
-    u[0] = fast_exp2(u[0] - m);
+    u[0] = fast_exp2(fmaf(u[0], kUnit, -m));
     float ps = u[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) {
-      u[r] = fast_exp2(u[r] - m);
+      u[r] = fast_exp2(fmaf(u[r], kUnit, -m));
       ps += u[r];
     }
     l += ps;
   };
 
-  // scores of block blk from stage `stage`, bias and key mask added
+  // scores of block blk from stage `stage` (in units of kDown, base 2 with a bias), bias and key mask added
   auto scores = [&](int stage, float (&u)[16]) {
     const u32x4* kb = lds + stage * STAGE + ks * BLK;
     f32x16 s = zero16();
@@ -270,7 +275,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      u[r] = s[r];
+      u[r] = BIAS == BIAS_NONE ? s[r] : s[r] * kDown;
       const int e = 8 * (r >> 2) + 4 * half + (r & 3);  // the register's key in the block
       if constexpr (BIAS == BIAS_DENSE) u[r] += bcur[r];
       if constexpr (BIAS == BIAS_RELPOS) u[r] += lds_rb[stage * RB + 32 * ks + e - qi + q0 + QT - 1];
@@ -282,7 +287,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const Split8 pt = split8(f32x4{pr[8 * i], pr[8 * i + 1], pr[8 * i + 2], pr[8 * i + 3]},
-                               f32x4{pr[8 * i + 4], pr[8 * i + 5], pr[8 * i + 6], pr[8 * i + 7]});
+                               f32x4{pr[8 * i + 4], pr[8 * i + 5], pr[8 * i + 6], pr[8 * i + 7]}, kUp);
 #pragma unroll
       for (int t0 = 0; t0 < NDB; t0 += 2) {
         u32x4 v[2][3];
@@ -315,7 +320,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
     if (blk < nblk) {
       float u[16];
       scores(stage, u);
-      softmax(u, blk * 32, step == 0);
+      softmax(u, blk * 32, step == 0, std::true_type{});
       output(stage, u);
     }
     if constexpr (STAGES == 1) __syncthreads();  // every wave is done with the stage
@@ -326,9 +331,10 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
     __syncthreads();
   }
 
-  // Values without three terms (infinity, NaN, past the bfloat16 range) turn into NaN: a wave that finds
-  // anything not finite in its state takes its key blocks again with fp32 products straight from memory,
-  // so such inputs give what float32 products give.
+  // Values without three terms (infinity, NaN, scaled queries and values from 2^104 up) turn into NaN, and
+  // sums past the scaled range into infinities: a wave that finds anything not finite in its state takes its
+  // key blocks again with fp32 products straight from memory, so such inputs give what float32 products
+  // give.
   {
     float z = l * 0.f;
 #pragma unroll
@@ -359,7 +365,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
           }
           if constexpr (MASK == MASK_KEY_MASK) pr[r] += key < p.Lk && kmask[kc] != 0 ? 0.f : -INFINITY;
         }
-        softmax(pr, blk * 32, blk == ks);
+        softmax(pr, blk * 32, blk == ks, std::false_type{});
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float* vrow = vbase + (int64_t)min(blk * 32 + 8 * (r >> 2) + 4 * half + (r & 3), kv_len - 1) * p.ldv + col;
@@ -367,6 +373,9 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
           for (int t = 0; t < NDB; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * t], pr[r], oacc[t], 0, 0, 0);
         }
       }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NDB; ++t) oacc[t] *= kDown * kDown;  // of P and V
     }
   }
 

@@ -166,7 +166,8 @@ __device__ __forceinline__ void redo_tile(const LinArgs& p, int m0, int n0, int 
 
 // Large and medium grids: the product on the bf16 matrix cores, each float32 operand as three bfloat16
 // terms (split.h) and each product as the six term products of 2^-24 and more of its size, smallest
-// first, summed in the float32 accumulators: x w ~ xl wh + xh wl + xm wm + xm wh + xh wm + xh wh.
+// first, summed in the float32 accumulators: x w ~ xl wh + xh wl + xm wm + xm wh + xh wm + xh wh. Both
+// operands are scaled by 2^24 before the split (kUp), the sums by 2^-48 after it.
 // Error against 64 bits (2-norm, N(0, 1) rows, K = 576 / 2304): 3.4e-7 / 7.2e-7, the fp32 MFMA chain
 // 4.3e-7 / 8.6e-7: one rounding per 32 k and term product instead of one per 2 k, and the terms
 // dropped are below the rounding of the sum.
@@ -188,7 +189,7 @@ __device__ __forceinline__ void redo_tile(const LinArgs& p, int m0, int n0, int 
 template <int NW, int MT, int NT, int ACT, int EPI>
 __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void linear_split_kernel(LinArgs p, TileOrder order) {
   constexpr int BM = 16 * MT * NW, BN = 16 * NT, BK = 32;
-  constexpr int GW = NT % 3 == 0 ? 3 : 2;   // column fragments per group: MT * GW independent chains
+  constexpr int GW = NT % 3 == 0 && MT * NT != 12 ? 3 : 2;  // column fragments per group: MT * GW independent chains (128 x 96 in threes spills)
   constexpr int G = NT / GW;
   constexpr int NF = (NT + NW - 1) / NW;    // W fragments per wave (the last waves may have one less)
   constexpr int STAGE = NT * 3 * 64;        // 16-byte chunks per stage: [fragment][term][lane]
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
   };
   auto put = [&](int f, int stage) {
     if (f * NW + wave < NT) {
-      const Split8 s = split8(wb[f][0], wb[f][1]);
+      const Split8 s = split8(wb[f][0], wb[f][1], kUp);
       u32x4* d = lds + stage * STAGE + (f * NW + wave) * 192 + lane;
       d[0] = s.h;
       d[64] = s.m;
@@ -291,7 +292,7 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
           if (f % G == g) put(f, C ^ 1);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-          if ((i + NF) % G == g) a[C ^ 1][i] = split8(xa[i][0], xa[i][1]);
+          if ((i + NF) % G == g) a[C ^ 1][i] = split8(xa[i][0], xa[i][1], kUp);
       }
     });
     if (kt + 2 < nkt) load(kt + 2);
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
 #pragma unroll
   for (int f = 0; f < NF; ++f) put(f, 0);
 #pragma unroll
-  for (int i = 0; i < MT; ++i) a[0][i] = split8(xa[i][0], xa[i][1]);
+  for (int i = 0; i < MT; ++i) a[0][i] = split8(xa[i][0], xa[i][1], kUp);
   if (nkt > 1) load(1);
   __syncthreads();
   int kt = 0;
@@ -312,8 +313,8 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
   }
   if (kt < nkt) step(kt, std::integral_constant<int, 0>{});
 
-  // An infinity, a NaN or a magnitude that rounds past the bfloat16 range has no three terms: the
-  // differences turn into NaN. A wave that finds anything not finite in its sums takes its whole tile
+  // An infinity, a NaN or a magnitude from 2^104 up has no three terms (the differences turn into NaN), and
+  // a product from 2^80 up leaves the range of the scaled sums. A wave that finds anything not finite in its sums takes its whole tile
   // again with fp32 MFMAs straight from memory, so such inputs give what float32 products give.
   float z = 0.f;
 #pragma unroll
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
       if constexpr (EPI == LIN_EPI_RESID_GATE) g = load4(p.gate + n, gate_vec, left);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] = apply_act<ACT>(fmaf(acc[i][j][e], p.alpha, v[e]));
+        v[e] = apply_act<ACT>(fmaf(acc[i][j][e] * (kDown * kDown), p.alpha, v[e]));
         if constexpr (EPI != LIN_EPI_STORE) v[e] = fmaf(g[e], v[e], old[j][e]);
       }
       float* dst = p.y + row + n;

@@ -10,7 +10,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // x = h + m + l with h, m, l the bfloat16 roundings of x, x - h and x - h - m (both differences exact):
-// the three terms hold all 24 bits of x. 11 VALU instructions per pair of values.
+// the three terms hold all 24 bits of x from 2^-110 up; below that l, and then m, run out of exponent
+// (20 bits at 2^-114, 8 at 2^-126). Operands that may be that small are split as kUp x: a multiple of
+// 2^-125 for every float32, so no term is ever subnormal, and the products are scaled back afterwards. From
+// 2^104 up kUp x is infinite, which the callers' checks of their sums send to the fp32 products.
+// 11 VALU instructions per pair of values, 13 with the scaling.
+constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;
+
 struct Split8 {
   u32x4 h, m, l;  // 8 bfloat16 each, in order
 };
@@ -19,25 +25,32 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
 }
 
-__device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = cvt_pk_bf16(a, b);
-  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+// The terms of scale * a and scale * b. EXACT: of the products before their rounding to float32 (for a scale that
+// is no power of two); otherwise the products are rounded first, which an fma would not make more
+// exact, but at twice the issue time of the subtraction.
+template <bool EXACT>
+__device__ __forceinline__ void split_pair(float a, float b, float scale, uint32_t& h, uint32_t& m, uint32_t& l) {
+#pragma clang fp contract(off)
+  const float xa = a * scale, xb = b * scale;
+  h = cvt_pk_bf16(xa, xb);
+  const float ha = __uint_as_float(h << 16), hb = __uint_as_float(h & 0xffff0000u);
+  const float ra = EXACT ? fmaf(a, scale, -ha) : xa - ha, rb = EXACT ? fmaf(b, scale, -hb) : xb - hb;
   m = cvt_pk_bf16(ra, rb);
   const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
   l = cvt_pk_bf16(sa, sb);
 }
 
-__device__ __forceinline__ Split8 split8(f32x4 a, f32x4 b) {
+template <bool EXACT = false>
+__device__ __forceinline__ Split8 split8(f32x4 a, f32x4 b, float scale = 1.f) {
   Split8 s;
-  uint32_t h, m, l;
-  split_pair(a[0], a[1], h, m, l);
-  s.h[0] = h, s.m[0] = m, s.l[0] = l;
-  split_pair(a[2], a[3], h, m, l);
-  s.h[1] = h, s.m[1] = m, s.l[1] = l;
-  split_pair(b[0], b[1], h, m, l);
-  s.h[2] = h, s.m[2] = m, s.l[2] = l;
-  split_pair(b[2], b[3], h, m, l);
-  s.h[3] = h, s.m[3] = m, s.l[3] = l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4& v = i < 2 ? a : b;
+    const int e = 2 * (i & 1);
+    uint32_t h, m, l;
+    split_pair<EXACT>(v[e], v[e + 1], scale, h, m, l);
+    s.h[i] = h, s.m[i] = m, s.l[i] = l;
+  }
   return s;
 }
 

@@ -528,14 +528,16 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
 #pragma unroll
     for (int i = 0; i < KR; ++i) load_k(i);
   }
-  // ---- Q terms into LDS, pre-scaled (rows past Lq re-read the last row)
+  // ---- Q terms into LDS, pre-scaled, and times kUp, so the scores come out in units of kDown (rows past Lq
+  // re-read the last row). K needs no scaling: an element below 2^-110 is short of bits by at most 2^-134,
+  // which a scaled query below 2^104 turns into at most 2^-30 of a score; a larger one overflows here.
   if (tid == 0) lds_bad = 0;
+  const float sc = p.scale_log2 * kUp;
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const int row = (n * 512 + tid) >> 6, c = lane;
     const float* src = qbase + (int64_t)min(q0 + row, p.Lq - 1) * p.ldq + 8 * c;
-    const Split8 t = split8(*reinterpret_cast<const f32x4*>(src) * p.scale_log2,
-                            *reinterpret_cast<const f32x4*>(src + 4) * p.scale_log2);
+    const Split8 t = split8<true>(*reinterpret_cast<const f32x4*>(src), *reinterpret_cast<const f32x4*>(src + 4), sc);
     u32x4* d = lds_q + (c >> 1) * 192 + (c & 1) * 32 + (row ^ (c & 31));
     d[0] = t.h;
     d[64] = t.m;
@@ -628,6 +630,8 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
         for (int c = 0; c < 4; ++c) u[4 * e + c] += v[c];
       }
     }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) u[r] *= kDown;
     if constexpr (kTerms) {  // of the block's 16 registers per lane, this wave's 8
       float w[16];
 #pragma unroll
@@ -674,7 +678,7 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
     ps = sum_with_partner(ps);
     if (half == 0) lds_l[wave * 32 + col] = ps;
     {
-      const Split8 t = split8(f32x4{u[0], u[1], u[2], u[3]}, f32x4{u[4], u[5], u[6], u[7]});
+      const Split8 t = split8(f32x4{u[0], u[1], u[2], u[3]}, f32x4{u[4], u[5], u[6], u[7]}, kUp);
       u32x4* d = lds_p + (blk * 2 + sub) * 192 + lane;
       d[0] = t.h;
       d[64] = t.m;
@@ -701,7 +705,7 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
           const f32x2* vb = vbuf[j & 1] + 8 * i;
 #pragma unroll
           for (int t = 0; t < 2; ++t)
-            vx[i][t] = split8(f32x4{vb[0][t], vb[1][t], vb[2][t], vb[3][t]}, f32x4{vb[4][t], vb[5][t], vb[6][t], vb[7][t]});
+            vx[i][t] = split8(f32x4{vb[0][t], vb[1][t], vb[2][t], vb[3][t]}, f32x4{vb[4][t], vb[5][t], vb[6][t], vb[7][t]}, kUp);
 #pragma unroll
           for (int t = 0; t < 3; ++t) px[i][t] = lds_p[(j * 2 + i) * 192 + 64 * t + lane];
         };
@@ -727,8 +731,9 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
     if (rd + 1 < rounds) __syncthreads();  // every wave is done with the round's exchange
   }
 
-  // Values without three terms (infinity, NaN, past the bfloat16 range) turn into NaN: if any wave finds
-  // anything not finite in its state, all take the chunk again with fp32 products straight from memory.
+  // Values without three terms (infinity, NaN, scaled queries and values from 2^104 up) turn into NaN, and
+  // sums past the scaled range into infinities: if any wave finds anything not finite in its state, all take the
+  // chunk again with fp32 products straight from memory.
   {
     float z = l * 0.f;
 #pragma unroll
@@ -781,6 +786,9 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
 #pragma unroll
           for (int t = 0; t < 2; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[r][t], u[r], oacc[t], 0, 0, 0);
       }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) oacc[t] *= kDown * kDown;  // of P and V
     }
   }
 

@@ -71,3 +71,24 @@ def test_values_without_three_terms(dev, D, B, H, Lq, Lk):
     np.testing.assert_array_equal(np.isposinf(got), np.isposinf(ref))
     fin = np.isfinite(ref)
     assert np.abs(got[fin] - ref[fin]).max() <= 1e-5 * np.abs(ref[fin]).max()
+
+
+@pytest.mark.parametrize("what", ["v", "k", "q"])
+@pytest.mark.parametrize("D,B,H,Lq,Lk", [(64, 9, 5, 333, 289), (64, 20, 13, 131, 65), (128, 9, 9, 257, 161), (512, 2, 1, 200, 333)])
+def test_tiny_operands(dev, D, B, H, Lq, Lk, what):
+    """Operands around 2^-120 have no third bfloat16 term of their own (14 of 24 bits would remain, 3e-5 in the
+    2-norm): they are as exact as any others. Tiny keys meet queries of 2^100, and the other way about."""
+    call = make_call(B, H, D, Lq, Lk, seed=7)
+    other = {"k": "q", "q": "k"}.get(what)
+    setattr(call, what, getattr(call, what) * np.float32(2.0 ** -120))
+    if other:
+        setattr(call, other, getattr(call, other) * np.float32(2.0 ** 100))
+        call.scale *= 2.0 ** 20
+    print(f"[tiny {what}] {call.name}", flush=True)
+    st = Staged(dev, call)
+    try:
+        got = orc.output_view(st.run(), call)
+    finally:
+        st.release()
+    e = orc.errors(got, orc.reference_fp64(call))
+    assert e["finite"] and e["rel_l2"] <= 2e-6 and e["max_rel"] <= 1e-5, e
