@@ -189,7 +189,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
     }
     if constexpr (BIAS == BIAS_DENSE) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bcur[r] = bx[r] * kLog2e;
+      for (int r = 0; r < 16; ++r) bcur[r] = bx[r];
     }
     if constexpr (BIAS == BIAS_RELPOS) {
       if (tid < RB) lds_rb[stage * RB + tid] = rbx * kLog2e;
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
     for (int r = 0; r < 16; ++r) {
       u[r] = BIAS == BIAS_NONE ? s[r] : s[r] * kDown;
       const int e = 8 * (r >> 2) + 4 * half + (r & 3);  // the register's key in the block
-      if constexpr (BIAS == BIAS_DENSE) u[r] += bcur[r];
+      if constexpr (BIAS == BIAS_DENSE) u[r] = fmaf(bcur[r], kLog2e, u[r]);
       if constexpr (BIAS == BIAS_RELPOS) u[r] += lds_rb[stage * RB + 32 * ks + e - qi + q0 + QT - 1];
       if constexpr (MASK == MASK_KEY_MASK) u[r] += lds_km[stage * KT + 32 * ks + e];
     }

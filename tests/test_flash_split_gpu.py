@@ -92,3 +92,22 @@ def test_tiny_operands(dev, D, B, H, Lq, Lk, what):
         st.release()
     e = orc.errors(got, orc.reference_fp64(call))
     assert e["finite"] and e["rel_l2"] <= 2e-6 and e["max_rel"] <= 1e-5, e
+
+
+@pytest.mark.parametrize("D,B,H,Lq,Lk", [(64, 9, 5, 333, 289), (128, 9, 9, 257, 161)])
+def test_large_dense_bias_is_rounded_once(dev, D, B, H, Lq, Lk):
+    """score + log2(e) bias as one fma: with biases ~ N(0, 200^2) that rounding is the error of the call. A sum
+    of a rounded product has sqrt(2) times as much; 1.15 lies between."""
+    call = make_call(B, H, D, Lq, Lk, seed=11, bias_mode=_lib.SA_BIAS_DENSE, bias_std=200.0)
+    got = run(dev, call)
+    ref = orc.reference_fp64(call)
+    log2e = np.float64(np.float32(1.4426950408889634))
+    q, k, v = (x.reshape(B, L, H, D).transpose(0, 2, 1, 3).astype(np.float64) for x, L in ((call.q, Lq), (call.k, Lk), (call.v, Lk)))
+    s = q @ k.transpose(0, 1, 3, 2) * np.float64(np.float32(call.scale)) * log2e
+    u = (s + call.bias.reshape(1, H, Lq, Lk) * log2e).astype(np.float32).astype(np.float64)
+    p = np.exp2(u - u.max(axis=-1, keepdims=True))
+    once = (p @ v) / p.sum(axis=-1, keepdims=True)
+    once = once.transpose(0, 2, 1, 3)  # [B, Lq, H, D], as the others
+    err, one = np.linalg.norm(got - ref), np.linalg.norm(once - ref)
+    print(f"{err / np.linalg.norm(ref):.3e} against {one / np.linalg.norm(ref):.3e}", flush=True)
+    assert err <= 1.15 * one
