@@ -36,8 +36,6 @@ struct FlashOrder {
 };
 struct NoOrder {};
 
-typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 z;
 #pragma unroll

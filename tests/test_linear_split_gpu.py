@@ -13,6 +13,7 @@ import pytest
 
 from oracle import linear as ol
 from supra_attn import _lib
+from supra_attn.device import Event
 from supra_attn.linear_workloads import make_linear
 from supra_attn.runner import StagedLinear
 
@@ -82,3 +83,36 @@ def test_tiny_operands(dev, M, N, K, what):
     got = run(dev, call)
     e = ol.errors(got, ol.linear_fp64(call.x, call.w, call.y0, **call.oracle_kwargs()))
     assert e["finite"] and e["rel_l2"] <= TOL and e["max_rel"] <= 1e-5, e
+
+
+@pytest.mark.parametrize("y_off,ldy", [(0, 1108), (1, 1108), (0, 1107), (3, 1109)])
+def test_store_at_any_alignment(dev, y_off, ldy):
+    """Plain stores into rows at every 4-byte alignment; nothing beside the rows is written."""
+    call = make_linear(f"store_{y_off}_{ldy}", 2047, 1107, 584, seed=ldy + y_off, y_off=y_off, ldy=ldy)
+    got = run(dev, call)
+    e = ol.errors(got, ol.linear_fp64(call.x, call.w, call.y0, **call.oracle_kwargs()))  # with the gaps of y0
+    assert e["finite"] and e["rel_l2"] <= TOL and e["max_rel"] <= 1e-5, e
+
+
+def test_unaligned_rows_cost_little(dev):
+    """Rows of y off a 16-byte boundary take at most twice as long as aligned ones (measured about the same; element by
+    element and past the L2 they took 4 times)."""
+    def best(y_off, ldy):
+        st = StagedLinear(dev, make_linear("rows", 5714, 1107, 56, y_off=y_off, ldy=ldy))
+        a, b = Event(), Event()
+        try:
+            times = []
+            for _ in range(6):
+                a.record(dev.stream)
+                for _ in range(50):
+                    st.launch()
+                b.record(dev.stream)
+                dev.sync()
+                times.append(a.elapsed_ms(b))
+            return min(times)
+        finally:
+            st.release()
+
+    aligned, unaligned = best(0, 1120), best(1, 1107)
+    print(f"[linear split] aligned {aligned:.4f} ms, unaligned {unaligned:.4f} ms", flush=True)
+    assert unaligned <= 2 * aligned
