@@ -30,6 +30,7 @@ __device__ __forceinline__ int xcd_remap(int bid, int n) {
 // IEEE 754-2019 maximum (a NaN operand gives NaN): one v_maximum3_f32 per two new operands on gfx950,
 // where fmaxf also canonicalizes its operands. A NaN score ends in a NaN output either way.
 __device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float min_nan(float a, float b) { return __builtin_elementwise_minimum(a, b); }
 
 // Exchange with the lane 32 away (v_permlane32_swap): returns {own, partner} in some order, so
 // symmetric reductions (max, +) can combine the two results directly.

@@ -15,7 +15,7 @@
 //   to match. Q is pre-scaled and split once.
 //   LDS: K terms [product step][term][half][key ^ chunk], so that the 8 threads of a row write 8 different
 //   bank groups; V terms [product step][32 dims][term][half][dim], transposed by loading a
-//   row of 64 dims per instruction, 8 keys per thread. Q, P and V are split as 2^24 times themselves.
+//   row of 64 dims per instruction, 8 keys per thread. Q and P are split as 2^24 times themselves.
 
 #include <string.h>
 
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
       const int u = n * NW + wave;
       const int s = (u / (D / 64)) >> 1 & 1, hh = (u / (D / 64)) & 1;
       const int t32 = 2 * (u % (D / 64)) + half;
-      const Split8 t = split8(f32x4{vx[n][0], vx[n][1], vx[n][2], vx[n][3]}, f32x4{vx[n][4], vx[n][5], vx[n][6], vx[n][7]}, kUp);
+      const Split8 t = split8(f32x4{vx[n][0], vx[n][1], vx[n][2], vx[n][3]}, f32x4{vx[n][4], vx[n][5], vx[n][6], vx[n][7]});
       u32x4* d = base + (u / (D / 16)) * BLK + KBLK + (s * NDB + t32) * 192 + hh * 32 + col;
       d[0] = t.h;
       d[64] = t.m;
@@ -329,17 +329,30 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
     __syncthreads();
   }
 
-  // Values without three terms (infinity, NaN, scaled queries and values from 2^104 up) turn into NaN, and
-  // sums past the scaled range into infinities: a wave that finds anything not finite in its state takes its
-  // key blocks again with fp32 products straight from memory, so such inputs give what float32 products
-  // give.
+  // Two kinds of values have no three terms, and a wave whose sums they may have reached takes its key blocks
+  // again with fp32 products straight from memory, so such inputs give what float32 products give:
+  // infinity, NaN, keys and values past the bfloat16 range and scaled queries from 2^104 up, which turn into NaN,
+  // and sums past the scaled range, which turn into infinities: anything not finite in its state;
+  // elements of V below 2^-110, whose terms are short by up to 2^-134, which costs an output at most 2^-134 l: one
+  // that is not zero and below 2^26 times that.
   {
-    float z = l * 0.f;
+    float most = fabsf(l), least = INFINITY;
+    const float floor = sum_with_partner(l) * (0x1p-108f * kUp);
 #pragma unroll
     for (int t = 0; t < NDB; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) z = fmaf(oacc[t][r], 0.f, z);
-    if (__builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0) {
+      for (int r = 0; r < 16; ++r) {
+        most = max_nan(most, fabsf(oacc[t][r]));
+        least = min_nan(least, fabsf(oacc[t][r]));
+      }
+    bool redo = !(most < INFINITY);
+    if (least < floor) {  // zeros too, which are exact: look again
+#pragma unroll
+      for (int t = 0; t < NDB; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) redo |= oacc[t][r] != 0.f && fabsf(oacc[t][r]) < floor;
+    }
+    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
 #pragma unroll
       for (int t = 0; t < NDB; ++t) oacc[t] = zero16();
       m = kMaxSeed;
@@ -373,7 +386,7 @@ __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArg
       }
     } else {
 #pragma unroll
-      for (int t = 0; t < NDB; ++t) oacc[t] *= kDown * kDown;  // of P and V
+      for (int t = 0; t < NDB; ++t) oacc[t] *= kDown;  // P was scaled
     }
   }
 

@@ -166,9 +166,8 @@ __device__ __forceinline__ void redo_tile(const LinArgs& p, int m0, int n0, int 
 
 // Large and medium grids: the product on the bf16 matrix cores, each float32 operand as three bfloat16
 // terms (split.h) and each product as the six term products of 2^-24 and more of its size, smallest
-// first, summed in the float32 accumulators: x w ~ xl wh + xh wl + xm wm + xm wh + xh wm + xh wh. Both
-// operands are scaled by 2^24 before the split (kUp), the sums by 2^-48 after it.
-// Error against 64 bits (2-norm, N(0, 1) rows, K = 576 / 2304): 3.4e-7 / 7.2e-7, the fp32 MFMA chain
+// first, summed in the float32 accumulators: x w ~ xl wh + xh wl + xm wm + xm wh + xh wm + xh wh.
+// Error against 64 bits (2-norm, N(0, 1) rows, K = 576 / 2304): 3.6e-7 / 7.4e-7, the fp32 MFMA chain
 // 4.3e-7 / 8.6e-7: one rounding per 32 k and term product instead of one per 2 k, and the terms
 // dropped are below the rounding of the sum.
 //
@@ -189,13 +188,14 @@ __device__ __forceinline__ void redo_tile(const LinArgs& p, int m0, int n0, int 
 template <int NW, int MT, int NT, int ACT, int EPI>
 __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void linear_split_kernel(LinArgs p, TileOrder order) {
   constexpr int BM = 16 * MT * NW, BN = 16 * NT, BK = 32;
-  constexpr int GW = NT % 3 == 0 && MT * NT != 12 ? 3 : 2;  // column fragments per group: MT * GW independent chains (128 x 96 in threes spills)
+  constexpr int GW = NT % 3 == 0 ? 3 : 2;   // column fragments per group: MT * GW independent chains
   constexpr int G = NT / GW;
   constexpr int NF = (NT + NW - 1) / NW;    // W fragments per wave (the last waves may have one less)
   constexpr int STAGE = NT * 3 * 64;        // 16-byte chunks per stage: [fragment][term][lane]
   static_assert(G * GW == NT, "column fragments must split into groups");
 
   __shared__ u32x4 lds[2 * STAGE];
+  __shared__ unsigned lds_norm;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -246,13 +246,15 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
       for (int i = 0; i < MT; ++i) xa[i][0] = xa[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
   };
+  f32x4 norm = {0.f, 0.f, 0.f, 0.f};  // on its diagonal, sums of squares over the rows of x and W that the wave splits
   auto put = [&](int f, int stage) {
     if (f * NW + wave < NT) {
-      const Split8 s = split8(wb[f][0], wb[f][1], kUp);
+      const Split8 s = split8(wb[f][0], wb[f][1]);
       u32x4* d = lds + stage * STAGE + (f * NW + wave) * 192 + lane;
       d[0] = s.h;
       d[64] = s.m;
       d[128] = s.l;
+      norm = mfma16(s.h, s.h, norm);
     }
   };
   Split8 a[2][MT];
@@ -267,6 +269,8 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
     constexpr int C = decltype(stage)::value;
     const bool more = kt + 1 < nkt;
     if (more) cut(kt + 1);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) norm = mfma16(a[C][i].h, a[C][i].h, norm);
     static_for<G>([&](auto gg) {
       constexpr int g = decltype(gg)::value;
       u32x4 b[GW][3];
@@ -292,18 +296,19 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
           if (f % G == g) put(f, C ^ 1);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-          if ((i + NF) % G == g) a[C ^ 1][i] = split8(xa[i][0], xa[i][1], kUp);
+          if ((i + NF) % G == g) a[C ^ 1][i] = split8(xa[i][0], xa[i][1]);
       }
     });
     if (kt + 2 < nkt) load(kt + 2);
     __syncthreads();
   };
+  if (tid == 0) lds_norm = 0;
   load(0);
   cut(0);
 #pragma unroll
   for (int f = 0; f < NF; ++f) put(f, 0);
 #pragma unroll
-  for (int i = 0; i < MT; ++i) a[0][i] = split8(xa[i][0], xa[i][1], kUp);
+  for (int i = 0; i < MT; ++i) a[0][i] = split8(xa[i][0], xa[i][1]);
   if (nkt > 1) load(1);
   __syncthreads();
   int kt = 0;
@@ -313,17 +318,38 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
   }
   if (kt < nkt) step(kt, std::integral_constant<int, 0>{});
 
-  // An infinity, a NaN or a magnitude from 2^104 up has no three terms (the differences turn into NaN), and
-  // a product from 2^80 up leaves the range of the scaled sums. A wave that finds anything not finite in its sums takes its whole tile
-  // again with fp32 MFMAs straight from memory, so such inputs give what float32 products give.
-  float z = 0.f;
+  // Two kinds of operands have no three terms, and a wave whose sums they may have reached takes its whole tile
+  // again with fp32 MFMAs straight from memory, so such inputs give what float32 products give:
+  // infinity, NaN and magnitudes that round past the bfloat16 range, whose differences turn into NaN: anything
+  // not finite in the sums;
+  // magnitudes below 2^-110, whose terms are short by up to 2^-134. That costs a sum at most 2^-134 (|x|_1 + |w|_1)
+  // <= 2^-133 sqrt(K) n, with n^2 the largest sum of squares over a row of x or W: a sum below 2^26 times that
+  // (zeros, which are mostly those of zero rows, only where it may be more than 2^-106 off). The squares come from the matrix cores, which have the time: one product of each
+  // fragment's first terms with themselves per 32 k. (Scaling every operand by 2^24 instead, at 2 VALU
+  // instructions per pair, took 10 to 20% longer: 16384 x 576 x 576 62.7 us against 56.6.)
+  if (lr >> 2 == lc) atomicMax(&lds_norm, __float_as_uint(norm[lr & 3]));
+  float most = 0.f, least = INFINITY;
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) z = fmaf(acc[i][j][e], 0.f, z);
-  if (__builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0) {
+      for (int e = 0; e < 4; ++e) {
+        most = max_nan(most, fabsf(acc[i][j][e]));
+        least = min_nan(least, fabsf(acc[i][j][e]));
+      }
+  __syncthreads();
+  const float floor = 0x1p-107f * sqrtf(static_cast<float>(p.K)) * sqrtf(__uint_as_float(lds_norm));
+  bool redo = !(most < INFINITY);
+  if (!(least >= floor)) {  // look again: zeros are exact, or off by no more than 2^-106
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) redo |= !(fabsf(acc[i][j][e]) >= floor) && (acc[i][j][e] != 0.f || floor > 0x1p-80f);
+  }
+  if (__builtin_amdgcn_ballot_w64(redo) != 0) {
     redo_tile<ACT, EPI>(p, mw, n0, 16 * MT, BN, lr, lc);
     return;
   }
@@ -365,7 +391,7 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
       if constexpr (EPI == LIN_EPI_RESID_GATE) g = load4(p.gate + n, left);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] = apply_act<ACT>(fmaf(acc[i][j][e] * (kDown * kDown), p.alpha, v[e]));
+        v[e] = apply_act<ACT>(fmaf(acc[i][j][e], p.alpha, v[e]));
         if constexpr (EPI != LIN_EPI_STORE) v[e] = fmaf(g[e], v[e], old[j][e]);
       }
       float* dst = p.y + row + n;

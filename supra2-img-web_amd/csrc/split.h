@@ -10,10 +10,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // x = h + m + l with h, m, l the bfloat16 roundings of x, x - h and x - h - m (both differences exact):
-// the three terms hold all 24 bits of x from 2^-110 up; below that l, and then m, run out of exponent
-// (20 bits at 2^-114, 8 at 2^-126). Operands that may be that small are split as kUp x: a multiple of
-// 2^-125 for every float32, so no term is ever subnormal, and the products are scaled back afterwards. From
-// 2^104 up kUp x is infinite, which the callers' checks of their sums send to the fp32 products.
+// the three terms hold all 24 bits of x from 2^-110 up. Below that l, and then m, run out of exponent: they are
+// short by up to 2^-134 (20 bits are left at 2^-114, 8 at 2^-126, none below 2^-134). So the kernels either split kUp
+// x, a multiple of 2^-125 for every float32 (from 2^104 up it is infinite, which their checks of the sums
+// see), or compare their sums with what such operands may have cost them, and fall back to fp32 products.
 // 11 VALU instructions per pair of values, 13 with the scaling.
 constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;
 

@@ -705,7 +705,7 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
           const f32x2* vb = vbuf[j & 1] + 8 * i;
 #pragma unroll
           for (int t = 0; t < 2; ++t)
-            vx[i][t] = split8(f32x4{vb[0][t], vb[1][t], vb[2][t], vb[3][t]}, f32x4{vb[4][t], vb[5][t], vb[6][t], vb[7][t]}, kUp);
+            vx[i][t] = split8(f32x4{vb[0][t], vb[1][t], vb[2][t], vb[3][t]}, f32x4{vb[4][t], vb[5][t], vb[6][t], vb[7][t]});
 #pragma unroll
           for (int t = 0; t < 3; ++t) px[i][t] = lds_p[(j * 2 + i) * 192 + 64 * t + lane];
         };
@@ -731,16 +731,27 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
     if (rd + 1 < rounds) __syncthreads();  // every wave is done with the round's exchange
   }
 
-  // Values without three terms (infinity, NaN, scaled queries and values from 2^104 up) turn into NaN, and
-  // sums past the scaled range into infinities: if any wave finds anything not finite in its state, all take the
-  // chunk again with fp32 products straight from memory.
+  // Values without three terms, as in flash_split_kernel: anything not finite in a wave's state, or an output that
+  // is not zero and below 2^26 times what V elements below 2^-110 may have cost it. If any wave finds one,
+  // all take the chunk again with fp32 products straight from memory.
   {
-    float z = l * 0.f;
+    float most = fabsf(l), least = INFINITY;
+    const float floor = l * (0x1p-108f * kUp);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) z = fmaf(oacc[t][r], 0.f, z);
-    if (__builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0 && lane == 0) lds_bad = 1;
+      for (int r = 0; r < 16; ++r) {
+        most = max_nan(most, fabsf(oacc[t][r]));
+        least = min_nan(least, fabsf(oacc[t][r]));
+      }
+    bool redo = !(most < INFINITY);
+    if (least < floor) {  // zeros too, which are exact: look again
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) redo |= oacc[t][r] != 0.f && fabsf(oacc[t][r]) < floor;
+    }
+    if (__builtin_amdgcn_ballot_w64(redo) != 0 && lane == 0) lds_bad = 1;
     __syncthreads();  // also: every wave is done with the Q terms
     if (lds_bad != 0) {
 #pragma unroll
@@ -788,7 +799,7 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
       }
     } else {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) oacc[t] *= kDown * kDown;  // of P and V
+      for (int t = 0; t < 2; ++t) oacc[t] *= kDown;  // P was scaled
     }
   }
 

@@ -73,13 +73,16 @@ def test_values_without_three_terms(dev, M, N, K):
     assert np.all(np.abs(got[fin] - ref[fin]) <= 1e-5 * rows[fin])
 
 
+@pytest.mark.parametrize("up,over", [(120, 0), (138, 60)])
 @pytest.mark.parametrize("what", ["x", "w"])
 @pytest.mark.parametrize("M,N,K", [(2047, 2050, 776), (16300, 570, 40)])
-def test_tiny_operands(dev, M, N, K, what):
+def test_tiny_operands(dev, M, N, K, what, up, over):
     """Operands around 2^-120 have no third bfloat16 term of their own (14 of 24 bits would remain, 3e-5 in the
-    2-norm): they are as exact as any others."""
+    2-norm), those around 2^-138 none at all: they are as exact as any others, whatever they meet."""
     call = make_linear(f"tiny_{what}_{M}x{N}x{K}", M, N, K, seed=K, bias=False)
-    setattr(call, what, getattr(call, what) * np.float32(2.0 ** -120))
+    other = "w" if what == "x" else "x"
+    setattr(call, what, np.ldexp(getattr(call, what).astype(np.float64), -up).astype(np.float32))
+    setattr(call, other, getattr(call, other) * np.float32(2.0 ** over))
     got = run(dev, call)
     e = ol.errors(got, ol.linear_fp64(call.x, call.w, call.y0, **call.oracle_kwargs()))
     assert e["finite"] and e["rel_l2"] <= TOL and e["max_rel"] <= 1e-5, e
