@@ -65,10 +65,15 @@ typedef struct sa_linear_args {
  * app/gpu/ops.js:35-43 + app/gpu/gemm.js:116-223. */
 int sa_linear_f32(const sa_linear_args* args, void* stream);
 
-/* Name of the kernel class sa_linear_f32 would launch for `args`, after the tile its size fills
- * ("linear_mfma_128x192", ..., "linear_generic"; the larger classes pick their tiles within), or NULL if the arguments are invalid. Host only; no counterpart in the
- * reference (its app/gpu/ops.js:17-24 tile choice is internal). */
+/* Name of the size class of `args`, after the fp32 tile its grid fills ("linear_mfma_128x192", ...,
+ * "linear_generic"), or NULL if the arguments are invalid; the kernel and tile that run it: sa_linear_tile. Host
+ * only; no counterpart in the reference (its app/gpu/ops.js:17-24 tile choice is internal). */
 const char* sa_linear_kernel_name(const sa_linear_args* args);
+
+/* The tile sa_linear_f32 runs `args` with: output rows and columns per workgroup, and the bfloat16 terms its
+ * operands are split into (3, or 1 for fp32 products). SA_OK, or the status of a rejected call. Host only;
+ * no counterpart in the reference. */
+int sa_linear_tile(const sa_linear_args* args, int32_t* rows, int32_t* cols, int32_t* terms);
 
 #ifdef __cplusplus
 }

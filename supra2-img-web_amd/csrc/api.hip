@@ -806,6 +806,15 @@ const char* sa_linear_kernel_name(const sa_linear_args* args) {
   return sa::linear_kernel_name(p, num_cus());
 }
 
+int sa_linear_tile(const sa_linear_args* args, int32_t* rows, int32_t* cols, int32_t* terms) {
+  if (!rows || !cols || !terms) return fail(SA_ERR_INVALID, "rows, cols and terms must be non-NULL");
+  sa::LinearParams p;
+  const int rc = resolve_linear(args, &p);
+  if (rc != SA_OK) return rc;
+  sa::linear_tile(p, num_cus(), rows, cols, terms);
+  return ok();
+}
+
 int sa_vae_attention_f32(const sa_vae_attn_args* a, void* stream) {
   if (a == nullptr) return fail(SA_ERR_INVALID, "args is NULL");
   VaeLayout L;

@@ -188,6 +188,8 @@ struct LinearTile {
 bool linear_mfma_supported(const LinearParams& p);
 LinearTile linear_mfma_tile(const LinearParams& p, int num_cus);
 const char* linear_kernel_name(const LinearParams& p, int num_cus);
+// The output tile that launch_linear runs p with, and the terms its operands are split into (1: fp32 products).
+void linear_tile(const LinearParams& p, int num_cus, int* rows, int* cols, int* terms);
 hipError_t launch_linear(const LinearParams& p, int num_cus, hipStream_t stream);
 
 // ---- GroupNorm over an NHWC image [HW, C] in `groups` channel groups (csrc/groupnorm.hip).

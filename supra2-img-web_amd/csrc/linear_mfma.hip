@@ -192,6 +192,10 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
   constexpr int G = NT / GW;
   constexpr int NF = (NT + NW - 1) / NW;    // W fragments per wave (the last waves may have one less)
   constexpr int STAGE = NT * 3 * 64;        // 16-byte chunks per stage: [fragment][term][lane]
+  // Sums per output: two on the smallest tile, which takes calls of the two-split fp32 kernel and must not be
+  // less exact: the products of first terms, and all others, whose sum is too small to round them (2-norm at
+  // K = 576 / 2304: 1.4e-7 / 2.9e-7, in one sum 3.6e-7 / 7.4e-7, that kernel 3.05e-7 / 6.1e-7)
+  constexpr int CH = MT * NT <= 4 ? 2 : 1;
   static_assert(G * GW == NT, "column fragments must split into groups");
 
   __shared__ u32x4 lds[2 * STAGE];
@@ -258,11 +262,13 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
     }
   };
   Split8 a[2][MT];
-  f32x4 acc[MT][NT];
+  f32x4 acc[CH][MT][NT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int c = 0; c < CH; ++c)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // k-tile kt from stage C; the splits of the next tile go between the groups' MFMAs
   auto step = [&](int kt, auto stage) {
@@ -278,18 +284,18 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
       for (int j = 0; j < GW; ++j)
 #pragma unroll
         for (int t = 0; t < 3; ++t) b[j][t] = lds[C * STAGE + (g * GW + j) * 192 + t * 64 + lane];
-      auto products = [&](int t, auto term) {
+      auto products = [&](int t, auto term, int ch = 0) {
 #pragma unroll
         for (int j = 0; j < GW; ++j)
 #pragma unroll
-          for (int i = 0; i < MT; ++i) acc[i][g * GW + j] = mfma16(b[j][t], term(a[C][i]), acc[i][g * GW + j]);
+          for (int i = 0; i < MT; ++i) acc[ch][i][g * GW + j] = mfma16(b[j][t], term(a[C][i]), acc[ch][i][g * GW + j]);
       };
       products(2, [](const Split8& s) { return s.h; });
       products(0, [](const Split8& s) { return s.l; });
       products(1, [](const Split8& s) { return s.m; });
       products(1, [](const Split8& s) { return s.h; });
       products(0, [](const Split8& s) { return s.m; });
-      products(0, [](const Split8& s) { return s.h; });
+      products(0, [](const Split8& s) { return s.h; }, CH - 1);
       if (more) {
 #pragma unroll
         for (int f = 0; f < NF; ++f)
@@ -317,6 +323,12 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
     step(kt + 1, std::integral_constant<int, 1>{});
   }
   if (kt < nkt) step(kt, std::integral_constant<int, 0>{});
+  if constexpr (CH == 2) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[0][i][j] += acc[1][i][j];
+  }
 
   // Two kinds of operands have no three terms, and a wave whose sums they may have reached takes its whole tile
   // again with fp32 MFMAs straight from memory, so such inputs give what float32 products give:
@@ -335,8 +347,8 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        most = max_nan(most, fabsf(acc[i][j][e]));
-        least = min_nan(least, fabsf(acc[i][j][e]));
+        most = max_nan(most, fabsf(acc[0][i][j][e]));
+        least = min_nan(least, fabsf(acc[0][i][j][e]));
       }
   __syncthreads();
   const float floor = 0x1p-107f * sqrtf(static_cast<float>(p.K)) * sqrtf(__uint_as_float(lds_norm));
@@ -347,7 +359,7 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) redo |= !(fabsf(acc[i][j][e]) >= floor) && (acc[i][j][e] != 0.f || floor > 0x1p-80f);
+        for (int e = 0; e < 4; ++e) redo |= !(fabsf(acc[0][i][j][e]) >= floor) && (acc[0][i][j][e] != 0.f || floor > 0x1p-80f);
   }
   if (__builtin_amdgcn_ballot_w64(redo) != 0) {
     redo_tile<ACT, EPI>(p, mw, n0, 16 * MT, BN, lr, lc);
@@ -391,7 +403,7 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
       if constexpr (EPI == LIN_EPI_RESID_GATE) g = load4(p.gate + n, left);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] = apply_act<ACT>(fmaf(acc[i][j][e], p.alpha, v[e]));
+        v[e] = apply_act<ACT>(fmaf(acc[0][i][j][e], p.alpha, v[e]));
         if constexpr (EPI != LIN_EPI_STORE) v[e] = fmaf(g[e], v[e], old[j][e]);
       }
       float* dst = p.y + row + n;
@@ -1055,7 +1067,9 @@ SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) 
   const int64_t n64x64 = per_cu(64, 64);
   const double t64x64[5] = {0, 2 + 14.5 * u, 6 + 16.4 * u, 6.5 + 23.6 * u, 6.5 + 32 * u};
   take(n64x64 / 4 * t64x64[4] + t64x64[n64x64 % 4], kSplit64x64);
-  if (cls.ksplit == 2) {
+  if (cls.ksplit == 2) {  // beside its kernel only the tile that is as exact
+    best = n64x64 / 4 * t64x64[4] + t64x64[n64x64 % 4];
+    t = kSplit64x64;
     take(0.9 * (2 + 6.2 * u * per_cu(32, 64)), kKsplit32x64);
   } else if (cls.wn == 1) {
     take(4 + 2e-6 / 135 * p.M * (double)p.N * p.K, kMfma64);
@@ -1073,6 +1087,21 @@ const char* linear_kernel_name(const LinearParams& p, int num_cus) {
   if (t.wm == 2) return "linear_mfma_128x192";
   if (t.wn == 3) return "linear_mfma_64x192";
   return "linear_mfma_64x64";
+}
+
+void linear_tile(const LinearParams& p, int num_cus, int* rows, int* cols, int* terms) {
+  struct Tile {
+    int rows, cols, terms;
+  };
+  static constexpr Tile kTiles[] = {{64, 64, 1}, {32, 64, 1}, {64, 64, 3}, {64, 96, 3}, {128, 96, 3}, {256, 144, 3}, {256, 192, 3}};
+  Tile t = {16, 16, 1};  // linear_generic_kernel
+  if (linear_mfma_supported(p)) {
+    const LinearTile cls = linear_mfma_tile(p, num_cus);
+    t = cls.ksplit == 4 ? Tile{32, 32, 1} : kTiles[split_tile(p, num_cus, cls)];
+  }
+  *rows = t.rows;
+  *cols = t.cols;
+  *terms = t.terms;
 }
 
 hipError_t launch_linear(const LinearParams& p, int num_cus, hipStream_t stream) {

@@ -55,6 +55,7 @@ SIGNATURES = {
     "sa_attention_variant": (c_int, [c_int32, c_void_p]),
     "sa_linear_f32": (c_int, [c_void_p, c_void_p]),
     "sa_linear_kernel_name": (c_char_p, [c_void_p]),
+    "sa_linear_tile": (c_int, [c_void_p, POINTER(c_int32), POINTER(c_int32), POINTER(c_int32)]),
     "sa_vae_attention_f32": (c_int, [c_void_p, c_void_p]),
     "sa_vae_attention_workspace_bytes": (c_int64, [c_void_p]),
     "sa_t5_bucket_lut": (c_int, [c_int32, c_int32, c_int32, c_int32, c_int32, POINTER(c_int32)]),
@@ -343,6 +344,13 @@ def linear_kernel_name(args: LinearArgs) -> str:
     if name is None:
         raise SaError(-1, lib.sa_last_error().decode())
     return name.decode()
+
+
+def linear_tile(args: LinearArgs) -> tuple[int, int, int]:
+    """(rows, columns, terms) of the tile that linear runs `args` with (sa_linear_tile)."""
+    t = [c_int32(0) for _ in range(3)]
+    check(load().sa_linear_tile(ctypes.byref(args), *(ctypes.byref(x) for x in t)))
+    return tuple(x.value for x in t)
 
 
 def vae_attention(args: VaeAttnArgs, stream: int | None = None) -> None:

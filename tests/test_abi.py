@@ -425,6 +425,17 @@ def test_linear_kernel_choice():
     assert _lib.linear_kernel_name(lin_args(ldy=1 << 22, M=64, y=FAKE + (1 << 44))) == "linear_generic"
 
 
+def test_linear_tile_of_the_two_split_class_is_as_exact():
+    """Wherever two fp32 sums of half the length were summed per output, two split sums or those still are."""
+    seen = set()
+    for N, K in [(1728, 576), (1152, 576), (576, 576), (2304, 576), (576, 2304), (768, 768), (512, 2048), (768, 3072)]:
+        for M in range(64, 5000, 64):
+            a = lin_args(M=M, N=N, K=K)
+            if _lib.linear_kernel_name(a) == "linear_mfma_32x64_ksplit":
+                seen.add(_lib.linear_tile(a))
+    assert seen == {(32, 64, 1), (64, 64, 3)}
+
+
 @pytest.mark.parametrize("over,code", [
     (dict(struct_size=8), _lib.SA_ERR_INVALID),
     (dict(M=0), _lib.SA_ERR_INVALID),

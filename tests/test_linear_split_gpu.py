@@ -88,6 +88,23 @@ def test_tiny_operands(dev, M, N, K, what, up, over):
     assert e["finite"] and e["rel_l2"] <= TOL and e["max_rel"] <= 1e-5, e
 
 
+@pytest.mark.parametrize("M,N,K,fp32", [(3136, 576, 576, 3.05e-7), (3136, 576, 2304, 6.07e-7), (1344, 1536, 512, 2.89e-7)])
+def test_two_sums_per_output(dev, M, N, K, fp32):
+    """Calls that took the two-split fp32 kernel (fp32: its measured 2-norm error on these inputs) are no less exact
+    on the split kernel's 64 x 64 tile, which sums the products of first terms apart (one sum: a fifth more than
+    the fp32 kernel; two: under half)."""
+    call = make_linear(f"two_sums_{M}x{N}x{K}", M, N, K, seed=1, bias=False)
+    st = StagedLinear(dev, call)
+    try:
+        assert _lib.linear_tile(st.args) == (64, 64, 3)
+        got = st.run()
+    finally:
+        st.release()
+    e = ol.errors(got, ol.linear_fp64(call.x, call.w, call.y0, **call.oracle_kwargs()))
+    print(f"[linear split] {call.name} {e['rel_l2']:.3e}", flush=True)
+    assert e["rel_l2"] <= 1.02 * fp32, e
+
+
 @pytest.mark.parametrize("y_off,ldy", [(0, 1108), (1, 1108), (0, 1107), (3, 1109)])
 def test_store_at_any_alignment(dev, y_off, ldy):
     """Plain stores into rows at every 4-byte alignment; nothing beside the rows is written."""
