@@ -1029,51 +1029,58 @@ LinearTile linear_mfma_tile(const LinearParams& p, int num_cus) {
 
 namespace {
 
-// The tile that linear_split_kernel runs a call of the larger classes with, or kMfma64: linear_mfma_kernel
-// on 64 x 64 tiles. Each candidate's time is estimated from how many of its tiles every CU gets, with
-// the times of 1, 2, ... tiles per CU measured at K = 576 and 2304 and linear in K (us; u = K / 576):
-//   256 x 144, 8 waves: 56 / 206 per tile of a CU            (N = 576, 16384 rows: exactly one)
-//   256 x 192, 8 waves: 70 / 249
-//   128 x 96, 4 waves:  35 / 120, 45 / 152, 56 / 213 for 1, 2, 3 tiles on a CU at once
-//   64 x 96, 4 waves:   22 / 78, 30 / 98, 39 / 128, 50 / 165 for 1 .. 4
-//   64 x 64, 4 waves:   16 / 60, 22 / 72, 30 / 101, 38 / 135 for 1 .. 4
-//   64 x 64 fp32 MFMA:  4 us + 135 TFLOP/s, its best rate
-//   32 x 64 fp32 MFMA, two k splits (its class): 2 us + 6.2 u per tile of a CU, and kept unless 10% slower
-//     (3072 x 576 x 576: 26.8 against 22.3 for 64 x 64, 3072 x 576 x 2304 91 / 72; but 1024 x 1536 x 512 18.3 / 20.4)
-// Measured over 8 (N, K) of 512..2304 x 14 row counts from 64 to 16128: the choices take 5.58 ms in all,
-// the fp32 kernels alone 7.13, the best of 13 tiles each time (256 x 128, 256 x 96, 128 x 64, 128 x 48,
-// 64 x 48 and 128 x 96 in 8 waves too) 5.41.
+// The tile that linear_split_kernel runs a call of the larger classes with, or one of the fp32 kernels:
+// kMfma64 (linear_mfma_kernel, 64 x 64) in its class, kKsplit32x64 in its own. Each candidate's time is
+// estimated from how many of its tiles every CU gets, a + b u us for 1, 2, ... of them at once (u = K / 576), fitted
+// over 12 (N, K) of 512..2304 x 64..2304 and 15 row counts of 512 to 16128, plus what the residual epilogues
+// add per million outputs (0.2 us to the fp32 64 x 64 kernel, 0.65 to four-wave tiles, 1.05 to eight-wave ones).
+// Measured over those 278 calls: the choices take 17.54 ms, the best tile each time 17.49, the fp32 kernels alone
+// 23.2 (none of the choices more than 4% longer). The fp32 64 x 64 kernel, the less exact, is taken from 7%
+// faster on: short K (6144 x 1024 x 128: 17 against 20 us), and 4096 x 512 x 2048 (72 / 79). The class of the
+// two-split fp32 kernel takes only the 64 x 64 split tile beside it, whose two sums per output are more
+// exact than its two halves of k.
 enum SplitTile { kMfma64, kKsplit32x64, kSplit64x64, kSplit64x96, kSplit128x96, kSplit256x144, kSplit256x192 };
 SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) {
+  struct Line {
+    double a, b;
+  };
+  static constexpr Line k64x64[] = {{3.4, 14.4}, {5.5, 18.5}, {6.8, 23.7}, {7.2, 31.3}};
+  static constexpr Line k64x96[] = {{5.0, 17.7}, {6.7, 22.5}, {7.8, 30.3}, {7.9, 42.3}};
+  static constexpr Line k128x96[] = {{7.4, 23.8}, {9.6, 32.4}, {10.4, 48.5}};
+  static constexpr Line k256x144[] = {{12.3, 39.5}};
+  static constexpr Line k256x192[] = {{14.1, 59.0}};
   const double u = p.K / 576.0;
+  const double resid = p.epi == LIN_EPI_STORE ? 0 : 1e-6 * p.M * (double)p.N;  // million outputs read back
   auto per_cu = [&](int bm, int bn) {
     const int64_t tiles = (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
     return (tiles + num_cus - 1) / num_cus;
   };
-  const int64_t n64 = per_cu(64, 96), n128 = per_cu(128, 96);
-  const double t64[5] = {0, 3.5 + 18.5 * u, 7.5 + 22.5 * u, 9 + 30 * u, 12 + 38 * u};
-  const double t128[4] = {0, 6 + 28.5 * u, 9 + 36 * u, 4 + 52 * u};
-  double best = n64 / 4 * t64[4] + t64[n64 % 4];
-  SplitTile t = kSplit64x96;
-  auto take = [&](double cost, SplitTile c) {
-    if (cost < best) {
-      best = cost;
-      t = c;
+  // n tiles per CU: whole residencies, then the rest at once; where several tiles share a CU the next one's start
+  // covers half of the last one's
+  auto cost = [&](int bm, int bn, const auto& lines, double per_output) {
+    constexpr int64_t cap = sizeof(lines) / sizeof(Line);
+    const int64_t n = per_cu(bm, bn);
+    auto t = [&](int64_t k) { return k == 0 ? 0.0 : lines[k - 1].a + lines[k - 1].b * u; };
+    const double covered = cap == 1 ? 0.0 : 0.5 * (double)((n - 1) / cap) * lines[cap - 1].a;
+    return n / cap * t(cap) + t(n % cap) - covered + per_output * resid;
+  };
+  double best = cost(64, 64, k64x64, 0.65);
+  SplitTile t = kSplit64x64;
+  auto take = [&](double c, SplitTile tile) {
+    if (c < best) {
+      best = c;
+      t = tile;
     }
   };
-  take(n128 / 3 * t128[3] + t128[n128 % 3], kSplit128x96);
-  take(per_cu(256, 144) * (6 + 50 * u), kSplit256x144);
-  take(per_cu(256, 192) * (10 + 60 * u), kSplit256x192);
-  const int64_t n64x64 = per_cu(64, 64);
-  const double t64x64[5] = {0, 2 + 14.5 * u, 6 + 16.4 * u, 6.5 + 23.6 * u, 6.5 + 32 * u};
-  take(n64x64 / 4 * t64x64[4] + t64x64[n64x64 % 4], kSplit64x64);
-  if (cls.ksplit == 2) {  // beside its kernel only the tile that is as exact
-    best = n64x64 / 4 * t64x64[4] + t64x64[n64x64 % 4];
-    t = kSplit64x64;
-    take(0.9 * (2 + 6.2 * u * per_cu(32, 64)), kKsplit32x64);
-  } else if (cls.wn == 1) {
-    take(4 + 2e-6 / 135 * p.M * (double)p.N * p.K, kMfma64);
+  if (cls.ksplit == 2) {  // three or four 32 x 64 tiles per CU
+    take((per_cu(32, 64) <= 3 ? 4.4 + 14.6 * u : 5.2 + 20.6 * u) + 0.85 * resid, kKsplit32x64);
+    return t;
   }
+  take(cost(64, 96, k64x96, 0.65), kSplit64x96);
+  take(cost(128, 96, k128x96, 0.65), kSplit128x96);
+  take(cost(256, 144, k256x144, 1.05), kSplit256x144);
+  take(cost(256, 192, k256x192, 1.05), kSplit256x192);
+  if (cls.wn == 1) take(1.07 * (3.4 + per_cu(64, 64) * (0.4 + 8.45 * u) + 0.2 * resid), kMfma64);
   return t;
 }
 

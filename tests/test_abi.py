@@ -425,6 +425,19 @@ def test_linear_kernel_choice():
     assert _lib.linear_kernel_name(lin_args(ldy=1 << 22, M=64, y=FAKE + (1 << 44))) == "linear_generic"
 
 
+@pytest.mark.parametrize("M,N,K,tile", [
+    (16384, 2304, 576, (256, 144, 3)), (16384, 576, 2304, (256, 144, 3)), (10240, 2304, 576, (256, 192, 3)),
+    (4096, 1536, 512, (128, 96, 3)),
+    (3072, 1152, 576, (64, 96, 3)), (4096, 576, 576, (64, 96, 3)),
+    (3136, 576, 576, (64, 64, 3)),     # class 32x64 of the two-split kernel: its split tile keeps two sums
+    (1024, 1536, 512, (32, 64, 1)),    # the same class, VAE q|k|v: the two-split kernel itself
+    (6144, 1024, 128, (64, 64, 1)),    # short K: fp32 products
+    (512, 1728, 576, (32, 32, 1)), (512, 1728, 36, (16, 16, 1)),
+])
+def test_linear_tile(M, N, K, tile):
+    assert _lib.linear_tile(lin_args(M=M, N=N, K=K)) == tile
+
+
 def test_linear_tile_of_the_two_split_class_is_as_exact():
     """Wherever two fp32 sums of half the length were summed per output, two split sums or those still are."""
     seen = set()
