@@ -1,5 +1,6 @@
-"""The linear layer on the bf16 matrix cores (linear_split_kernel): every tile at ragged M, N and K, every
-epilogue, rows that are not 16-byte aligned, and values that have no three bfloat16 terms.
+"""The linear layer on the bf16 matrix cores (linear_split_kernel): every tile (asserted) at ragged M, N and K,
+every epilogue and activation on each, rows that are not 16-byte aligned, and values that have no three
+bfloat16 terms on each tile.
 
 Tolerance: each operand is held to 24 bits and six of the nine term products are kept, so a sum of K
 products differs from 64 bits by the rounding of its K/32 * 6 float32 additions, at most
@@ -21,50 +22,65 @@ pytestmark = pytest.mark.gpu
 
 TOL = 2e-6
 
-# (M, N, K): 64 x 96, 128 x 96, 256 x 144 and 256 x 192 tiles on 256 CUs, each ragged in M and N, with
-# K % 32 of 8, 24 and 16 (and one k-tile more or less than even), and K shorter than one k-tile
+# tile: (M, N, K) that take it on 256 CUs whatever the epilogue, ragged in M and N, K % 32 of 8, 16 and 24, K shorter
+# than one k-tile and an odd and an even number of them
+TILES = {
+    (64, 64): [(1225, 1225, 264), (4715, 1945, 8), (3100, 570, 584)],
+    (64, 96): [(1798, 1091, 336), (2767, 2202, 8), (2047, 2050, 776)],
+    (128, 96): [(10355, 389, 264), (3715, 2103, 8), (3071, 1730, 584)],
+    (256, 144): [(10909, 517, 272), (5841, 1574, 88)],
+    (256, 192): [(11528, 775, 264), (3905, 2313, 264)],
+}
+CASES = [(tile, *size) for tile, sizes in TILES.items() for size in sizes]
+# sizes between the tiles' classes, and two where the fp32 64 x 64 kernel takes over
 SIZES = [(2047, 2050, 776), (3071, 1730, 584), (16300, 570, 40), (16300, 760, 72), (16299, 571, 24), (16299, 763, 48),
          (16333, 1729, 8)]
+EPILOGUES = [
+    (_lib.SA_EPI_STORE, _lib.SA_ACT_NONE, {}),
+    (_lib.SA_EPI_RESID_GATE, _lib.SA_ACT_GELU_TANH, dict(gate_off=3)),  # gate not 16-byte aligned
+    (_lib.SA_EPI_RESID, _lib.SA_ACT_SILU, dict(y_off=1)),               # rows of y not aligned
+    (_lib.SA_EPI_STORE, _lib.SA_ACT_GELU, dict(y_off=2)),
+]
 
 
-def run(dev, call):
-    print(f"[linear split] {call.name} M={call.M} N={call.N} K={call.K} act={call.act} epi={call.epi}", flush=True)
+def run(dev, call, tile=None):
     st = StagedLinear(dev, call)
     try:
+        took = _lib.linear_tile(st.args)
+        print(f"[linear split] {call.name} M={call.M} N={call.N} K={call.K} act={call.act} epi={call.epi} tile={took}", flush=True)
+        assert tile is None or took == (*tile, 3)
         return st.run()
     finally:
         st.release()
 
 
-@pytest.mark.parametrize("M,N,K", SIZES)
-@pytest.mark.parametrize("epi,act,kw", [
-    (_lib.SA_EPI_STORE, _lib.SA_ACT_NONE, {}),
-    (_lib.SA_EPI_RESID_GATE, _lib.SA_ACT_GELU_TANH, dict(gate_off=3)),  # gate not 16-byte aligned
-    (_lib.SA_EPI_RESID, _lib.SA_ACT_SILU, dict(y_off=1)),               # rows of y not aligned
-])
-def test_tiles(dev, M, N, K, epi, act, kw):
+@pytest.mark.parametrize("tile,M,N,K", CASES + [(None, *size) for size in SIZES])
+@pytest.mark.parametrize("epi,act,kw", EPILOGUES)
+def test_tiles(dev, tile, M, N, K, epi, act, kw):
     kw = dict(kw, ldy=(N + 7) // 4 * 4)
     call = make_linear(f"split_{M}x{N}x{K}", M, N, K, seed=M + N + K + epi, act=act, epi=epi, **kw)
-    got = run(dev, call)
+    got = run(dev, call, tile)
     e = ol.errors(got, ol.linear_fp64(call.x, call.w, call.y0, **call.oracle_kwargs()))
     assert e["finite"] and e["rel_l2"] <= TOL and e["max_rel"] <= 1e-5, e
 
 
-@pytest.mark.parametrize("M,N,K", [(2047, 2050, 776), (16300, 570, 40)])
-def test_values_without_three_terms(dev, M, N, K):
+@pytest.mark.parametrize("tile,M,N,K", [(tile, *sizes[0]) for tile, sizes in TILES.items()] + [(None, 2047, 2050, 776), (None, 16300, 570, 40)])
+@pytest.mark.parametrize("epi,act,kw", EPILOGUES[:3])
+def test_values_without_three_terms(dev, tile, M, N, K, epi, act, kw):
     """Infinities, NaN, and magnitudes that round past the bfloat16 range (finite products) give what
     float32 products give: the same elements infinite, NaN or finite, and the finite ones to tolerance."""
-    call = make_linear(f"special_{M}x{N}x{K}", M, N, K, seed=K)
+    call = make_linear(f"special_{M}x{N}x{K}", M, N, K, seed=K, act=act, epi=epi, **dict(kw, ldy=(N + 7) // 4 * 4))
     x = call.x.reshape(-1)
     x[5 * K + 3] = np.inf
     x[700 * K + 7] = -np.inf
-    x[1400 * K] = np.nan
-    x[2046 * K + 1] = np.float32(3.4e38)
+    x[900 * K] = np.nan
+    x[(M - 1) * K + 1] = np.float32(3.4e38)
     w = call.w.reshape(-1)
     w[(N - 1) * K + 2] = np.inf
     w[40 * K + 3] = 0.0  # inf * 0
-    got = run(dev, call).reshape(-1)
-    ref = ol.linear_torch_fp32(call.x, call.w, call.y0, **call.oracle_kwargs()).reshape(-1)
+    idx = (call.y_off + np.arange(M)[:, None] * call.ldy + np.arange(N)).reshape(-1)
+    got = run(dev, call, tile).reshape(-1)[idx]
+    ref = ol.linear_torch_fp32(call.x, call.w, call.y0, **call.oracle_kwargs()).reshape(-1)[idx]
     np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
     np.testing.assert_array_equal(np.isinf(got), np.isinf(ref))
     np.testing.assert_array_equal(got[np.isinf(got)], ref[np.isinf(ref)])
