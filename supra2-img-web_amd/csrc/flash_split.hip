@@ -19,6 +19,7 @@
 
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -500,35 +501,60 @@ hipError_t launch_bias(const AttnParams& p, hipStream_t stream) {
 
 }  // namespace
 
-// Waves per workgroup by how many 128-query units every CU gets (us, unmasked, 256 keys unless stated;
-// fp32: the fp32 MFMA flash kernel that these replace):
-//   head dim 64                    4 groups x 1   4 x 2 splits   2 x 4 splits   fp32
-//     72 units                          16.7           15.4            12.0     13.7
-//     72 units, 77 keys                  8.7            9.8             8.5      9.0
-//     192 units, 512 keys               29.5           26.5            34.9     38.7
-//     234 units                         17.0           17.0            22.8     22.1
-//     234 units, 77 keys                 9.3           10.8            15.8     14.0
-//     288 units                         24.1           30.9            33.0     32.8
-//     1026 units                        57.2           80.9            96.9     77.2
-//   head dim 128             4 x 1, two stages  4 x 1, one stage   2 x 2 splits   fp32
-//     64 units of 64, 500 keys          51.5           69.7            37.0     42.8
-//     256 units, 777 keys               87.5          124              117      142
-//     384 units, 1000 keys             195            188              206      238
-// So: at most half a unit per CU, 64-query workgroups that split the keys; one per CU, the 4 x 2 split
-// for long keys; past that 4 groups (three workgroups per CU at head dim 64, two at 128 in one stage).
-hipError_t launch_flash_split(const AttnParams& p, int num_cus, hipStream_t stream) {
-  const int64_t units = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
+// Groups of 32 queries x key splits per workgroup, [stages], by the workgroups a launch makes. Means of
+// 1416 (head dim 128) and 888 (64) calls of 1 to 58 sequences x 4 to 12 heads, 4 to 700 queries, 8 to 1000 keys, with and without
+// dense bias and key lengths, as a ratio to the fp32 MFMA kernel that these replaced:
+//   head dim 64                                       2x2 [2]  2x2 [1]  2x4 [1]  4x2 [2]  4x1 [2]
+//     up to 256 workgroups of 64 queries, 2-4 blocks    0.91     0.92     1.04     1.18     1.11
+//       5-10 blocks                                     0.85     0.89     0.90     1.04     1.16
+//       more                                            0.80     0.85     0.71     0.93     1.14
+//     at most 64 queries, more workgroups, 2+ blocks    1.08     0.83     1.05     1.23     1.03
+//     up to 256 of 128 queries, 2 / 3-4 blocks          1.2      0.9      1.3      0.95/0.78  0.83/0.76
+//       5-10 blocks                                     1.03     0.81     1.09     0.71     0.75
+//     more                                              1.1-1.5  0.7-1.0  0.9-1.9  0.7-1.3  0.62-0.74
+//     one block of keys                                 1.0-2.3  0.9-1.5  1.2-3.0  1.1-1.7  0.71-0.91
+//   head dim 128                                      2x2 [1]  4x1 [2]  4x1 [1], no bias
+//     one block of keys                                 1.0-1.8  0.87-1.0  0.9-1.2
+//     up to 128 units of 128 queries                    0.71-0.99  1.04-1.2  1.4-2.2
+//     257-512 units, 3+ blocks                          0.90     0.94     0.92 (600 units of 1000 keys 168 us against 201)
+//     more                                              0.7-1.1  0.56-0.83  0.78-0.84
+// Head dim 64 therefore counts the workgroups of a shape; head dim 128, where one workgroup fills a CU, takes the
+// least of three estimates fitted to the same calls (us per round of workgroups). 4x1 [1] puts two workgroups
+// on a CU at 256 registers a wave and spills 47 to 65 of them, more with a bias (1.4 times the fp32 kernel):
+// it is not compiled with one.
+struct FlashShape {
+  int groups, splits, stages;
+};
+FlashShape flash_shape(const AttnParams& p, int num_cus) {
+  const int64_t units = (int64_t)p.B * p.H * ((p.Lq + 127) / 128), half_units = (int64_t)p.B * p.H * ((p.Lq + 63) / 64);
   const int nblk = (p.Lk + 31) / 32;
+  if (nblk == 1) return {4, 1, 2};
   if (p.D == 64) {
-    // (up to four key blocks two splits, whose merge is a third: 108 units, 40 keys 6.2 us against 7.6)
-    if (2 * units <= num_cus) return nblk <= 4 ? launch_bias<64, 2, 2, 2, 2>(p, stream) : launch_bias<64, 2, 4, 1, 2>(p, stream);
-    if (units <= num_cus && nblk > 8) return launch_bias<64, 4, 2, 2, 2>(p, stream);
-    return launch_bias<64, 4, 1, 2, 2>(p, stream);
+    if (half_units <= num_cus) return nblk <= 8 ? FlashShape{2, 2, 2} : FlashShape{2, 4, 1};
+    if (p.Lq <= 64) return {2, 2, 1};
+    if (units <= num_cus && nblk > 8) return {4, 2, 2};
+    return {4, 1, 2};
+  }
+  const int64_t per_cu = (units + num_cus - 1) / num_cus, half_per_cu = (half_units + num_cus - 1) / num_cus;
+  const bool bias = p.bias_mode != BIAS_NONE;
+  const int steps = (nblk + 1) / 2;  // of two blocks
+  const double split = (double)half_per_cu * (bias ? 6.2 + 4.45 * steps : 5.4 + 4.1 * steps);
+  const double whole = (double)per_cu * (bias ? 5.9 + 3.5 * nblk : 5.5 + 2.98 * nblk);
+  const double pairs = 1.03 * ((double)(per_cu / 2) * (10 + 5.8 * nblk) + (double)(per_cu % 2) * (6 + 3.9 * nblk));
+  if (!bias && pairs < std::min(split, whole)) return {4, 1, 1};
+  return split < whole ? FlashShape{2, 2, 1} : FlashShape{4, 1, 2};
+}
+
+hipError_t launch_flash_split(const AttnParams& p, int num_cus, hipStream_t stream) {
+  const FlashShape s = flash_shape(p, num_cus);
+  if (p.D == 64) {
+    if (s.groups == 2 && s.splits == 4) return launch_bias<64, 2, 4, 1, 2>(p, stream);
+    if (s.groups == 2) return s.stages == 2 ? launch_bias<64, 2, 2, 2, 2>(p, stream) : launch_bias<64, 2, 2, 1, 2>(p, stream);
+    return s.splits == 2 ? launch_bias<64, 4, 2, 2, 2>(p, stream) : launch_bias<64, 4, 1, 2, 2>(p, stream);
   }
   if (p.D == 128) {
-    if (2 * units <= num_cus) return launch_bias<128, 2, 2, 1, 1>(p, stream);
-    if (units <= num_cus) return launch_bias<128, 4, 1, 2, 1>(p, stream);
-    return launch_bias<128, 4, 1, 1, 2>(p, stream);
+    if (s.groups == 2) return launch_bias<128, 2, 2, 1, 1>(p, stream);
+    return s.stages == 2 ? launch_bias<128, 4, 1, 2, 1>(p, stream) : launch_mask<128, 4, 1, 1, 2, BIAS_NONE>(p, stream);
   }
   return hipErrorInvalidValue;
 }
