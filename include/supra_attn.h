@@ -153,16 +153,17 @@ int64_t sa_attention_workspace_bytes(const sa_attn_args* args);
  * is then sa_last_status()). Host only. */
 const char* sa_attention_kernel_name(const sa_attn_args* args);
 
-/* ---- kernel plan: the compiled kernel a call launches, and every compiled variant ----
+/* ---- kernel plan: how a call is run, and the kernel variants ----
  * The reference picks a matmul tile (app/gpu/ops.js:15-31) and decides fused vs unfused
  * (ops.js:111-112) inside the operator; these host-only queries make the equivalent choice of
- * this library inspectable, so tests can show that every compiled variant runs. */
-#define SA_KERNEL_FLASH 1   /* flash attention, head dim 64 or 128. A plan counts these calls by launch class:
-                               units of 128 queries (64 at key_split 2), units past the last whole
-                               round as a tail. The kernel that runs a class (flash_split_kernel) groups
-                               queries, splits keys and shapes its grid by itself. */
-#define SA_KERNEL_WIDE 2    /* wide_mfma_kernel<head_dim, bias_mode, mask_variant> (no bias or a dense one), + a
-                                merge kernel when key_chunks > 1 */
+ * this library inspectable. */
+#define SA_KERNEL_FLASH 1   /* flash attention, head dim 64 or 128: one launch of flash_split_kernel, whose shape the
+                               plan's flash_* fields give. key_split, keys_per_step, workgroups, the name and the
+                               tail fields are those of the call's launch class, which counts it in units of 128
+                               queries (64 at key_split 2): what the key-length schedule works on, and what
+                               earlier revisions launched. */
+#define SA_KERNEL_WIDE 2    /* wide_split_kernel (head dim 512) or wide_mfma_kernel (256) <bias_mode, mask_variant> (no
+                                bias or a dense one), + a merge kernel when key_chunks > 1 */
 #define SA_KERNEL_GENERIC 3 /* generic_kernel (any head dim <= 1024, any alignment) */
 #define SA_KERNEL_FLASH_SMALL 4 /* flash_small_kernel<key_split waves, bias_mode, mask_variant>: head dim 64,
                                    one workgroup per 32 queries, for launches of at most 256 such groups */
@@ -179,25 +180,21 @@ typedef struct sa_attn_plan {
   uint32_t struct_size;    /* set to sizeof(sa_attn_plan) before the call */
   int32_t kernel;          /* SA_KERNEL_* */
   int32_t head_dim;        /* head dim the kernel is compiled for (the call's D for GENERIC) */
-  int32_t key_split;       /* FLASH, FLASH_SMALL: waves of a workgroup that split one query group's key blocks */
+  int32_t key_split;       /* FLASH_SMALL: waves of a workgroup that split one query group's key blocks; FLASH: the class's */
   int32_t key_chunks;      /* WIDE: workgroups that split one query group's keys (merged after) */
   int32_t bias_mode;       /* SA_BIAS_* compiled into the kernel */
   int32_t mask_variant;    /* SA_MASK_* compiled into the kernel, or SA_MASK_VARIANT_KEY_LEN_SCHEDULED */
-  int32_t keys_per_step;   /* FLASH: keys a workgroup stages per loop step (32 per splitting wave); WIDE: keys per chunk */
-  int64_t workgroups;      /* grid of the attention kernel */
+  int32_t keys_per_step;   /* FLASH, FLASH_SMALL: 32 per key_split; WIDE: keys per chunk */
+  int64_t workgroups;      /* grid of the attention kernel (FLASH: of its class, less the tail) */
   int64_t workspace_bytes; /* sa_attention_workspace_bytes(args) */
   const char* name;        /* sa_attention_kernel_name(args) (static storage) */
-  /* FLASH launches of more units (query tiles) than fit the GPU at once whose last round holds
-   * few units: those last units run at one workgroup per CU, in a second launch of the
-   * small-launch kernel (tail_kernel SA_KERNEL_FLASH_SMALL, tail_key_split 4 waves per 32 queries)
-   * or of the flash kernel split by keys over 2 waves per 32 queries (SA_KERNEL_FLASH, 2), or, when
-   * tail_folded is 1, as 64-query units of the latter run inside the first launch (see tail_folded);
-   * tail_kernel is 0 when there are no such units, tail_workgroups the number of workgroups (or, folded,
-   * of 64-query units) they take. WIDE calls whose query groups fill whole rounds of workgroups
+  /* WIDE calls whose query groups fill whole rounds of workgroups
    * (one per CU at head dim 512, two at 256) and a few more: the whole rounds run unsplit (key_chunks
    * 1, workgroups = their groups) and the groups past them follow in a second launch of the wide
    * kernel (tail_kernel SA_KERNEL_WIDE), each split into tail_key_split key chunks merged after;
-   * tail_workgroups is that launch's grid. */
+   * tail_workgroups is that launch's grid. FLASH classes of more units than four per CU whose last round
+   * holds few: those units, as 32-query groups (tail_kernel SA_KERNEL_FLASH_SMALL) or 64-query units
+   * (SA_KERNEL_FLASH); a figure of the class, the launch runs them with the others. Otherwise 0. */
   int32_t tail_kernel;
   int32_t tail_key_split;
   int64_t tail_workgroups;
@@ -208,22 +205,29 @@ typedef struct sa_attn_plan {
    * the next domain's first) and order_n is B; otherwise order_n is 0 and sequence_order all zero. */
   int32_t order_n;
   uint8_t sequence_order[256];
-  /* Revision 3 (appended: revision-1 and revision-2 structs are still accepted, without it). 1 when
-   * the units past the first round run inside the first launch: a launch of one round plus at most
-   * half a round, whose first tail_workgroups workgroups (the first one on each CU) each run one
-   * 64-query unit of them, split by keys over 2 waves per 32 queries, after their own unit; 0 otherwise. */
+  /* Revision 3 (appended: revision-1 and revision-2 structs are still accepted, without it). FLASH classes: 1
+   * when the tail is 64-query units past a single round. */
   int32_t tail_folded;
+  /* Revision 4 (appended: the shorter structs are still accepted, without these). The launch of a FLASH
+   * call, 0 otherwise: workgroups of flash_groups x flash_splits waves, a group of 32 queries seen by flash_splits
+   * waves that share its key blocks, the keys and values of a step in flash_stages LDS buffers, flash_workgroups of
+   * them. */
+  int32_t flash_groups;
+  int32_t flash_splits;
+  int32_t flash_stages;
+  int64_t flash_workgroups;
 } sa_attn_plan;
 
 /* Fills *plan for these arguments: SA_OK, or the status sa_attention_f32 would return for a
- * rejected call (nothing is launched either way). plan->struct_size: sizeof(sa_attn_plan), or the
- * revision-2 size (offsetof(sa_attn_plan, tail_folded)) or the revision-1 size
+ * rejected call (nothing is launched either way). plan->struct_size: sizeof(sa_attn_plan), or the size of
+ * revision 3 (offsetof(sa_attn_plan, flash_groups)), 2 (offsetof(sa_attn_plan, tail_folded)) or 1
  * (offsetof(sa_attn_plan, order_n)). Host only. */
 int sa_attention_plan(const sa_attn_args* args, sa_attn_plan* plan);
 
-/* Number of compiled kernel variants; sa_attention_variant(i, plan) describes variant i
- * (kernel, head_dim, key_split, bias_mode, mask_variant, name; the other fields 0). FLASH
- * variants come first, one per <head_dim, key_split, bias_mode, mask_variant>. Host only. */
+/* Number of kernel variants; sa_attention_variant(i, plan) describes variant i
+ * (kernel, head_dim, key_split, bias_mode, mask_variant, name; the other fields 0): the compiled variants of
+ * the other kernels, and the launch classes of FLASH, which come first, one per <head_dim, key_split, bias_mode,
+ * mask_variant> (each runs in one of the compiled shapes that the plan's flash_* fields name). Host only. */
 int32_t sa_attention_variant_count(void);
 int sa_attention_variant(int32_t index, sa_attn_plan* plan);
 

@@ -91,11 +91,14 @@ bool too_large(int64_t v) { return v >= kMaxExtent; }
 
 // Size of the revision-2 struct (it ended at workspace_bytes); still accepted.
 constexpr uint32_t kAttnArgsV2Size = offsetof(sa_attn_args, key_len_host);
-// Sizes of the revision-1 sa_attn_plan (it ended at tail_workgroups) and of revision 2 (it ended at
-// sequence_order); still accepted.
+// Sizes of the revision-1 sa_attn_plan (it ended at tail_workgroups), of revision 2 (it ended at
+// sequence_order) and of revision 3 (it ended at tail_folded); still accepted.
 constexpr uint32_t kPlanV1Size = offsetof(sa_attn_plan, order_n);
 constexpr uint32_t kPlanV2Size = offsetof(sa_attn_plan, tail_folded);
-bool plan_size_ok(uint32_t size) { return size == sizeof(sa_attn_plan) || size == kPlanV2Size || size == kPlanV1Size; }
+constexpr uint32_t kPlanV3Size = offsetof(sa_attn_plan, flash_groups);
+bool plan_size_ok(uint32_t size) {
+  return size == sizeof(sa_attn_plan) || size == kPlanV3Size || size == kPlanV2Size || size == kPlanV1Size;
+}
 
 int num_cus();
 
@@ -103,8 +106,8 @@ int num_cus();
 // grid's workgroup remap gives L2 domain (XCD) x the ranks [x*B/8, (x+1)*B/8) in launch order, T
 // consecutive units (query tiles x heads) per rank, and within a domain the hardware deals
 // workgroup j of the first residency to CU j % C (C CUs per domain, S workgroups per CU: 4 for the
-// unbiased head-dim-64 single-split kernel, 1 for the others; the later workgroups take the first
-// slots that free up). A CU's time is about the sum of its units' key blocks, so:
+// unbiased head-dim-64 single-split class, 1 for the others, as measured best, flash_mfma_per_cu; the later
+// workgroups take the first slots that free up). A CU's time is about the sum of its units' key blocks, so:
 //   1. sequences sorted by key blocks, longest first (stable), go to the domain with the least work
 //      so far among those not yet full (B/8 each) - the sums per domain come out nearly equal;
 //   2. in each domain, from longest first, pairs of positions are swapped while that lowers the
@@ -929,6 +932,11 @@ int sa_attention_plan(const sa_attn_args* args, sa_attn_plan* plan) {
     plan->mask_variant = fv.mask;
     plan->keys_per_step = 32 * fv.nsplit;
     plan->workgroups = sa::flash_mfma_workgroups(p, c.nsplit, num_cus());
+    const sa::FlashShape fs = sa::flash_shape(p, num_cus());
+    plan->flash_groups = fs.groups;
+    plan->flash_splits = fs.splits;
+    plan->flash_stages = fs.stages;
+    plan->flash_workgroups = (int64_t)p.B * p.H * ((p.Lq + 32 * fs.groups - 1) / (32 * fs.groups));
     const int64_t tail = sa::flash_mfma_tail_units(p, c.nsplit, num_cus());
     if (tail > 0) {
       const int tk = sa::flash_mfma_tail_kernel(p, c.nsplit, num_cus());

@@ -1,7 +1,7 @@
 // Host side of the flash attention launches (head dim 64 or 128, csrc/flash_split.hip): the packed kernel
 // arguments, and the launch classes that a plan reports and the key-length schedule works on. A class
-// counts a call in units of 128 queries (64 with a 2-way key split, calls of under 2048 groups of 32);
-// the kernel that runs it may group queries and split keys differently (launch_flash_split).
+// counts a call in units of 128 queries (64 with a 2-way key split, calls of under 2048 groups of 32), which is
+// not how it is launched: flash_shape groups queries and splits keys, and one grid runs them all.
 
 #include <string.h>
 
@@ -62,23 +62,20 @@ const char* flash_mfma_name(int D, int nsplit) {
 constexpr int kSplits64[] = {1, 2};
 constexpr int kSplits128[] = {1, 2};
 
-static int compiled_split(int D, int nsplit) {
-  (void)D;
-  return nsplit >= 2 ? 2 : 1;
-}
+static int class_split(int nsplit) { return nsplit >= 2 ? 2 : 1; }
 
 FlashVariant flash_mfma_variant(const AttnParams& p, int nsplit) {
   int mask = p.mask_mode;
   if (mask == MASK_KEY_LEN && p.order_n > 0) mask = MASK_KEY_LEN_ORDERED;
-  return {p.D, compiled_split(p.D, nsplit), p.bias_mode, mask};
+  return {p.D, class_split(nsplit), p.bias_mode, mask};
 }
 
-// Units past the last whole round of four per CU, and how a plan reports them: few enough for 32-query
-// groups or 64-query units at one per CU in a launch of their own, or, after a single round, within it.
-// flash_split_kernel runs every unit in one grid, three workgroups per CU, where the leftover of
-// a round costs what it holds: batch 57 / 60 / 64 of the DiT self-attention take 57 / 59 / 62 us.
+// Units of a class past the last whole round of four per CU, and what plans call them: few enough for 32-query
+// groups or 64-query units at one per CU. No launch of theirs follows: flash_split_kernel runs every
+// unit in one grid (three workgroups per CU without a mask, two in the other variants, by registers), where the
+// leftover of a round costs what it holds: batch 57 / 60 / 64 of the DiT self-attention take 57 / 59 / 62 us.
 int64_t flash_mfma_tail_units(const AttnParams& p, int nsplit, int num_cus) {
-  const bool eligible = p.D == 64 && compiled_split(p.D, nsplit) == 1 && p.bias_mode == BIAS_NONE &&
+  const bool eligible = p.D == 64 && class_split(nsplit) == 1 && p.bias_mode == BIAS_NONE &&
                         p.mask_mode == MASK_NONE && p.Lk > 32;
   if (!eligible) return 0;
   const int64_t tiles = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
@@ -111,8 +108,12 @@ int64_t flash_mfma_tail_groups(const AttnParams& p, int nsplit, int num_cus, int
   return (int64_t)p.B * p.H * q_sub - *first;
 }
 
-int flash_mfma_unit_queries(int nsplit) { return 32 * (4 / compiled_split(64, nsplit)); }
+int flash_mfma_unit_queries(int nsplit) { return 32 * (4 / class_split(nsplit)); }
 
+// Four and one are what the schedule's model does best with, not what fits a CU (two of the scheduled
+// variant's workgroups at head dim 64): batch 64, prompts of 1 to 128 tokens 27.7 / 27.1 / 27.7 us over three draws
+// with four, 29.2 / 27.6 / 28.9 with two, 29.4 / 27.7 / 28.9 with one, 31.8 / 30.6 / 29.6 in launch order; batch 24 in 64-query
+// units and one per CU 13.5 / 15.0 / 12.5, in 128-query units and two 14.4 / 15.3 / 13.7.
 int flash_mfma_per_cu(const AttnParams& p, int nsplit) {
   const FlashVariant v = flash_mfma_variant(p, nsplit);
   const bool four = v.D == 64 && v.nsplit == 1 && v.bias == BIAS_NONE && v.mask != MASK_KEY_MASK;
@@ -120,7 +121,7 @@ int flash_mfma_per_cu(const AttnParams& p, int nsplit) {
 }
 
 int64_t flash_mfma_workgroups(const AttnParams& p, int nsplit, int num_cus) {
-  const int qt = 32 * (4 / compiled_split(p.D, nsplit));
+  const int qt = 32 * (4 / class_split(nsplit));
   return (int64_t)p.B * p.H * ((p.Lq + qt - 1) / qt) - flash_mfma_tail_units(p, nsplit, num_cus);
 }
 

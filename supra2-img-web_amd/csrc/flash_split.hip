@@ -522,9 +522,6 @@ hipError_t launch_bias(const AttnParams& p, hipStream_t stream) {
 // least of three estimates fitted to the same calls (us per round of workgroups). 4x1 [1] puts two workgroups
 // on a CU at 256 registers a wave and spills 47 to 65 of them, more with a bias (1.4 times the fp32 kernel):
 // it is not compiled with one.
-struct FlashShape {
-  int groups, splits, stages;
-};
 FlashShape flash_shape(const AttnParams& p, int num_cus) {
   const int64_t units = (int64_t)p.B * p.H * ((p.Lq + 127) / 128), half_units = (int64_t)p.B * p.H * ((p.Lq + 63) / 64);
   const int nblk = (p.Lk + 31) / 32;

@@ -75,7 +75,13 @@ FlashArgs flash_args(const AttnParams& p, int64_t tiles);
 // Flash kernel on the bf16 matrix cores, three-term operands (csrc/flash_split.hip), for D in {64, 128} with
 // 16-byte aligned rows (small head-dim-64 launches take flash_small instead).
 hipError_t launch_flash_split(const AttnParams& p, int num_cus, hipStream_t stream);
-// Launch classes of that kernel (csrc/flash_mfma.hip): nsplit in {1, 2}, units of 128 / 64 queries.
+// The shape of that launch: groups of 32 queries x key splits (waves) per workgroup, LDS stages.
+struct FlashShape {
+  int groups, splits, stages;
+};
+FlashShape flash_shape(const AttnParams& p, int num_cus);
+// Launch classes, as plans report them and the key-length schedule works on them (csrc/flash_mfma.hip): nsplit in
+// {1, 2}, units of 128 / 64 queries.
 const char* flash_mfma_name(int D, int nsplit);
 // The flash kernels take 32-bit strides, at most 32767 heads and buckets; other calls take the
 // generic kernel.
@@ -89,13 +95,13 @@ struct FlashVariant {
 FlashVariant flash_mfma_variant(const AttnParams& p, int nsplit);
 // Units of that launch class.
 int64_t flash_mfma_workgroups(const AttnParams& p, int nsplit, int num_cus);
-// Queries per unit of a class, and the units per CU that its key-length schedule assumes (4 for unbiased
-// head-dim-64 single-split classes, 1 for the others).
+// Queries per unit of a class, and the units per CU that its key-length schedule's model takes (4 for unbiased
+// head-dim-64 single-split classes, 1 for the others: flash_mfma.hip).
 int flash_mfma_unit_queries(int nsplit);
 int flash_mfma_per_cu(const AttnParams& p, int nsplit);
-// Units (128-query tiles) past the last whole round that a plan reports as a tail (0 = none), the kernel
-// class of that tail, and its work items [*first, *first + count) (returns count): 32-query groups or
-// 64-query units.
+// Units (128-query tiles) past the last whole round that a plan reports as the tail of the class (0 = none), the kind
+// of that tail, and its items [*first, *first + count) (returns count): 32-query groups or 64-query
+// units. Figures of the class: the launch runs them with the others.
 constexpr int TAIL_NONE = 0, TAIL_SMALL = 1, TAIL_SPLIT2 = 2, TAIL_FOLD = 3;
 int64_t flash_mfma_tail_units(const AttnParams& p, int nsplit, int num_cus);
 int flash_mfma_tail_kernel(const AttnParams& p, int nsplit, int num_cus);

@@ -185,7 +185,11 @@ class AttnPlan(ctypes.Structure):
         ("tail_workgroups", c_int64),
         ("order_n", c_int32),  # revision 2: the host sequence schedule of a scheduled flash call
         ("sequence_order", ctypes.c_uint8 * 256),
-        ("tail_folded", c_int32),  # revision 3: the units past the first round run inside it
+        ("tail_folded", c_int32),  # revision 3: the class's tail is 64-query units past a single round
+        ("flash_groups", c_int32),  # revision 4: the launch of a flash call
+        ("flash_splits", c_int32),
+        ("flash_stages", c_int32),
+        ("flash_workgroups", c_int64),
     ]
 
     def __init__(self):
@@ -193,7 +197,7 @@ class AttnPlan(ctypes.Structure):
         self.struct_size = ctypes.sizeof(AttnPlan)
 
     def variant(self) -> tuple:
-        """(kernel, head_dim, key_split, bias_mode, mask_variant): the compiled variant."""
+        """(kernel, head_dim, key_split, bias_mode, mask_variant): the compiled variant, or a flash call's class."""
         return (self.kernel, self.head_dim, self.key_split, self.bias_mode, self.mask_variant)
 
 

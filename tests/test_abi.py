@@ -110,6 +110,24 @@ def big(B, Lq=256, **over):
 SMALL, FLASH = _lib.SA_KERNEL_FLASH_SMALL, _lib.SA_KERNEL_FLASH
 
 
+@pytest.mark.parametrize("D,B,Lq,Lk,shape,wg", [
+    (64, 64, 256, 256, (4, 1, 2), 1152), (64, 13, 256, 320, (4, 2, 2), 234), (64, 13, 256, 256, (4, 1, 2), 234),
+    (64, 5, 320, 288, (2, 4, 1), 225), (64, 5, 320, 256, (2, 2, 2), 225), (64, 64, 64, 96, (2, 2, 1), 576),
+    (64, 64, 64, 32, (4, 1, 2), 576), (128, 2, 100, 90, (2, 2, 1), 36), (128, 9, 256, 160, (4, 1, 2), 162),
+    (128, 16, 256, 96, (4, 1, 1), 288), (128, 16, 256, 32, (4, 1, 2), 288),
+])
+def test_plan_reports_the_flash_launch(D, B, Lq, Lk, shape, wg):
+    """The shape and grid of the one launch (9 heads, no bias), and none for the other kernels."""
+    hd = 9 * D
+    a = _lib.AttnArgs(B=B, H=9, D=D, Lq=Lq, Lk=Lk, q=FAKE, k=FAKE + (1 << 36), v=FAKE + (1 << 37), o=FAKE + (1 << 38),
+                      ldq=hd, ldk=hd, ldv=hd, sq=Lq * hd, sk=Lk * hd, sv=Lk * hd, so=Lq * hd, scale=0.125)
+    p = _lib.plan(a)
+    assert p.kernel == _lib.SA_KERNEL_FLASH
+    assert (p.flash_groups, p.flash_splits, p.flash_stages) == shape and p.flash_workgroups == wg
+    small = _lib.plan(good_args())
+    assert (small.kernel, small.flash_groups, small.flash_workgroups) == (SMALL, 0, 0)
+
+
 @pytest.mark.parametrize("B,Lq,tail_units,tail_kernel,tail_split,tail_wg,folded", [
     (56, 256, 0, 0, 0, 0, 0),          # 1008 units: one round on 256 CUs
     (57, 256, 2, SMALL, 4, 8, 0),      # 1026: a round of 1024, two left: 8 groups of 32 queries
@@ -124,9 +142,9 @@ SMALL, FLASH = _lib.SA_KERNEL_FLASH_SMALL, _lib.SA_KERNEL_FLASH
     (61, 200, 74, FLASH, 2, 148, 1),   # 4 units of 64 per head (the last one 8 queries)
 ])
 def test_plan_reports_the_tail_launch(B, Lq, tail_units, tail_kernel, tail_split, tail_wg, folded):
-    """The batch-B, 9-head self-attention call on 256 CUs (the count without a device): the units past
-    the last whole round of 1024 run at one workgroup per CU, in a second launch, or, after a single
-    round, as 64-query units folded into the round's first workgroups."""
+    """The launch class of the batch-B, 9-head self-attention call on 256 CUs (the count without a device): the
+    units past the last whole round of 1024 are its tail, in 32-query groups or 64-query units (folded: past a
+    single round). The launch itself runs them with the others (test_plan_reports_the_flash_launch)."""
     plan = _lib.plan(big(B, Lq))
     assert plan.kernel == _lib.SA_KERNEL_FLASH and plan.name == b"flash_mfma_d64"
     assert plan.workgroups == B * 9 * ((Lq + 127) // 128) - tail_units

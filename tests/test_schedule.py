@@ -354,10 +354,10 @@ def test_schedule_follows_the_chosen_kernel():
     assert q.kernel == _lib.SA_KERNEL_FLASH_SMALL16 and q.order_n == 0
 
 
-@pytest.mark.parametrize("field", ["order_n", "tail_folded"])
+@pytest.mark.parametrize("field", ["order_n", "tail_folded", "flash_groups"])
 def test_plan_revision_1_and_2_are_accepted_and_not_overrun(field):
-    """A revision-1 sa_attn_plan (ending at tail_workgroups) or revision-2 one (ending at
-    sequence_order) still works; nothing past it is written."""
+    """A revision-1 sa_attn_plan (ending at tail_workgroups), revision-2 one (ending at
+    sequence_order) or revision-3 one (ending at tail_folded) still works; nothing past it is written."""
     v1 = getattr(_lib.AttnPlan, field).offset
     buf = (ctypes.c_uint8 * ctypes.sizeof(_lib.AttnPlan))(*([0xAB] * ctypes.sizeof(_lib.AttnPlan)))
     plan = _lib.AttnPlan.from_buffer(buf)
