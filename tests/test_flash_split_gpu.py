@@ -1,5 +1,6 @@
-"""Flash attention on the bf16 matrix cores (flash_split_kernel): every workgroup shape it is launched with, at
-ragged query and key lengths, each bias and mask, and values that have no three bfloat16 terms.
+"""Flash attention on the bf16 matrix cores (flash_split_kernel): every workgroup shape it is launched with
+(asserted), at ragged query and key lengths with each bias and mask, and values that have no three bfloat16
+terms, those of the D = 512 kernel too.
 
 Tolerance: scores and outputs are sums of six-term products whose dropped terms and roundings are below
 those of a float32 sum of the same length (2^-24 per addition); an error e in a score enters a
@@ -20,53 +21,92 @@ from supra_attn.runner import Staged
 pytestmark = pytest.mark.gpu
 
 BIAS = [_lib.SA_BIAS_NONE, _lib.SA_BIAS_DENSE, _lib.SA_BIAS_RELPOS]
-MASK = [_lib.SA_MASK_NONE, _lib.SA_MASK_KEY_LEN, _lib.SA_MASK_KEY_MASK]
+SCHEDULED = _lib.SA_MASK_VARIANT_KEY_LEN_SCHEDULED
+MASK = [_lib.SA_MASK_NONE, _lib.SA_MASK_KEY_LEN, _lib.SA_MASK_KEY_MASK, SCHEDULED]
 
-# 128-query units per CU (256 CUs): under half, at most one with over 8 key blocks, and more, per head dim;
-# query and key counts that end inside a group, a block and a step (1 key past one included)
-SHAPES = [(64, 5, 6, 333, 97), (64, 9, 5, 333, 289), (64, 12, 12, 130, 33), (64, 10, 11, 129, 321), (64, 20, 13, 131, 65),
-          (128, 3, 5, 200, 97), (128, 9, 9, 257, 161), (128, 22, 12, 150, 33)]
+# (groups, splits, stages) of the workgroups: (D, B, H, Lq, Lk) that take them on 256 CUs; query and key counts end inside
+# a group, a block and a step (1 key past one included)
+SHAPES = [
+    ((2, 2, 2), (64, 8, 4, 333, 97)), ((2, 2, 2), (64, 9, 4, 300, 225)),
+    ((2, 4, 1), (64, 8, 4, 333, 289)), ((2, 4, 1), (64, 9, 4, 300, 330)),
+    ((2, 2, 1), (64, 24, 12, 50, 97)), ((2, 2, 1), (64, 33, 9, 61, 193)),
+    ((4, 2, 2), (64, 9, 5, 333, 289)), ((4, 2, 2), (64, 10, 11, 129, 321)),
+    ((4, 1, 2), (64, 20, 13, 131, 65)), ((4, 1, 2), (64, 12, 12, 130, 33)), ((4, 1, 2), (64, 12, 12, 130, 31)),
+    ((2, 2, 1), (128, 8, 2, 200, 97)), ((2, 2, 1), (128, 9, 5, 100, 289)),
+    ((4, 1, 2), (128, 9, 9, 257, 161)), ((4, 1, 2), (128, 22, 12, 150, 31)),
+    ((4, 1, 1), (128, 16, 12, 200, 97)), ((4, 1, 1), (128, 11, 12, 257, 65)),
+]
 
 
-def run(dev, call):
-    print(f"[flash split] {call.name} bias={call.bias_mode} mask={call.mask_mode}", flush=True)
-    st = Staged(dev, call)
+def run(dev, call, shape=None, host=True):
+    st = Staged(dev, call, host_key_len=host)
     try:
-        assert st.kernel.startswith("flash_mfma")
-        return orc.output_view(st.run(), call)
+        p = _lib.plan(st.args)
+        took = (p.flash_groups, p.flash_splits, p.flash_stages)
+        print(f"[flash split] {call.name} bias={call.bias_mode} mask={p.mask_variant} shape={took} {p.flash_workgroups} workgroups", flush=True)
+        assert p.kernel == _lib.SA_KERNEL_FLASH and (shape is None or took == shape)
+        assert p.flash_workgroups == call.B * call.H * -(-call.Lq // (32 * took[0]))
+        return orc.output_view(st.run(), call), p
     finally:
         st.release()
 
 
 @pytest.mark.parametrize("mask", MASK)
 @pytest.mark.parametrize("bias", BIAS)
-@pytest.mark.parametrize("D,B,H,Lq,Lk", SHAPES)
-def test_shapes(dev, D, B, H, Lq, Lk, bias, mask):
+@pytest.mark.parametrize("shape,dims", SHAPES)
+def test_shapes(dev, shape, dims, bias, mask):
+    D, B, H, Lq, Lk = dims
+    if shape == (4, 1, 1) and bias != _lib.SA_BIAS_NONE:
+        shape = (4, 1, 2)  # not compiled with a bias
     lens = None
-    if mask == _lib.SA_MASK_KEY_LEN:  # none, one, a block and one more, all
-        lens = ([0, 1, 32, 33, Lk, Lk - 1] * B)[:B]
+    if mask in (_lib.SA_MASK_KEY_LEN, SCHEDULED):  # none, one, a block and one more, all
+        lens = ([0, 1, min(32, Lk), min(33, Lk), Lk, Lk - 1] * B)[:B]
     call = make_call(B, H, D, Lq, Lk, seed=B + Lq + Lk, packed=Lq == Lk, pad_cols=4, o_off=4, ldo_pad=8, bias_mode=bias,
-                     mask_mode=mask, key_len=lens, dense_bias_batched=B % 2 == 1)
-    e = orc.errors(run(dev, call), orc.reference_fp64(call))
+                     mask_mode=_lib.SA_MASK_KEY_LEN if mask == SCHEDULED else mask, key_len=lens, dense_bias_batched=B % 2 == 1)
+    got, plan = run(dev, call, shape, host=mask == SCHEDULED)
+    assert plan.mask_variant == mask or (Lk <= 32 and plan.mask_variant == _lib.SA_MASK_KEY_LEN)  # equal blocks: no order
+    e = orc.errors(got, orc.reference_fp64(call))
     assert e["finite"] and e["rel_l2"] <= 2e-6 and e["max_rel"] <= 1e-5, e
 
 
-@pytest.mark.parametrize("D,B,H,Lq,Lk", [(64, 9, 5, 333, 289), (64, 20, 13, 131, 65), (128, 9, 9, 257, 161)])
-def test_values_without_three_terms(dev, D, B, H, Lq, Lk):
+# key masks, key lengths and biases of the retry in fp32 products, on the shapes of every split
+RETRY = [((2, 4, 1), (64, 8, 4, 333, 289)), ((4, 2, 2), (64, 9, 5, 333, 289)), ((4, 1, 2), (64, 20, 13, 131, 65)),
+         ((2, 2, 1), (64, 24, 12, 50, 97)), ((4, 1, 2), (128, 9, 9, 257, 161)), ((2, 2, 1), (128, 8, 2, 200, 97)),
+         (None, (512, 5, 1, 100, 333)), (None, (512, 18, 1, 500, 300))]
+
+
+@pytest.mark.parametrize("mask", MASK[:3])
+@pytest.mark.parametrize("shape,dims,bias", [(s, d, b) for s, d in RETRY for b in (BIAS if s else BIAS[:2])])  # 512: no relpos
+def test_values_without_three_terms(dev, shape, dims, bias, mask):
     """Infinities and magnitudes that round past the bfloat16 range give what float32 products give: a key
-    whose scores are -inf drops out, a query or value that is not finite shows where it reaches."""
-    call = make_call(B, H, D, Lq, Lk, seed=3)
+    whose scores are -inf drops out, a query or value that is not finite shows where it reaches. With every bias
+    and mask (the special keys attended), at head dim 512 in one key chunk and in several that are merged."""
+    D, B, H, Lq, Lk = dims
+    lens = [Lk, Lk - 1, 40, Lk, 33] + [Lk] * (B - 5) if mask == _lib.SA_MASK_KEY_LEN else None
+    call = make_call(B, H, D, Lq, Lk, seed=3, bias_mode=bias, mask_mode=mask, key_len=lens)
+    if call.key_mask is not None:
+        call.key_mask[:, [0, 3, 5, 9]] = 1
     k = call.k.reshape(B, Lk, H, D)
     q = call.q.reshape(B, Lq, H, D)
     v = call.v.reshape(B, Lk, H, D)
-    q[0, :, 0] = np.abs(q[0, :, 0]) + 0.01
-    k[0, 5, 0, 3] = -np.inf              # scores -inf for every query of that head: as if masked
-    q[1, 7, 1, 2] = np.inf               # one query's row NaN
-    v[2, 9, 2, 1] = np.inf               # one output column of every query infinite
-    v[3, 3, 3, 4] = np.nan
-    k[4, 0, 4, 0] = np.float32(3.4e38)   # finite or infinite scores, by the query's sign
-    q[4, :, 4] = -np.abs(q[4, :, 4]) * np.float32(1e-38)
-    got = run(dev, call)
+    h = [i % H for i in range(5)]
+    q[0, :, h[0]] = np.abs(q[0, :, h[0]]) + 0.01
+    k[0, 5, h[0], 3] = -np.inf              # scores -inf for every query of that head: as if masked
+    q[1, 7, h[1], 2] = np.inf               # one query's row NaN
+    v[2, 9, h[2], 1] = np.inf               # one output column of every query infinite
+    v[3, 3, h[3], 4] = np.nan
+    k[4, 0, h[4], 0] = np.float32(3.4e38)   # finite or infinite scores, by the query's sign
+    q[4, :, h[4]] = -np.abs(q[4, :, h[4]]) * np.float32(1e-38)
+    if D == 512:
+        print(f"[wide split] {call.name} bias={bias} mask={mask}", flush=True)
+        st = Staged(dev, call)
+        try:
+            assert _lib.plan(st.args).kernel == _lib.SA_KERNEL_WIDE
+            got = orc.output_view(st.run(), call)
+        finally:
+            st.release()
+    else:
+        got, _ = run(dev, call, shape)
     ref = orc.reference_torch(call)
     np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
     np.testing.assert_array_equal(np.isposinf(got), np.isposinf(ref))
@@ -100,7 +140,7 @@ def test_large_dense_bias_is_rounded_once(dev, D, B, H, Lq, Lk):
     """score + log2(e) bias as one fma: with biases ~ N(0, 200^2) that rounding is the error of the call. A sum
     of a rounded product has sqrt(2) times as much; 1.15 lies between."""
     call = make_call(B, H, D, Lq, Lk, seed=11, bias_mode=_lib.SA_BIAS_DENSE, bias_std=200.0)
-    got = run(dev, call)
+    got, _ = run(dev, call)
     ref = orc.reference_fp64(call)
     log2e = np.float64(np.float32(1.4426950408889634))
     q, k, v = (x.reshape(B, L, H, D).transpose(0, 2, 1, 3).astype(np.float64) for x, L in ((call.q, Lq), (call.k, Lk), (call.v, Lk)))

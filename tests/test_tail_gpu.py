@@ -1,9 +1,7 @@
-"""GPU parity of flash launches whose last round holds few units: more units (128-query tiles) than
-the 4-per-CU kernel holds at once, with few enough left over for one workgroup per CU of the
-small-launch kernel (32-query groups) or of the 2-way key-split flash kernel (64-query units). The
-first launch covers the leading units; the rest go to a second launch, or, after a single round, run
-as 64-query units inside it, on its first workgroups after their own units. Every output row is
-checked against the PyTorch fp32 CPU path and the float64 brute force (1e-5)."""
+"""GPU parity of flash calls whose launch class has a tail: more units (128-query tiles) than four per
+CU, with few past the last whole round. One launch runs them all (two or three workgroups per CU); the
+class's figures are checked beside it. Every output row is checked against the PyTorch fp32 CPU path and
+the float64 brute force (1e-5)."""
 
 from __future__ import annotations
 
@@ -29,13 +27,13 @@ def tail_units(call) -> int:
 
 
 @pytest.mark.parametrize("B,Lq,Lk", [
-    (57, 256, 256),   # 1026 units: a tail of two (small-launch kernel)
-    (60, 256, 256),   # 1080 units: a tail of 56 (224 small workgroups)
+    (57, 256, 256),   # 1026 units: a tail of two
+    (60, 256, 256),   # 1080 units: a tail of 56 (224 groups)
     (60, 250, 250),   # ragged
     (57, 200, 230),   # 7 groups of 32 per (b, h): the tail starts inside a head
-    (64, 256, 256),   # the batch-64 DiT call: 128 left, 2-way key-split units folded into the round
-    (61, 200, 230),   # 74 left, folded split units, ragged 64-query units
-    (118, 256, 250),  # two rounds and 76 left: a second launch of the split kernel
+    (64, 256, 256),   # the batch-64 DiT call: 128 left, past a single round
+    (61, 200, 230),   # 74 left, ragged 64-query units
+    (118, 256, 250),  # two rounds and 76 left
 ])
 def test_tail_launch_parity(dev, B, Lq, Lk):
     call = make_call(B=B, H=9, D=64, Lq=Lq, Lk=Lk, seed=B * 7 + Lq, packed=(Lq == Lk), name=f"tail_B{B}_q{Lq}_k{Lk}")
@@ -44,6 +42,7 @@ def test_tail_launch_parity(dev, B, Lq, Lk):
     try:
         plan = _lib.plan(st.args)
         assert plan.kernel == _lib.SA_KERNEL_FLASH
+        assert plan.flash_workgroups == B * 9 * -(-Lq // (32 * plan.flash_groups))  # one grid
         n_tail = tail_units(call)
         assert n_tail > 0
         assert plan.workgroups == B * 9 * ((Lq + 127) // 128) - n_tail
@@ -69,9 +68,8 @@ def test_tail_launch_parity(dev, B, Lq, Lk):
 
 
 def _fold_draw(seed: int, n: int) -> list[dict]:
-    """Seeded calls whose units fill one round and part of a second that folds into it (more than 64
-    and at most 128 of them past the 1024 slots): any batch, head count and ragged lengths, packed or
-    separate q/k/v, padded rows and element offsets."""
+    """Seeded calls of 65 to 128 units past 1024 (a class whose tail is 64-query units past a single round): any
+    batch, head count and ragged lengths, packed or separate q/k/v, padded rows and element offsets."""
     rng = np.random.default_rng(seed)
     out = []
     while len(out) < n:

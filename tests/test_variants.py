@@ -1,5 +1,6 @@
-"""Host-only: the variant cases reach every compiled flash-kernel variant, each with at least two
-loop steps for every splitting wave and ragged query and key lengths (sa_attention_plan, no GPU)."""
+"""Host-only: the variant cases reach every variant that sa_attention_variant lists (compiled small-launch and
+wide variants, launch classes of the flash kernel), each with at least two loop steps for every splitting
+wave and ragged query and key lengths (sa_attention_plan, no GPU)."""
 
 from __future__ import annotations
 

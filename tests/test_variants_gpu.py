@@ -1,5 +1,5 @@
-"""GPU parity of every compiled flash and small-launch kernel variant <kernel, D, key_split, bias, mask>, each at a shape
-that real callers give it, with ragged lengths and at least two loop steps per splitting wave,
+"""GPU parity of every small-launch and wide kernel variant <kernel, D, key_split, bias, mask> and every launch
+class of the flash kernel (its compiled shapes: test_flash_split_gpu.py), each at a shape that real callers give it, with ragged lengths and at least two loop steps per splitting wave,
 against the PyTorch fp32 CPU path and the float64 brute force (both <= 1e-5, relative L2 and
 normwise max). The cases come from variant_cases.py; test_variants.py shows on the host that they
 reach every compiled variant."""

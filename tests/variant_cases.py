@@ -1,4 +1,4 @@
-"""One attention call per compiled flash-kernel and small-launch-kernel variant <kernel, D, key_split, bias, mask>.
+"""One attention call per launch class of the flash kernel and per small-launch-kernel variant <kernel, D, key_split, bias, mask>.
 
 Each call has the shape real callers give that variant (T5 batches with the relative-position
 bias, DiT-sized batches, head dim 128 with every bias and mask), ragged Lq and Lk (not multiples
