@@ -5,6 +5,8 @@
 #include <float.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace sa {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -16,6 +18,22 @@ constexpr float kLog2e = 1.4426950408889634f;
 // Running-max seed: finite, so that (m_old - m_new) is never (-inf) - (-inf) on rows whose keys
 // are all masked so far; exp2(-FLT_MAX - x) is 0 for any real x.
 constexpr float kMaxSeed = -FLT_MAX;
+
+__device__ __forceinline__ f32x16 zero16() {
+  f32x16 z;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) z[i] = 0.f;
+  return z;
+}
+
+// f(std::integral_constant<int, 0>{}) ... f(std::integral_constant<int, N - 1>{}), in order
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
 
 // Workgroups are handed to the 8 XCDs round-robin (workgroup i runs on XCD i % 8). Remap the
 // hardware index so that consecutive logical tiles (the query tiles of one head) run on one XCD

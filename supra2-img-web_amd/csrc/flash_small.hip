@@ -39,13 +39,6 @@ constexpr float kRescaleSlack = 8.f;  // log2 units: p stays <= 256 between resc
 constexpr int kD = 64;
 constexpr int kWaves = 4;
 
-__device__ __forceinline__ f32x16 zero16() {
-  f32x16 z;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) z[i] = 0.f;
-  return z;
-}
-
 // K rows of one block as loaded: kr[i] = chunk lane % 16 of key row 4i + lane / 16 (whole rows per
 // instruction); transposed through LDS into the MFMA layout when the block is consumed.
 struct KBlock {

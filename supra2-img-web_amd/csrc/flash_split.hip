@@ -37,17 +37,6 @@ struct FlashOrder {
 };
 struct NoOrder {};
 
-__device__ __forceinline__ f32x16 zero16() {
-  f32x16 z;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) z[i] = 0.f;
-  return z;
-}
-
-__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
 template <int D, int QG, int KS, int STAGES, int WPE, int BIAS, int MASK, typename Order>
 __global__ __launch_bounds__(64 * QG * KS, WPE) void flash_split_kernel(FlashArgs p, Order ord) {
   constexpr int NW = QG * KS;

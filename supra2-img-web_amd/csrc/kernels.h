@@ -185,14 +185,8 @@ struct LinearParams {
   float alpha;
   int act, epi;
 };
-struct LinearTile {
-  int wm, wn;  // 32x32 accumulators per wave along M and N (tile 64*wm x 64*wn)
-  int bk, ns;  // k-tile depth and LDS stages
-  int ksplit;  // k splits of linear_ksplit_kernel (4: 32 x 32 tiles, 2: 32 x 64 tiles), 0: linear_mfma_kernel
-};
-// MFMA kernel when K % 8 == 0 and x, W rows are 16-byte aligned; the generic kernel otherwise.
+// MFMA kernels when K % 8 == 0 and x, W rows are 16-byte aligned; the generic kernel otherwise.
 bool linear_mfma_supported(const LinearParams& p);
-LinearTile linear_mfma_tile(const LinearParams& p, int num_cus);
 const char* linear_kernel_name(const LinearParams& p, int num_cus);
 // The output tile that launch_linear runs p with, and the terms its operands are split into (1: fp32 products).
 void linear_tile(const LinearParams& p, int num_cus, int* rows, int* cols, int* terms);

@@ -8,24 +8,23 @@
 //
 // Three kernels: linear_split_kernel (large and medium grids, bf16 matrix cores, described there),
 // linear_mfma_kernel (fp32 MFMA, grids between those and the small ones) and linear_ksplit_kernel (small
-// grids, fp32 MFMA); split_tile and linear_mfma_tile choose. Any other alignment: linear_generic_kernel.
+// grids, fp32 MFMA); split_tile and linear_class choose. Any other alignment: linear_generic_kernel.
 //
 // Work decomposition of linear_mfma_kernel
-//   A workgroup is 4 wave64s in a 2 x 2 grid computing a BM x BN tile (BM = 64*WM, BN = 64*WN);
-//   each wave owns (32*WM) x (32*WN) outputs as WM x WN 32x32 accumulators of
-//   v_mfma_f32_32x32x2f32. The x rows are the MFMA A operand and the W rows the B operand, so
+//   A workgroup is 4 wave64s in a 2 x 2 grid computing a 64 x 64 tile; each wave owns 32 x 32 outputs, one
+//   accumulator of v_mfma_f32_32x32x2f32. The x rows are the MFMA A operand and the W rows the B operand, so
 //   lane l of an accumulator holds column n = l%32 and rows 8*(r/4) + 4*(l/32) + r%4 of register r:
 //   every store instruction writes 128 contiguous bytes of two rows.
-//   K advances in tiles of BK. Within a group of 8 consecutive k, half-wave h supplies
+//   K advances in tiles of 32. Within a group of 8 consecutive k, half-wave h supplies
 //   k = 8g + 4h + s at MFMA step s (s = 0..3): one b128 LDS read per operand row and group feeds
 //   four MFMAs, and every (x, W) pair of k meets exactly once.
 //
 // Tiles move HBM/L2 -> LDS with buffer_load_dwordx4 ... lds (no VGPR staging; scalar descriptor and
-// k offset, loop-invariant lane offsets), NS stages, one barrier per k-tile. The k-loop advances NS
+// k offset, loop-invariant lane offsets), two stages, one barrier per k-tile. The k-loop advances two
 // tiles at a time so every stage index is a compile-time constant: the steady-state loop issues
 // no VALU instruction, which on gfx950 would serialize with the MFMAs of the SIMD. LDS rows are
-// BK floats (BK/4 chunks of 16 bytes); chunk c of row r sits at c ^ ((r / RP) % (BK/4)) with
-// RP = 64/BK rows per 256 bytes, which makes the b128 operand reads of 16 consecutive rows
+// 32 floats (8 chunks of 16 bytes); chunk c of row r sits at c ^ ((r / 2) % 8) (two rows per 256
+// bytes), which makes the b128 operand reads of 16 consecutive rows
 // conflict-free (measured SQ_LDS_BANK_CONFLICT = 0). The operands of the next
 // group of 8 k are read from LDS while the MFMAs of the current group run, and the barrier of the
 // next k-tile sits before the last group's MFMAs.
@@ -56,13 +55,6 @@
 namespace sa {
 
 namespace {
-
-__device__ __forceinline__ f32x16 zero16() {
-  f32x16 z;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) z[i] = 0.f;
-  return z;
-}
 
 // Activations of app/gpu/gemm.js:21-36. The epilogue runs on the same SIMD datapath as the fp32
 // MFMAs, so the two logistic forms use one hardware exp2 and one reciprocal:
@@ -118,15 +110,6 @@ __device__ __forceinline__ void tile_coords(int t, const TileOrder& o, int& mi, 
   const int w = min(o.group_n, o.tiles_n - g * o.group_n);
   mi = sb * o.sb_rows + off / w;
   ni = g * o.group_n + off % w;
-}
-
-// f(std::integral_constant<int, 0>{}) ... f(std::integral_constant<int, N - 1>{}), in order
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(f);
-  }
 }
 
 // Waves per SIMD that the register budget of linear_split_kernel is set for (its VGPRs: 64 x 96 110,
@@ -420,26 +403,22 @@ __global__ __launch_bounds__(64 * NW, (split_waves_per_simd<NW, MT, NT>())) void
   }
 }
 
-// WM x WN accumulators per wave, BK k per tile (16 or 32), NS tiles in flight (LDS stages); the
+// 64 x 64 tiles, one 32 x 32 accumulator per wave, 32 k per tile, two tiles in flight (LDS stages); the
 // activation and the epilogue are compile-time, so the store loop has no per-element branches.
-template <int WM, int WN, int BK, int NS, int ACT, int EPI>
+template <int ACT, int EPI>
 __global__ __launch_bounds__(256, 2) void linear_mfma_kernel(LinArgs p, TileOrder order) {
-  constexpr int BM = 64 * WM;
-  constexpr int BN = 64 * WN;
+  constexpr int BM = 64, BN = 64, BK = 32;
   constexpr int CPR = BK / 4;            // 16-byte chunks per tile row
   constexpr int RP = 64 / BK;            // tile rows per 256 bytes (one pass over the 64 banks)
   constexpr int NG = BK / 8;             // groups of 8 k per tile
   constexpr int A_TILE = BM * BK;        // floats per stage
   constexpr int B_TILE = BN * BK;
   constexpr int STAGE = A_TILE + B_TILE;
-  constexpr int NIA = BM * CPR / 256;    // DMA instructions per wave and stage (64 chunks each)
-  constexpr int NIB = BN * CPR / 256;
-  constexpr int NI = NIA + NIB;
-  static_assert(NIA * 256 == BM * CPR && NIB * 256 == BN * CPR, "tiles must split into whole wave copies");
-  static_assert(NS == 2 || NS == 3, "two or three stages");
+  constexpr int NI = BM * CPR / 256;     // DMA instructions per wave, operand and stage (64 chunks each)
+  static_assert(NI * 256 == BM * CPR && BM == BN, "tiles must split into whole wave copies");
   static_assert(NG % 2 == 0, "an even number of groups per tile");
 
-  __shared__ __attribute__((aligned(16))) float lds[NS * STAGE];
+  __shared__ __attribute__((aligned(16))) float lds[2 * STAGE];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -453,7 +432,6 @@ __global__ __launch_bounds__(256, 2) void linear_mfma_kernel(LinArgs p, TileOrde
   tile_coords(xcd_remap(blockIdx.x, order.tiles_m * order.tiles_n), order, mi, ni);
   const int m0 = mi * BM;
   const int n0 = ni * BN;
-
   const float* xbase = p.x + (int64_t)m0 * p.ldx;
   const float* wbase = p.w + (int64_t)n0 * p.ldw;
   const int mlast = min(BM, p.M - m0) - 1;  // last valid tile row
@@ -462,22 +440,15 @@ __global__ __launch_bounds__(256, 2) void linear_mfma_kernel(LinArgs p, TileOrde
   // Per-lane byte offsets (from the tile's first row at k = 0) of this lane's 16-byte chunk in
   // each DMA instruction: instruction n of wave w fills physical chunks (n*4 + w)*64 + lane; the
   // chunk c of row r sits at physical chunk c ^ ((r / RP) % CPR).
-  unsigned aoff[NIA], boff[NIB];
-  int acol[NIA], bcol[NIB];  // logical column (floats) of the chunk, for the clamped k-tile
+  unsigned aoff[NI], boff[NI];
+  int kcol[NI];  // logical column (floats) of the chunk, for the clamped k-tile
 #pragma unroll
-  for (int n = 0; n < NIA; ++n) {
+  for (int n = 0; n < NI; ++n) {
     const int pc_all = (n * 4 + wave) * 64 + lane;
     const int row = pc_all / CPR;
     const int c = (pc_all % CPR) ^ ((row / RP) % CPR);
-    acol[n] = 4 * c;
+    kcol[n] = 4 * c;
     aoff[n] = 4u * (unsigned)(min(row, mlast) * (int)p.ldx + 4 * c);
-  }
-#pragma unroll
-  for (int n = 0; n < NIB; ++n) {
-    const int pc_all = (n * 4 + wave) * 64 + lane;
-    const int row = pc_all / CPR;
-    const int c = (pc_all % CPR) ^ ((row / RP) % CPR);
-    bcol[n] = 4 * c;
     boff[n] = 4u * (unsigned)(min(row, nlast) * (int)p.ldw + 4 * c);
   }
 
@@ -490,81 +461,58 @@ __global__ __launch_bounds__(256, 2) void linear_mfma_kernel(LinArgs p, TileOrde
   const int nkt = (p.K + BK - 1) / BK;
   const int nfull = p.K / BK;  // whole k-tiles; with K % BK != 0 the last tile (nfull) holds K
   // Copies of k-tile kt into LDS stage S. The stage is a compile-time constant (the main loop
-  // advances NS tiles at a time), so every LDS address below is a constant offset.
+  // advances two tiles at a time), so every LDS address below is a constant offset.
   auto issue = [&](int kt, auto stage) {
     constexpr int S = decltype(stage)::value;
     float* at = lds + S * STAGE;
     float* bt = at + A_TILE;
-    if (kt < nfull) {
-      const unsigned soff = 4u * (unsigned)(kt * BK);
+    // the tile holding K (always tile nfull, so its offsets are loop-invariant): columns at or
+    // past K re-read the last group (never multiplied)
+    const bool last = kt >= nfull;
+    const int k0 = last ? nfull * BK : kt * BK;
+    const unsigned soff = 4u * (unsigned)k0;
+    const int kmax = p.K - 8 - k0;
+    unsigned back[NI];  // whole groups back
 #pragma unroll
-      for (int n = 0; n < NIA; ++n) buffer_to_lds16(xr, aoff[n], at + (n * 4 + wave) * 256, soff);
+    for (int n = 0; n < NI; ++n) back[n] = last && kcol[n] > kmax + 4 ? 4u * (unsigned)((kcol[n] & ~7) - kmax) : 0u;
 #pragma unroll
-      for (int n = 0; n < NIB; ++n) buffer_to_lds16(wr, boff[n], bt + (n * 4 + wave) * 256, soff);
-    } else {
-      // the tile holding K (always tile nfull, so its offsets are loop-invariant): columns at or
-      // past K re-read the last group (never multiplied)
-      const int k0 = nfull * BK;
-      const unsigned soff = 4u * (unsigned)k0;
-      const int kmax = p.K - 8 - k0;
+    for (int n = 0; n < NI; ++n) buffer_to_lds16(xr, aoff[n] - back[n], at + (n * 4 + wave) * 256, soff);
 #pragma unroll
-      for (int n = 0; n < NIA; ++n) {
-        const int shift = acol[n] > kmax + 4 ? (acol[n] & ~7) - kmax : 0;  // whole groups back
-        buffer_to_lds16(xr, aoff[n] - 4u * (unsigned)shift, at + (n * 4 + wave) * 256, soff);
-      }
-#pragma unroll
-      for (int n = 0; n < NIB; ++n) {
-        const int shift = bcol[n] > kmax + 4 ? (bcol[n] & ~7) - kmax : 0;
-        buffer_to_lds16(wr, boff[n] - 4u * (unsigned)shift, bt + (n * 4 + wave) * 256, soff);
-      }
-    }
+    for (int n = 0; n < NI; ++n) buffer_to_lds16(wr, boff[n] - back[n], bt + (n * 4 + wave) * 256, soff);
   };
 
-  f32x16 acc[WM][WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int j = 0; j < WN; ++j) acc[i][j] = zero16();
+  f32x16 acc = zero16();
 
-  // LDS read offsets (floats) of this lane's operand chunk in group g: row (32*i + col) of the
-  // wave's block, logical chunk 2g + half; the swizzle depends on the row only through col
+  // LDS read offsets (floats) of this lane's operand chunk in group g: row `col` of the
+  // wave's block, logical chunk 2g + half
   const int swz = (col / RP) % CPR;
   int goff[NG];
 #pragma unroll
   for (int g = 0; g < NG; ++g) goff[g] = col * BK + 4 * ((2 * g + half) ^ swz);
-  const int arow0 = wm * 32 * WM * BK;  // wave's first A row, in floats
-  const int brow0 = wn * 32 * WN * BK;
+  const int arow0 = wm * 32 * BK;  // wave's first A row, in floats
+  const int brow0 = wn * 32 * BK;
 
   // Operands of one group in registers, double-buffered: group g + 1 (or group 0 of the next
   // tile) is read from LDS while the MFMAs of group g run.
-  f32x4 ra[2][WM], rb[2][WN];
+  f32x4 ra[2], rb[2];
   auto read_group = [&](auto stage, int g, int slot) {
     constexpr int S = decltype(stage)::value;
-    const float* at = lds + S * STAGE + arow0 + goff[g];
-    const float* bt = lds + S * STAGE + A_TILE + brow0 + goff[g];
-#pragma unroll
-    for (int i = 0; i < WM; ++i) ra[slot][i] = *reinterpret_cast<const f32x4*>(at + i * 32 * BK);
-#pragma unroll
-    for (int j = 0; j < WN; ++j) rb[slot][j] = *reinterpret_cast<const f32x4*>(bt + j * 32 * BK);
+    ra[slot] = *reinterpret_cast<const f32x4*>(lds + S * STAGE + arow0 + goff[g]);
+    rb[slot] = *reinterpret_cast<const f32x4*>(lds + S * STAGE + A_TILE + brow0 + goff[g]);
   };
-  // tile kt (in stage S) has landed for this thread (the younger tiles may still be in flight);
-  // the barrier makes it whole and guarantees every wave has read the stage the next copies
-  // overwrite: tile kt + NS - 1 goes to stage (S + NS - 1) % NS, the one tile kt - 1 used
+  // tile kt (in stage S) has landed for this thread; the barrier makes it whole and guarantees every wave has
+  // read the stage the next copies overwrite: tile kt + 1 goes to stage S ^ 1, the one tile kt - 1 used
   auto sync_tile = [&](int kt, auto stage) {
     constexpr int S = decltype(stage)::value;
-    if (NS == 3 && kt + 1 < nkt) {
-      wait_vmcnt<(NS == 3 ? NI : 0)>();
-    } else {
-      wait_vmcnt<0>();
-    }
+    wait_vmcnt<0>();
     __syncthreads();
-    if (kt + NS - 1 < nkt) issue(kt + NS - 1, std::integral_constant<int, (S + NS - 1) % NS>{});
+    if (kt + 1 < nkt) issue(kt + 1, std::integral_constant<int, S ^ 1>{});
   };
   // the MFMAs of tile kt (stage S); the operands of group g + 1, or of the next tile's group 0,
   // are read while those of group g are multiplied
   auto step = [&](int kt, auto stage) {
     constexpr int S = decltype(stage)::value;
-    constexpr int S1 = (S + 1) % NS;
+    using Next = std::integral_constant<int, S ^ 1>;
     const int ng = kt < nfull ? NG : (p.K - nfull * BK) >> 3;  // valid groups of 8 k in this tile
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
@@ -572,85 +520,67 @@ __global__ __launch_bounds__(256, 2) void linear_mfma_kernel(LinArgs p, TileOrde
       if (g + 1 < NG) {
         read_group(stage, g + 1, cur ^ 1);
       } else if (kt + 1 < nkt) {
-        sync_tile(kt + 1, std::integral_constant<int, S1>{});
-        read_group(std::integral_constant<int, S1>{}, 0, cur ^ 1);
+        sync_tile(kt + 1, Next{});
+        read_group(Next{}, 0, cur ^ 1);
       }
       if (g < ng) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[cur][i][s], rb[cur][j][s], acc[i][j], 0, 0, 0);
+        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[cur][s], rb[cur][s], acc, 0, 0, 0);
       }
     }
   };
   using S0 = std::integral_constant<int, 0>;
-  using S1c = std::integral_constant<int, 1>;
-  using S2c = std::integral_constant<int, 2 % NS>;
+  using S1 = std::integral_constant<int, 1>;
 
   issue(0, S0{});  // tile 0 (a tile always exists: K >= 8)
-  if (NS == 3 && nkt > 1) issue(1, S1c{});
   sync_tile(0, S0{});
   read_group(S0{}, 0, 0);
   int kt = 0;
-  for (; kt + NS <= nkt; kt += NS) {  // tile kt + u sits in stage u
+  for (; kt + 2 <= nkt; kt += 2) {
     step(kt, S0{});
-    step(kt + 1, S1c{});
-    if constexpr (NS == 3) step(kt + 2, S2c{});
+    step(kt + 1, S1{});
   }
   if (kt < nkt) step(kt, S0{});
-  if (NS == 3 && kt + 1 < nkt) step(kt + 1, S1c{});
 
-  // ---- epilogue: lane holds column n = nw + 32j + col, rows mw + 32i + 8(r/4) + 4*half + r%4.
+  // ---- epilogue: lane holds column n = nw + col, rows mw + 8(r/4) + 4*half + r%4.
   // Buffer loads/stores over the wave's output block: a scalar descriptor, a 32-bit per-lane
   // offset and a scalar per-row offset (no 64-bit address arithmetic per element); whole tiles
   // skip the bounds checks.
-  const int mw = m0 + wm * 32 * WM;
-  const int nw = n0 + wn * 32 * WN;
+  const int mw = m0 + wm * 32;
+  const int nw = n0 + wn * 32;
   const bool full = m0 + BM <= p.M && n0 + BN <= p.N;
   const __amdgpu_buffer_rsrc_t yr =
       __builtin_amdgcn_make_buffer_rsrc(p.y + (int64_t)mw * p.ldy + nw, 0, 0x7fffffff, 0x00020000);
-  const float* rsrc_base = p.resid + (int64_t)mw * p.ldy + nw;  // residual rows
-  const __amdgpu_buffer_rsrc_t rr_ = buffer_rsrc(rsrc_base);
+  const __amdgpu_buffer_rsrc_t rr_ = buffer_rsrc(p.resid + (int64_t)mw * p.ldy + nw);  // residual rows
   const int ldy4 = 4 * (int)p.ldy;
   // Plain stores are non-temporal (cache policy NT): y is not read back here, and keeping it out of
-  // the L2 leaves the W panels and x rows there (measured on the 16384-row qkv layer: 1.55x fewer L2
-  // fetches). The residual epilogues keep the default policy: there NT cost 3.5% (proj, cproj).
+  // the L2 leaves the W panels and x rows there. The residual epilogues keep the default policy.
   constexpr int kStoreCpol = EPI == LIN_EPI_STORE ? 2 : 0;
   auto store = [&](auto check) {
     constexpr bool kCheck = decltype(check)::value;
+    const bool n_ok = !kCheck || nw + col < p.N;
+    const float bias_n = (p.bias && n_ok) ? p.bias[nw + col] : 0.f;
+    float gate_n = 1.f;
+    if constexpr (EPI == LIN_EPI_RESID_GATE) gate_n = n_ok ? p.gate[nw + col] : 0.f;
+    const int voff = 4 * half * ldy4 + 4 * col;
+    // residual epilogues: the 16 old values of the block are loaded together, then combined
+    float old[16];
+    if constexpr (EPI != LIN_EPI_STORE) {
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const int nl = 32 * j + col;
-      const bool n_ok = !kCheck || nw + nl < p.N;
-      const float bias_n = (p.bias && n_ok) ? p.bias[nw + nl] : 0.f;
-      float gate_n = 1.f;
-      if constexpr (EPI == LIN_EPI_RESID_GATE) gate_n = n_ok ? p.gate[nw + nl] : 0.f;
+      for (int r = 0; r < 16; ++r) {
+        const int rr = 8 * (r >> 2) + (r & 3);
+        old[r] = 0.f;
+        if (!kCheck || (n_ok && mw + 4 * half + rr < p.M))
+          old[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rr_, voff, rr * ldy4, 0));
+      }
+    }
 #pragma unroll
-      for (int i = 0; i < WM; ++i) {
-        const int voff = (32 * i + 4 * half) * ldy4 + 4 * nl;
-        // residual epilogues: the 16 old values of the block are loaded together, then combined
-        float old[16];
-        if constexpr (EPI != LIN_EPI_STORE) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int rr = 8 * (r >> 2) + (r & 3);
-            old[r] = 0.f;
-            if (!kCheck || (n_ok && mw + 32 * i + 4 * half + rr < p.M))
-              old[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rr_, voff, rr * ldy4, 0));
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int rr = 8 * (r >> 2) + (r & 3);
-          if (!kCheck || (n_ok && mw + 32 * i + 4 * half + rr < p.M)) {
-            float v = apply_act<ACT>(fmaf(acc[i][j][r], p.alpha, bias_n));
-            if constexpr (EPI != LIN_EPI_STORE) v = fmaf(gate_n, v, old[r]);
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), yr, voff, rr * ldy4, kStoreCpol);
-          }
-        }
+    for (int r = 0; r < 16; ++r) {
+      const int rr = 8 * (r >> 2) + (r & 3);
+      if (!kCheck || (n_ok && mw + 4 * half + rr < p.M)) {
+        float v = apply_act<ACT>(fmaf(acc[r], p.alpha, bias_n));
+        if constexpr (EPI != LIN_EPI_STORE) v = fmaf(gate_n, v, old[r]);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), yr, voff, rr * ldy4, kStoreCpol);
       }
     }
   };
@@ -893,22 +823,22 @@ LinArgs lin_args(const LinearParams& p) {
   return a;
 }
 
-template <int WM, int WN, int BK, int NS, int ACT, int EPI>
+template <int ACT, int EPI>
 hipError_t launch_tiles(const LinearParams& p, hipStream_t stream) {
-  const int64_t tm = (p.M + 64 * WM - 1) / (64 * WM);
-  const int64_t tn = (p.N + 64 * WN - 1) / (64 * WN);
+  const int64_t tm = (p.M + 63) / 64;
+  const int64_t tn = (p.N + 63) / 64;
   if (tm * tn > 0x7fffffff) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((linear_mfma_kernel<WM, WN, BK, NS, ACT, EPI>), dim3((unsigned)(tm * tn)), dim3(256), 0, stream,
-                     lin_args(p), tile_order(p, 64 * WM, 64 * WN));
+  hipLaunchKernelGGL((linear_mfma_kernel<ACT, EPI>), dim3((unsigned)(tm * tn)), dim3(256), 0, stream, lin_args(p),
+                     tile_order(p, 64, 64));
   return hipGetLastError();
 }
 
-template <int WM, int WN, int BK, int NS, int ACT>
+template <int ACT>
 hipError_t launch_epi(const LinearParams& p, hipStream_t stream) {
   switch (p.epi) {
-    case LIN_EPI_STORE: return launch_tiles<WM, WN, BK, NS, ACT, LIN_EPI_STORE>(p, stream);
-    case LIN_EPI_RESID: return launch_tiles<WM, WN, BK, NS, ACT, LIN_EPI_RESID>(p, stream);
-    case LIN_EPI_RESID_GATE: return launch_tiles<WM, WN, BK, NS, ACT, LIN_EPI_RESID_GATE>(p, stream);
+    case LIN_EPI_STORE: return launch_tiles<ACT, LIN_EPI_STORE>(p, stream);
+    case LIN_EPI_RESID: return launch_tiles<ACT, LIN_EPI_RESID>(p, stream);
+    case LIN_EPI_RESID_GATE: return launch_tiles<ACT, LIN_EPI_RESID_GATE>(p, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -979,13 +909,12 @@ hipError_t launch_ksplit(const LinearParams& p, hipStream_t stream) {
   }
 }
 
-template <int WM, int WN, int BK, int NS>
 hipError_t launch_act(const LinearParams& p, hipStream_t stream) {
   switch (p.act) {
-    case LIN_ACT_NONE: return launch_epi<WM, WN, BK, NS, LIN_ACT_NONE>(p, stream);
-    case LIN_ACT_GELU: return launch_epi<WM, WN, BK, NS, LIN_ACT_GELU>(p, stream);
-    case LIN_ACT_GELU_TANH: return launch_epi<WM, WN, BK, NS, LIN_ACT_GELU_TANH>(p, stream);
-    case LIN_ACT_SILU: return launch_epi<WM, WN, BK, NS, LIN_ACT_SILU>(p, stream);
+    case LIN_ACT_NONE: return launch_epi<LIN_ACT_NONE>(p, stream);
+    case LIN_ACT_GELU: return launch_epi<LIN_ACT_GELU>(p, stream);
+    case LIN_ACT_GELU_TANH: return launch_epi<LIN_ACT_GELU_TANH>(p, stream);
+    case LIN_ACT_SILU: return launch_epi<LIN_ACT_SILU>(p, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1016,18 +945,19 @@ bool linear_mfma_supported(const LinearParams& p) {
 // splits 18.9-19.4). The split kernel's smallest tiles (64 x 48, 32 x 48) measured slower on the small grids:
 // 13-20 against 6-15 us at K = 576, with one, two or four k-tiles of loads in flight alike: a wave alone
 // on its SIMD issues one VALU instruction per 6 cycles, and the splits are most of its work.
-LinearTile linear_mfma_tile(const LinearParams& p, int num_cus) {
+namespace {
+
+enum LinearClass { kClass128x192, kClass64x192, kClass64x64, kClass32x64, kClass32x32 };
+LinearClass linear_class(const LinearParams& p, int num_cus) {
   const int64_t tiles_wide = ((p.M + 127) / 128) * ((p.N + 191) / 192);
   const int64_t tiles_tall = ((p.M + 63) / 64) * ((p.N + 191) / 192);
   const int64_t tiles_64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
-  if (p.N >= 2048 && tiles_wide >= num_cus) return {2, 3, 32, 2, 0};
-  if ((p.N % 192 == 0 || p.N >= 1024) && tiles_tall >= 3 * (int64_t)num_cus) return {1, 3, 16, 3, 0};
-  if (4 * tiles_64 < 5 * (int64_t)num_cus) return {1, 1, 64, 2, 4};
-  if (tiles_64 < 2 * (int64_t)num_cus) return {1, 2, 64, 2, 2};
-  return {1, 1, 32, 2, 0};
+  if (p.N >= 2048 && tiles_wide >= num_cus) return kClass128x192;
+  if ((p.N % 192 == 0 || p.N >= 1024) && tiles_tall >= 3 * (int64_t)num_cus) return kClass64x192;
+  if (4 * tiles_64 < 5 * (int64_t)num_cus) return kClass32x32;
+  if (tiles_64 < 2 * (int64_t)num_cus) return kClass32x64;
+  return kClass64x64;
 }
-
-namespace {
 
 // The tile that linear_split_kernel runs a call of the larger classes with, or one of the fp32 kernels:
 // kMfma64 (linear_mfma_kernel, 64 x 64) in its class, kKsplit32x64 in its own. Each candidate's time is
@@ -1040,7 +970,7 @@ namespace {
 // two-split fp32 kernel takes only the 64 x 64 split tile beside it, whose two sums per output are more
 // exact than its two halves of k.
 enum SplitTile { kMfma64, kKsplit32x64, kSplit64x64, kSplit64x96, kSplit128x96, kSplit256x144, kSplit256x192 };
-SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) {
+SplitTile split_tile(const LinearParams& p, int num_cus, LinearClass cls) {
   struct Line {
     double a, b;
   };
@@ -1072,7 +1002,7 @@ SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) 
       t = tile;
     }
   };
-  if (cls.ksplit == 2) {  // three or four 32 x 64 tiles per CU
+  if (cls == kClass32x64) {  // three or four 32 x 64 tiles per CU
     take((per_cu(32, 64) <= 3 ? 4.4 + 14.6 * u : 5.2 + 20.6 * u) + 0.85 * resid, kKsplit32x64);
     return t;
   }
@@ -1080,7 +1010,7 @@ SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) 
   take(cost(128, 96, k128x96, 0.65), kSplit128x96);
   take(cost(256, 144, k256x144, 1.05), kSplit256x144);
   take(cost(256, 192, k256x192, 1.05), kSplit256x192);
-  if (cls.wn == 1) take(1.07 * (3.4 + per_cu(64, 64) * (0.4 + 8.45 * u) + 0.2 * resid), kMfma64);
+  if (cls == kClass64x64) take(1.07 * (3.4 + per_cu(64, 64) * (0.4 + 8.45 * u) + 0.2 * resid), kMfma64);
   return t;
 }
 
@@ -1088,12 +1018,13 @@ SplitTile split_tile(const LinearParams& p, int num_cus, const LinearTile& cls) 
 
 const char* linear_kernel_name(const LinearParams& p, int num_cus) {
   if (!linear_mfma_supported(p)) return "linear_generic";
-  const LinearTile t = linear_mfma_tile(p, num_cus);
-  if (t.ksplit == 4) return "linear_mfma_32x32_ksplit";
-  if (t.ksplit == 2) return "linear_mfma_32x64_ksplit";
-  if (t.wm == 2) return "linear_mfma_128x192";
-  if (t.wn == 3) return "linear_mfma_64x192";
-  return "linear_mfma_64x64";
+  switch (linear_class(p, num_cus)) {
+    case kClass128x192: return "linear_mfma_128x192";
+    case kClass64x192: return "linear_mfma_64x192";
+    case kClass32x64: return "linear_mfma_32x64_ksplit";
+    case kClass32x32: return "linear_mfma_32x32_ksplit";
+    default: return "linear_mfma_64x64";
+  }
 }
 
 void linear_tile(const LinearParams& p, int num_cus, int* rows, int* cols, int* terms) {
@@ -1103,8 +1034,8 @@ void linear_tile(const LinearParams& p, int num_cus, int* rows, int* cols, int* 
   static constexpr Tile kTiles[] = {{64, 64, 1}, {32, 64, 1}, {64, 64, 3}, {64, 96, 3}, {128, 96, 3}, {256, 144, 3}, {256, 192, 3}};
   Tile t = {16, 16, 1};  // linear_generic_kernel
   if (linear_mfma_supported(p)) {
-    const LinearTile cls = linear_mfma_tile(p, num_cus);
-    t = cls.ksplit == 4 ? Tile{32, 32, 1} : kTiles[split_tile(p, num_cus, cls)];
+    const LinearClass cls = linear_class(p, num_cus);
+    t = cls == kClass32x32 ? Tile{32, 32, 1} : kTiles[split_tile(p, num_cus, cls)];
   }
   *rows = t.rows;
   *cols = t.cols;
@@ -1118,16 +1049,16 @@ hipError_t launch_linear(const LinearParams& p, int num_cus, hipStream_t stream)
     hipLaunchKernelGGL(linear_generic_kernel, grid, dim3(256), 0, stream, p);
     return hipGetLastError();
   }
-  const LinearTile t = linear_mfma_tile(p, num_cus);
-  if (t.ksplit == 4) return launch_ksplit<1, 1, 4>(p, stream);
-  switch (split_tile(p, num_cus, t)) {
+  const LinearClass cls = linear_class(p, num_cus);
+  if (cls == kClass32x32) return launch_ksplit<1, 1, 4>(p, stream);
+  switch (split_tile(p, num_cus, cls)) {
     case kKsplit32x64: return launch_ksplit<1, 2, 2>(p, stream);
     case kSplit64x64: return launch_split<4, 1, 4>(p, stream);
     case kSplit64x96: return launch_split<4, 1, 6>(p, stream);
     case kSplit128x96: return launch_split<4, 2, 6>(p, stream);
     case kSplit256x144: return launch_split<8, 2, 9>(p, stream);
     case kSplit256x192: return launch_split<8, 2, 12>(p, stream);
-    default: return launch_act<1, 1, 32, 2>(p, stream);
+    default: return launch_act(p, stream);
   }
 }
 

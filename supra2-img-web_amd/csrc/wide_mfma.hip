@@ -34,16 +34,6 @@ namespace {
 
 constexpr float kRescaleSlack = 8.f;
 
-// f(std::integral_constant<int, 0>{}) ... f(std::integral_constant<int, N - 1>{}), in order
-template <typename F, int... Is>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>) {
-  (f(std::integral_constant<int, Is>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 // Asks the scheduler for N times one MFMA and V VALU instructions, in turn.
 template <int N, int V>
 __device__ __forceinline__ void mix() {
@@ -51,17 +41,6 @@ __device__ __forceinline__ void mix() {
     __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
     __builtin_amdgcn_sched_group_barrier(0x2, V, 0);
   });
-}
-
-__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ f32x16 zero16() {
-  f32x16 z;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) z[i] = 0.f;
-  return z;
 }
 
 // Arguments of the attention kernels, packed into 112 bytes (launches start about 0.8 us sooner
@@ -169,8 +148,9 @@ struct BlockTerms {
   }
 };
 
-template <int D, int NW, int BIAS, int MASK>
-__global__ __launch_bounds__(64 * NW, 1) void wide_mfma_kernel(WideArgs p) {
+template <int BIAS, int MASK>
+__global__ __launch_bounds__(256, 1) void wide_mfma_kernel(WideArgs p) {
+  constexpr int D = 256, NW = 4;
   constexpr int DS = D / NW;      // head dims per wave
   constexpr int QREG = DS / 2;    // Q values per lane
   constexpr int NDB = DS / 32;    // 32-dim output tiles per wave
@@ -310,24 +290,11 @@ __global__ __launch_bounds__(64 * NW, 1) void wide_mfma_kernel(WideArgs p) {
     // barrier every wave reads the summed tile from partial 0.
     {
       float* ldsf = reinterpret_cast<float*>(lds_s);
-      constexpr int PER_LANE = 1024 / NW / 64;  // floats of the tile each lane sums
-      const int e0 = wave * (1024 / NW) + lane * PER_LANE;
-      if constexpr (PER_LANE == 4) {
-        f32x4 a = *reinterpret_cast<const f32x4*>(ldsf + e0);
+      const int e0 = wave * (1024 / NW) + lane * 4;  // four floats of the tile per lane
+      f32x4 a = *reinterpret_cast<const f32x4*>(ldsf + e0);
 #pragma unroll
-        for (int ww = 1; ww < NW; ++ww) a += *reinterpret_cast<const f32x4*>(ldsf + ww * 1024 + e0);
-        *reinterpret_cast<f32x4*>(ldsf + e0) = a;
-      } else {
-        static_assert(PER_LANE == 2, "4 or 8 waves");
-        float2 a = *reinterpret_cast<const float2*>(ldsf + e0);
-#pragma unroll
-        for (int ww = 1; ww < NW; ++ww) {
-          const float2 b = *reinterpret_cast<const float2*>(ldsf + ww * 1024 + e0);
-          a.x += b.x;
-          a.y += b.y;
-        }
-        *reinterpret_cast<float2*>(ldsf + e0) = a;
-      }
+      for (int ww = 1; ww < NW; ++ww) a += *reinterpret_cast<const f32x4*>(ldsf + ww * 1024 + e0);
+      *reinterpret_cast<f32x4*>(ldsf + e0) = a;
     }
     __syncthreads();
     float u[16];
@@ -910,18 +877,12 @@ __global__ __launch_bounds__(256) void wide_merge_kernel(MergeArgs p) {
   *reinterpret_cast<f32x4*>(p.o + (int64_t)b * p.so + (int64_t)qi * p.ldo + h * D + 4 * d4) = y;
 }
 
-// Waves per workgroup of the head-dim-split kernel (D = 256): each owns D / 4 head dims, 80 KiB of
-// LDS, two workgroups per CU. (At D = 512 it ran 8 waves, two per SIMD, in 160 KiB: VAE call
-// 34.9 us against 29.9 for whole score tiles per wave, as wide_split_kernel has them.)
-template <int D>
-constexpr int kWideWaves = 4;
-
 template <int D, int BIAS, int MASK>
 void launch_main(const WideArgs& a, dim3 grid, hipStream_t stream) {
   if constexpr (D == 512)
     hipLaunchKernelGGL((wide_split_kernel<BIAS, MASK>), grid, dim3(512), 0, stream, a);
   else
-    hipLaunchKernelGGL((wide_mfma_kernel<D, kWideWaves<D>, BIAS, MASK>), grid, dim3(64 * kWideWaves<D>), 0, stream, a);
+    hipLaunchKernelGGL((wide_mfma_kernel<BIAS, MASK>), grid, dim3(256), 0, stream, a);
 }
 
 template <int D, int BIAS>
