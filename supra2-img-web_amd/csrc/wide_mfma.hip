@@ -419,7 +419,7 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
   constexpr int DS = D / 8;          // output head dims per wave
   constexpr int NS = D / 64;         // product steps of a quarter of the head dims
   constexpr int REC = 32 * D + 64;   // workspace floats per partial: O [32][D], m [32], l [32]
-  constexpr int KR = 3;              // product steps whose K loads are in flight
+  constexpr int KR = BIAS == BIAS_NONE ? 3 : 2;  // product steps whose K loads are in flight (three do not fit beside a bias)
 
   __shared__ u32x4 lds_q[D / 16 * 3 * 64];  // [product step][term][half][query ^ chunk], then the output
   __shared__ u32x4 lds_p[8 * 3 * 2 * 64];   // probability terms [16 keys][term][lane] (8 * 3 * 64); before that
@@ -604,8 +604,13 @@ __global__ __launch_bounds__(512, 2) void wide_split_kernel(WideArgs p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) w[r] = u[r & 7];
       terms.apply(w);
+      // (opaque: a choice between two loads of w would become one at a run-time index, and w memory)
 #pragma unroll
-      for (int r = 0; r < 8; ++r) u[r] = sub ? w[8 + r] : w[r];
+      for (int r = 0; r < 8; ++r) {
+        float lo = w[r], hi = w[8 + r];
+        asm("" : "+v"(lo), "+v"(hi));
+        u[r] = sub ? hi : lo;
+      }
     }
     if (kb0 + 32 > kend) {
 #pragma unroll
