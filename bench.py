@@ -49,7 +49,20 @@ for _p in (ROOT, PKG):
 
 METRIC = "fused-attn µs/call + TFLOP/s (DiT 2×9×256×64 fp32), % of fp32 MFMA peak"
 PEAK_TFLOPS = 157.3  # MI355X dense fp32 MFMA
+PEAK_SPLIT_TFLOPS = 2500 / 6  # dense bf16 MFMA, float32 products of three-term operands taking six each
 PEAK_HBM_GBS = 8000.0
+
+
+def unit_peak(args) -> float:
+    """The peak, in float32 products, of the matrix unit that runs an attention or linear call: three-term bf16
+    products (flash and D = 512 attention, split linear tiles) or fp32 MFMA."""
+    from supra_attn import _lib
+
+    if isinstance(args, _lib.LinearArgs):
+        return PEAK_SPLIT_TFLOPS if _lib.linear_tile(args)[2] == 3 else PEAK_TFLOPS
+    p = _lib.plan(args)
+    split = p.kernel == _lib.SA_KERNEL_FLASH or (p.kernel == _lib.SA_KERNEL_WIDE and p.head_dim == 512)
+    return PEAK_SPLIT_TFLOPS if split else PEAK_TFLOPS
 
 
 def log(msg: str) -> None:
@@ -251,6 +264,7 @@ def linear_block(dev, B: int = 64, reps: int = 20, cpu: bool = True) -> dict:
     """The six linears of one DiT block at batch B (app/models/dit.js:167-193: qkv, proj, q, cproj,
     fc1, fc2 at B*256 rows) through sa_linear_f32: per-layer us, TFLOP/s and kernel, and the block
     total; with cpu, the PyTorch fp32 CPU time of the same block (torch.mm + epilogue)."""
+    from supra_attn import _lib
     from supra_attn.linear_workloads import dit_block_linears
     from supra_attn.runner import StagedLinear
 
@@ -262,13 +276,16 @@ def linear_block(dev, B: int = 64, reps: int = 20, cpu: bool = True) -> dict:
             st.launch()
         dev.sync()
     layers = {}
-    total_us = 0.0
+    total_us = at_peak_us = 0.0
     for st in staged:
         ms = time_calls(dev, st.launch, reps, warmup=2)
         tf = st.call.flops() / (ms * 1e-3) / 1e12
         total_us += ms * 1e3
+        peak = unit_peak(st.args)
         layers[st.call.name] = {"shape": [st.call.M, st.call.N, st.call.K], "kernel": st.kernel,
-                                "us": round(ms * 1e3, 2), "tflops": round(tf, 2), "frac_peak": round(tf / PEAK_TFLOPS, 4)}
+                                "tile": _lib.linear_tile(st.args), "us": round(ms * 1e3, 2), "tflops": round(tf, 2),
+                                "peak": round(peak, 1), "frac_peak": round(tf / peak, 4)}
+        at_peak_us += st.call.flops() / peak * 1e-6
     for st in staged:
         st.release()
     flops = sum(c.flops() for c in calls)
@@ -276,7 +293,7 @@ def linear_block(dev, B: int = 64, reps: int = 20, cpu: bool = True) -> dict:
                        "cproj (residual), fc1 (GELU tanh), fc2 (gated residual)",
            "layers": layers, "block_us": round(total_us, 2),
            "block_tflops": round(flops / (total_us * 1e-6) / 1e12, 2),
-           "block_frac_peak": round(flops / (total_us * 1e-6) / 1e12 / PEAK_TFLOPS, 4)}
+           "block_frac_peak": round(at_peak_us / total_us, 4)}
     if cpu:
         import torch
 
@@ -304,7 +321,7 @@ def vae_block_timing(dev, calls: int = 200) -> dict:
     tf = call.flops() / (ms * 1e-3) / 1e12
     return {"workload": f"VAE mid-block attention, {call.HW} pixels x {call.C} channels: GroupNorm, q|k|v, "
                         "attention, output projection + residual in one call",
-            "us_per_call": round(ms * 1e3, 2), "tflops": round(tf, 2), "frac_peak": round(tf / PEAK_TFLOPS, 4),
+            "us_per_call": round(ms * 1e3, 2), "tflops": round(tf, 2), "peak": PEAK_TFLOPS, "frac_peak": round(tf / PEAK_TFLOPS, 4),
             "flops_per_call": call.flops()}
 
 
@@ -589,7 +606,7 @@ def summarize(run: str, workloads: list[str], out_md: str, title: str, trace_cmd
             d.setdefault("dur", []).append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
     lines += ["", "## Counters per dispatch (median over the launches); HBM bytes calibrated with a 256 MiB copy", "",
               "| workload | kernel | avg us (counter runs) | FETCH_SIZE KiB | WRITE_SIZE KiB | HBM MB (cal.) | "
-              "MFMA FLOP (MOPS_F32 x 512) | MFMA busy | LDS bank conflicts / LDS active | mean waves/CU |",
+              "MFMA FLOP (MOPS_F32 and _BF16 x 512) | MFMA busy | LDS bank conflicts / LDS active | mean waves/CU |",
               "|---|---|---|---|---|---|---|---|---|---|"]
     tj = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     traffic = {}
@@ -618,7 +635,7 @@ def summarize(run: str, workloads: list[str], out_md: str, title: str, trace_cmd
             if "GRBM_GUI_ACTIVE" in a:
                 grbm = med(a["GRBM_GUI_ACTIVE"]) / xcds
                 util = f"{100 * med(a['SQ_VALU_MFMA_BUSY_CYCLES']) / simds / grbm:.1f}%"
-                mops = f"{med(a['SQ_INSTS_VALU_MFMA_MOPS_F32']) * 512:.4g}"
+                mops = f"{sum(med(a[f'SQ_INSTS_VALU_MFMA_MOPS_{t}']) for t in ('F32', 'BF16') if f'SQ_INSTS_VALU_MFMA_MOPS_{t}' in a) * 512:.4g}"
                 lds = f"{med(a['SQ_LDS_BANK_CONFLICT']):.0f} / {med(a['SQ_LDS_IDX_ACTIVE']):.0f}"
                 waves = f"{4 * med(a['SQ_WAVE_CYCLES']) / grbm / cus:.1f}"
             else:
@@ -684,6 +701,7 @@ def main() -> int:
         staged.append((Staged(dev, s), Staged(dev, c)))
     dev.sync()
     self_kernel = staged[0][0].kernel
+    self_peak = unit_peak(staged[0][0].args)
     cross_kernel = staged[0][1].kernel
     step_flops = sum(s.call.flops() + c.call.flops() for s, c in staged)
     log(f"sweep staged: {data.blocks} blocks, self={self_kernel}, cross={cross_kernel}, "
@@ -772,11 +790,13 @@ def main() -> int:
         st = Staged(dev, call)
         ms = time_calls(dev, st.launch, args.calls, warmup=10)
         tf = call.flops() / (ms * 1e-3) / 1e12
+        peak = unit_peak(st.args)
         per_config[name] = {
             "kernel": st.kernel,
             "us_per_call": ms * 1e3,
             "tflops": tf,
-            "frac_peak": tf / PEAK_TFLOPS,
+            "peak": peak,
+            "frac_peak": tf / peak,
             "gbs": call.algorithmic_bytes() / (ms * 1e-3) / 1e9,
             "flops_per_call": call.flops(),
             "bytes_per_call": call.algorithmic_bytes(),
@@ -837,9 +857,9 @@ def main() -> int:
             "kernel": self_kernel,
             "bound": "mfma",
             "achieved": round(achieved, 3),
-            "peak": PEAK_TFLOPS,
+            "peak": round(self_peak, 1),
             "unit": "TFLOP/s",
-            "frac": round(achieved / PEAK_TFLOPS, 4),
+            "frac": round(achieved / self_peak, 4),
             "traffic": traffic_from_profiles("sweep_self"),
             "traffic_sources_sha256": kernel_sources_digest(),
             "algorithmic_flops_per_launch": self_flops,

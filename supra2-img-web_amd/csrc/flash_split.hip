@@ -1,7 +1,7 @@
 // Flash attention on the bf16 matrix cores of gfx950, head dim 64 or 128, for launches that fill the chip
 // (app/gpu/kernels.js:164-316 and, with bias and masks fused, the unfused chain of
 // app/gpu/ops.js:119-147): every float32 operand as three bfloat16 terms (split.h), every product as
-// six term products summed in float32, smallest first. Same contract as flash_mfma.hip.
+// six term products summed in float32, smallest first. Packed arguments and launch classes: flash_mfma.hip.
 //
 // Work decomposition
 //   A workgroup is QG * KS waves: QG groups of 32 queries of one (sequence, head), each seen by KS waves
@@ -9,8 +9,9 @@
 //   covers KS blocks. All waves load the step's K and V rows into registers one step ahead, split
 //   them once for the workgroup, and leave the terms in LDS in operand order.
 //   Scores S^T = K Q^T and output O^T += V^T P^T with v_mfma_f32_32x32x16_bf16: a lane holds query l%32 and
-//   keys 8(r/4) + 4(l/32) + r%4 in register r, as with the fp32 32x32x2 products, so the softmax, masks and
-//   epilogue are those of flash_mfma.hip. The 8 keys that a half-wave multiplies per product step of 16
+//   keys 8(r/4) + 4(l/32) + r%4 in register r, as with the fp32 32x32x2 products (the retry below uses them on the
+//   same softmax). The row maximum is an in-lane chain and one exchange between the half-waves, the row sum a
+//   per-lane partial until the end. The 8 keys that a half-wave multiplies per product step of 16
 //   are the 8 of its own registers (order of the sum over keys: any), so P needs no exchange: V is laid out
 //   to match. Q is pre-scaled and split once.
 //   LDS: K terms [product step][term][half][key ^ chunk], so that the 8 threads of a row write 8 different
@@ -30,7 +31,9 @@ namespace sa {
 
 namespace {
 
-constexpr float kRescaleSlack = 8.f;  // log2 units: p stays <= 256 between rescales
+// O and l are rescaled only when a block's maximum exceeds the reference by more than this (log2 units: p
+// stays <= 256); numerator and denominator share the reference.
+constexpr float kRescaleSlack = 8.f;
 
 struct FlashOrder {
   uint8_t order[kMaxOrder];

@@ -112,8 +112,8 @@ __device__ __forceinline__ void tile_coords(int t, const TileOrder& o, int& mi, 
   ni = g * o.group_n + off % w;
 }
 
-// Waves per SIMD that the register budget of linear_split_kernel is set for (its VGPRs: 64 x 96 110,
-// 128 x 96 168, 256 x 144 196, 256 x 192 224).
+// Waves per SIMD that the register budget of linear_split_kernel is set for (its VGPRs: 64 x 64 106,
+// 64 x 96 116, 128 x 96 168, 256 x 144 198, 256 x 192 228; no scratch).
 template <int NW, int MT, int NT>
 constexpr int split_waves_per_simd() {
   return MT * NT <= 6 ? 4 : MT * NT <= 12 ? 3 : 2;
@@ -165,7 +165,7 @@ __device__ __forceinline__ void redo_tile(const LinArgs& p, int m0, int n0, int 
 // What bounds it: the matrix cores at the clock they hold under this load (random operands: 2.06 of
 // the nominal 2.5 PFLOP/s measured with nothing but these MFMAs, i.e. 344 TFLOP/s of products) and the
 // issue slots the split takes beside them (11 VALU instructions per two elements; without the split,
-// results discarded, 263 TFLOP/s at K = 2304, with it 235). 16x16x32 measured faster than 32x32x16 on
+// results discarded, 263 TFLOP/s at K = 2304, with it 235, with the row norms of the retry 225). 16x16x32 measured faster than 32x32x16 on
 // whole grids (qkv layer of 16384 rows 160 against 191-211 us), and 8 waves over 256 rows faster than
 // twice 4 waves over 128 (half the W splits).
 template <int NW, int MT, int NT, int ACT, int EPI>
@@ -931,6 +931,8 @@ bool linear_mfma_supported(const LinearParams& p) {
          (int64_t)64 * 2 * p.ldy * 4 < 0x7fffffffLL;
 }
 
+namespace {
+
 // Size class of a call: the tile of the fp32 kernels that its grid fills, and the kernel's name in the
 // API. Classes 128 x 192 and 64 x 192 (at least one 128 x 192 tile per CU, or three 64 x 192 ones) run
 // linear_split_kernel, class 64 x 64 that or linear_mfma_kernel, the 32 x 64 class that or
@@ -945,8 +947,6 @@ bool linear_mfma_supported(const LinearParams& p) {
 // splits 18.9-19.4). The split kernel's smallest tiles (64 x 48, 32 x 48) measured slower on the small grids:
 // 13-20 against 6-15 us at K = 576, with one, two or four k-tiles of loads in flight alike: a wave alone
 // on its SIMD issues one VALU instruction per 6 cycles, and the splits are most of its work.
-namespace {
-
 enum LinearClass { kClass128x192, kClass64x192, kClass64x64, kClass32x64, kClass32x32 };
 LinearClass linear_class(const LinearParams& p, int num_cus) {
   const int64_t tiles_wide = ((p.M + 127) / 128) * ((p.N + 191) / 192);

@@ -409,8 +409,8 @@ __global__ __launch_bounds__(256, 1) void wide_mfma_kernel(WideArgs p) {
 // K and V rows come straight from memory into registers, pipelined ahead of their products, and are split
 // there: with 32 queries per workgroup every element is used once, 7 VALU instructions per MFMA, put
 // between the products that cover them. That is what bounds it: a wave alone issues one of them per
-// 6 cycles, two waves per SIMD one per 4.4, so 8 waves and not 4 (4096 tokens, the whole call: 331 against 345 us; fp32
-// products: 401). Q is split once, into LDS; two blocks per wave halve its reads, which at one block
+// 6 cycles, two waves per SIMD one per 4.4, so 8 waves and not 4 (the VAE block of 4096 tokens: 331 against 345 us,
+// fp32 products 401; its attention alone 256 us, fp32 299). Q is split once, into LDS; two blocks per wave halve its reads, which at one block
 // would take LDS (64 bytes per clock and CU) as long as the MFMAs.
 // Writes the same partial records as wide_mfma_kernel (merged by wide_merge_kernel).
 template <int BIAS, int MASK>
@@ -993,9 +993,11 @@ int wide_mfma_variants(FlashVariant* out, int cap) {
 // Key chunks per query group: of the plans whose merge records fit kWideMaxRecordBytes, the one
 // with the shortest modelled makespan (ties: the first found, fewer chunks). A workgroup costs the
 // key blocks of its chunk plus about two blocks of start-up and stores; workgroups run in rounds of
-// one per CU (D = 512: one wave per SIMD at 400 registers) or two (D = 256: 80 KiB of LDS); a split
+// one per CU (D = 512: 8 waves, 146 KiB of LDS) or two (D = 256: 80 KiB of LDS); a split
 // adds the merge, about half a block plus one block per 22 MB of records. One block is 32 queries x
-// 32 keys over all head dims (about 4.4 us of a CU at D = 512). The plans: every group in the same
+// 32 keys over all head dims. (At D = 512 the constants are those of an fp32 kernel of 4.7 us per block; wide_split_kernel
+// takes 3.9 us per block, 0.5 to 1.6 blocks more per workgroup, and its merge of 16.8 MB 5.2 us, 1.3 blocks, as
+// modelled.) The plans: every group in the same
 // number of chunks (up to kWideMaxChunks), or, when the groups fill whole rounds and a few more,
 // the whole rounds unsplit and only the groups past them in chunks, in a second launch. For one
 // head of 1024 tokens this is 8 chunks of 4 blocks (256 workgroups, one round); for 2304 tokens 3
